@@ -211,13 +211,12 @@ int pdgpu_setup_gb(pdgpu_engine *e, const pdgpu_gb_params *p, const double *gbra
                    const int32_t *off12, const int32_t *idx12, const double *d12,
                    const int32_t *off13, const int32_t *idx13, const double *d13);
 
-/* Work split of the GB tile kernels (k_gb_radii, k_gb_pair, k_gb_chain: one
- * 64x64 atom tile pair per workgroup): split[k] wavefronts share a tile pair of
- * kernel k, each taking 64/split[k] of its rotated j steps with its own partial
- * sums, added in wavefront order (1, 2 or 4; default 1, NULL: all 1).  A split
- * changes the FP32 rounding of the tile sums (within the stated error), so runs
- * are bitwise reproducible for a fixed split.  No counterpart in PD: the launch
- * shape of the GB passes. */
+/* Work split of the GB passes (Born radii, pair terms, chain rule): split[k]
+ * wavefronts share a task of pass k (one or two 64-atom i tiles against a run of j
+ * tiles), taking its chunks of 16 rotated j steps in turn (1, 2 or 4; NULL: all 1;
+ * until it is called, the number that suits the number of tasks).  Sums beyond a
+ * chunk are integers, so forces and radii are the same bits for every split; energies
+ * differ by FP64 rounding.  No counterpart in PD: the launch shape of the GB passes. */
 int pdgpu_set_gb_split(pdgpu_engine *e, const int32_t *split);
 /* The autotuner: one full GB pass on the current positions, then each tile kernel
  * 5 times at split 1, 2 and 4 (HIP events); keeps the fastest split per kernel,

@@ -150,21 +150,43 @@ struct GBK {
   double cut2;          // Cutoff^2
   double cut;           // Cutoff
   double still2;        // GbsaStillCutoff^2
-  double vdwcut2;       // VdwCutoff^2
-  double vdwcut;        // VdwCutoff: PD's LJ test is on the distance (gbff.cpp:1686)
-  float premul;         // -halfeconv (1/eps_in - 1/eps_out), kcal/mol A
-  float ec_in, ec_out;  // econv / eps_in, econv / eps_out
+  double vdw_lim;       // sqrt(r2) < VdwCutoff is r2 < vdw_lim (gbff.cpp:1686)
+  double gb_lim;        // sqrt(r2) <= Cutoff is r2 < gb_lim (gbff.cpp:560)
+  double premul_d;      // -halfeconv (1/eps_in - 1/eps_out), kcal/mol A
+  double ec_in_d;       // econv / eps_in
+  float premul2;        // 2 premul_d
+  float ec_in, ec_out, ec_ratio;  // ec_in_d, econv / eps_out, eps_in / eps_out
   float inner, invw, invw2_4;
   float vdwinner, vinvw, vinvw2_4;
   float thresh;         // ExpApproxThreshold
-  float P4, P5, invP5;
+  float P4, invP5, half_pi_P5;  // P4, 1 / P5, pi P5 / 2
   float vdw14, elec14;
-  float pi;
+  float inside, outside, far_k, fix_lim, edge;  // per pass (GBState::set_params)
 };
-// One 64x64 tile pair of one system: first atoms of the i and j tiles (global
-// indices) and whether bond orders must be looked up.
-struct GBWork {
-  int sys, i0, j0, special;
+// A piece of work of the GB passes: i tiles ti .. ti+ni-1 (ni 1 or 2) against j
+// tiles tj .. tj+nj-1 (indices over all systems' tiles), the table of its pair codes
+// (-1: none), its energy slot (contiguous within a system).
+struct GBTask {
+  int sys, ti, ni, tj, nj, code, slot, pad;
+};
+// A tile's centre, the largest distance of an atom from it, its largest GB radius
+// and its largest Born radius, at the current positions.
+struct GBTile {
+  double x, y, z, rad;
+  float rmax, amax;
+};
+struct GBPassArgs {
+  GBK K;
+  const GBTask *tasks;
+  const int2 *tile_atoms;  // per tile: first atom, atoms
+  const GBTile *tiles;
+  const unsigned *codes;
+  const double *x, *y, *z;
+  const float *q, *ljr, *lje, *bornf, *gbrad, *Vj;
+  const double *born;
+  const long long *deda_in;
+  long long *s0, *s1, *s2, *s3;  // the pass's sums per atom
+  double *e_part;
 };
 struct GBSys {
   int first, count;     // atom range in the concatenated arrays
@@ -230,16 +252,22 @@ struct PlainGB {
 };
 struct GBState {
   pdgpu_gb_params prm{};
-  GBK kp{};
+  GBK kp{}, kr{};  // of the pair pass; of radii and chain
   int n_atoms_total = 0;
-  std::vector<GBWork> h_work;
+  std::vector<GBTask> h_tasks;
   std::vector<GBSys> h_sys;
+  std::vector<int2> h_tile_atoms;
+  std::vector<std::vector<std::pair<int, int>>> h_linked;  // per system: tile pairs with a sparse partner
   std::vector<int8_t> h_band;
-  std::vector<int> h_sp_off, h_sp_part, h_sp_ord, h_work_beg, h_work_end;
-  DBuf<GBWork> work;
+  std::vector<int> h_sp_off, h_sp_part, h_sp_ord, h_tile_beg, h_slot_beg, h_slot_end, h_coded;
+  int n_slots = 0;
+  DBuf<GBTask> tasks;
   DBuf<GBSys> sysd;
+  DBuf<int2> tile_atoms;
+  DBuf<GBTile> tiles;
+  DBuf<unsigned> codes;
   DBuf<int8_t> band;
-  DBuf<int> sp_off, sp_part, sp_ord, work_beg, work_end, sys_first, sys_count;
+  DBuf<int> sp_off, sp_part, sp_ord, slot_beg, slot_end, sys_first, sys_count, coded;
   DBuf<long long> gpol, deda;
   DBuf<double> born, eself, e_part, terms123;
   DBuf<float> bornf, q, ljr, lje, gbrad, Vj;
@@ -250,8 +278,14 @@ struct GBState {
   void upload(hipStream_t s);
   void run(hipStream_t s, const double *x, const double *y, const double *z, long long *fx, long long *fy,
            long long *fz, double *out, int out_stride, int out_off, Engine *timer_owner, bool energy_only = false);
-  // wavefronts per tile pair of k_gb_radii, k_gb_pair, k_gb_chain (1, 2 or 4)
-  int split[3] = {1, 1, 1};
+  // wavefronts per task of the radii, pair and chain passes (1, 2 or 4; 0: by the
+  // number of tasks)
+  int split[3] = {0, 0, 0};
+  void make_tasks();
+  GBPassArgs pass_args(const double *x, const double *y, const double *z, long long *fx, long long *fy,
+                       long long *fz) const;
+  template <int PASS>
+  void launch_pass(hipStream_t s, const GBPassArgs &A, int sp);
   // the plain comparator (one thread per atom, FP64 sums): on for a single system
   bool plain = false;
   DBuf<double> pl_q, pl_r, pl_e, pl_gr, pl_vj, pl_deda, pl_e3;

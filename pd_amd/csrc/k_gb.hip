@@ -1,5 +1,5 @@
-// k_gb.hip -- FF_GeneralizedBorn_Still (FastMode) on the device, for one system
-// or a batch of independent systems.
+// k_gb.hip -- FF_GeneralizedBorn_Still on the device, for one system or a batch
+// of independent systems.
 //
 // PD evaluates three passes over its (shadow) neighbour list each step:
 //   1. calcBornRadii_PairwiseApprox (gbff.cpp:432-483): Gpol_i = terms123_i +
@@ -12,15 +12,37 @@
 //      terms premul q^2 / a (gbff.cpp:1750-1757);
 //   3. the Born-radius chain rule (gbff.cpp:1768-1825) with gpi = a_i^2 / 166.0.
 // Here every pass is an all-pairs walk over 64x64 atom tiles of each system
-// (upper triangle of tile pairs), one wavefront per tile pair: lanes hold the i
-// atoms, the j tile sits in LDS and is visited in the rotated order
-// j = (lane + t) mod 64, so every lane touches a different j in each step and
-// the j accumulators in LDS need no atomics.  Pairs are tested with PD's
-// per-pair cutoffs (FP64 r^2 as PD computes it); the radii, dE/da and force
-// sums are 64-bit fixed point, so they are independent of summation order.
-// Tile pairs whose atoms lie within BondOrder::m_MaxIndexDelta of each other,
-// or hold an off-diagonal covalent partner, are flagged and look the bond order
-// up exactly as the list builder does; all other pairs have order 7.
+// (upper triangle of tile pairs): lanes hold the i atoms, the j tile sits in LDS
+// and is visited in the rotated order j = (lane + t) mod 64.
+//
+// What bounds the passes is VALU issue (a wave64 instruction holds its SIMD for
+// four cycles), so a tile pair runs the shortest loop its geometry allows.  One
+// small kernel per evaluation gives every tile a centre and a radius; from these
+// (and the tiles' largest GB and Born radii) a tile pair is
+//   far   every pair lies inside all cutoffs and beyond the reach of the short-range
+//         part of the pass (the exp threshold of the cross term, the CCF function of
+//         the radii): no tests, and only the terms that are left (the pair pass:
+//         solvent Coulomb and LJ).  Two i tiles share each j read.  FP32
+//         displacements from FP32 offsets about the midpoint of the two tiles,
+//         which the distance of the tiles keeps at the precision of r itself;
+//   near  everything else: FP64 displacements and r^2, rounded once, with PD's per-pair
+//         cutoff tests unless every pair is inside them;
+//   out   beyond every cutoff: left at once.
+// Tile pairs whose atoms lie within BondOrder::m_MaxIndexDelta of each other, or
+// hold an off-diagonal covalent partner, and the diagonal ones are tasks of their
+// own with a table of 2-bit codes (in the rotated order, built once at setup), so
+// the loop looks no bond order up.
+// The j partial sums stay in registers and move with the rotation: acc =
+// rotate(acc) + term is one DPP add.  Every 16 steps (a chunk) the FP32 partial
+// sums go to 64-bit fixed point; chunks, tasks and wavefronts then only add
+// integers, so forces, radii and dE/da are the same bits for every work split.
+// Measured (radii / pair / chain): 256 chains of 20-120 residues (54,560 tile pairs) 243
+// / 467 / 299 -> 101 / 304 / 170 us, both sums of the pair pass at 0.95 of the VALU issue
+// rate; a 300-residue chain 36 / 55 / 44 -> 14 / 31 / 22 us; a 20-residue chain at 15 A
+// cutoffs 34 / 45 / 36 -> 9 / 16 / 11 us, where the latency of one wavefront's 16 steps is
+// what is left.  The near loops' 1 / r^2 to full FP32 precision and the FP64 decision at the
+// exp threshold cost 30 of the 304 us; they take the forces' error against FP64 from 5.6e-7 to
+// 3.5e-7 (20 residues) and 1.1e-6 to 3.8e-7 (300 residues).
 #include <algorithm>
 #include <array>
 #include <cmath>
@@ -35,6 +57,10 @@ namespace pdgpu {
 namespace {
 
 constexpr int kTile = 64;
+constexpr int kChunk = 16;  // rotated steps between two conversions to fixed point
+// codes of a pair in a task's table: 0 non-bonded, 1 1-4 partner, 2 1-2 or 1-3
+// partner, 3 no pair (beyond the tile's atoms, or a diagonal pair taken elsewhere)
+enum { kPairPlain = 0, kPair14 = 1, kPairBonded = 2, kPairNone = 3 };
 
 // Bond order of pair (a, b) as NeighbourList::calcNewList + correctOffDiagonalBondOrders
 // assign it (neighbourlist.cpp:399-406, 179-220); indices are local to the system.
@@ -49,432 +75,135 @@ __device__ __forceinline__ int gb_bond_order(int a, int b, int mid, const int8_t
   return bo & 7;
 }
 
-__device__ __forceinline__ bool tile_pair_valid(int lane, int t, int ni, int nj, bool diag, int jj) {
-  bool v = lane < ni && jj < nj;
-  if (diag) v = v && ((t >= 1 && t < 32) || (t == 32 && lane < 32));
-  return v;
-}
-
-// A bound on every (i, j) distance of a tile pair: the distance between the two
-// tiles' first atoms plus each tile's largest distance from its first atom.  A
-// tile pair whose bound (plus 1e-3 A) lies inside every cutoff (and inside the
-// switching radii) skips the per-pair tests: they would all pass, and the
-// switch would be exactly 1 with zero slope.  Such tiles also take their pair
-// displacements as FP32 differences of FP32 offsets from the i tile's first atom
-// (p0), within ~1e-6 A of PD's FP64 displacement.  Lane 0 holds a real i and j atom.
-__device__ __forceinline__ double tile_bound(double xi, double yi, double zi, bool iv, double xj, double yj,
-                                             double zj, bool jv, double &x0, double &y0, double &z0) {
-  x0 = __shfl(xi, 0, 64);
-  y0 = __shfl(yi, 0, 64);
-  z0 = __shfl(zi, 0, 64);
-  const double xj0 = __shfl(xj, 0, 64), yj0 = __shfl(yj, 0, 64), zj0 = __shfl(zj, 0, 64);
-  auto sq = [](double v) { return v * v; };
-  const double di = wave_max(iv ? sqrt(sq(xi - x0) + sq(yi - y0) + sq(zi - z0)) : 0.0);
-  const double dj = wave_max(jv ? sqrt(sq(xj - xj0) + sq(yj - yj0) + sq(zj - zj0)) : 0.0);
-  return sqrt(sq(xj0 - x0) + sq(yj0 - y0) + sq(zj0 - z0)) + di + dj + 1e-3;
-}
-
-// ---- pass 1: Born radii -------------------------------------------------------------
-// SPLIT wavefronts share a tile pair: wavefront w takes the rotated steps
-// t = w*64/SPLIT .. (w+1)*64/SPLIT-1 with its own i and j partial sums, which are
-// added in wavefront order at the end (SPLIT = 1: one wavefront, every step).
-template <int SPLIT>
-__global__ __launch_bounds__(64 * SPLIT) void k_gb_radii(GBK K, const GBWork *__restrict__ work,
-                                                         const GBSys *__restrict__ sys, const double *__restrict__ x,
-                                                         const double *__restrict__ y, const double *__restrict__ z,
-                                                         const float *__restrict__ gbrad, const float *__restrict__ Vj,
-                                                         const int8_t *__restrict__ band,
-                                                         const int *__restrict__ sp_off,
-                                                         const int *__restrict__ sp_part,
-                                                         const int *__restrict__ sp_ord, long long *__restrict__ gpol) {
-  __shared__ double sx[kTile], sy[kTile], sz[kTile];
-  __shared__ float sxf[kTile], syf[kTile], szf[kTile];
-  __shared__ float sR[kTile], sV[kTile], acc[SPLIT][kTile], ipart[SPLIT][kTile];
-  const GBWork w = work[blockIdx.x];
+// The code tables of the tasks with codes (once, at setup): one wavefront per
+// task, word c * 64 + lane holds lane's codes of steps 16 c .. 16 c + 15.
+__global__ __launch_bounds__(64) void k_gb_codes(const GBTask *__restrict__ tasks, const int *__restrict__ coded,
+                                                 const int2 *__restrict__ tile_atoms, const GBSys *__restrict__ sys,
+                                                 const int8_t *__restrict__ band, const int *__restrict__ sp_off,
+                                                 const int *__restrict__ sp_part, const int *__restrict__ sp_ord,
+                                                 unsigned *__restrict__ codes) {
+  const GBTask w = tasks[coded[blockIdx.x]];
   const GBSys S = sys[w.sys];
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const int end = S.first + S.count;
-  const int ni = min(kTile, end - w.i0), nj = min(kTile, end - w.j0);
-  const bool diag = w.i0 == w.j0;
-  const int i = w.i0 + lane;
-  const bool iv = lane < ni;
-  const double xi = iv ? x[i] : 0.0, yi = iv ? y[i] : 0.0, zi = iv ? z[i] : 0.0;
-  const float Ri = iv ? gbrad[i] : 0.0f, Vi = iv ? Vj[i] : 0.0f;
-  double x0, y0, z0;
-  bool fast;
-  {
-    const int j = w.j0 + lane;
-    const bool v = lane < nj;
-    const double xj = v ? x[j] : 0.0, yj = v ? y[j] : 0.0, zj = v ? z[j] : 0.0;
-    const double bd = tile_bound(xi, yi, zi, iv, xj, yj, zj, v, x0, y0, z0);
-    fast = bd * bd < K.still2;
-    if (wv == 0) {
-      sx[lane] = xj;
-      sy[lane] = yj;
-      sz[lane] = zj;
-      sxf[lane] = (float)(xj - x0);
-      syf[lane] = (float)(yj - y0);
-      szf[lane] = (float)(zj - z0);
-      sR[lane] = v ? gbrad[j] : 0.0f;
-      sV[lane] = v ? Vj[j] : 0.0f;
-    }
-    acc[wv][lane] = 0.0f;
-  }
-  const float xif = (float)(xi - x0), yif = (float)(yi - y0), zif = (float)(zi - z0);
-  __syncthreads();
-  float gi = 0.0f;
-  auto tile = [&](auto fast_c) {
-  constexpr bool FAST = decltype(fast_c)::value;
-  for (int t = wv * (kTile / SPLIT); t < (wv + 1) * (kTile / SPLIT); t++) {
-    const int jj = (lane + t) & (kTile - 1);
-    bool on = tile_pair_valid(lane, t, ni, nj, diag, jj);
-    float r2f;
-    if (FAST) {
-      const float dx = xif - sxf[jj], dy = yif - syf[jj], dz = zif - szf[jj];
-      r2f = dx * dx + dy * dy + dz * dz;
-    } else {
-      double r2;
-      {
-#pragma clang fp contract(off)
-        const double dx = xi - sx[jj], dy = yi - sy[jj], dz = zi - sz[jj];
-        r2 = dx * dx + dy * dy + dz * dz;  // sqrdist, gbff.cpp:455
+  const int2 A = tile_atoms[w.ti], B = tile_atoms[w.tj];
+  const bool diag = w.ti == w.tj;
+  const int lane = threadIdx.x;
+  for (int c = 0; c < kTile / kChunk; c++) {
+    unsigned word = 0u;
+    for (int u = 0; u < kChunk; u++) {
+      const int t = c * kChunk + u, jj = (lane + t) & (kTile - 1);
+      bool v = lane < A.y && jj < B.y;
+      if (diag) v = v && ((t >= 1 && t < 32) || (t == 32 && lane < 32));
+      unsigned code = kPairNone;
+      if (v) {
+        const int bo = gb_bond_order(A.x + lane - S.first, B.x + jj - S.first, S.mid, band + S.band_off,
+                                     sp_off + S.sp_base, sp_part, sp_ord);
+        code = bo <= 2 ? kPairBonded : (bo == 3 ? kPair14 : kPairPlain);
       }
-      on = on && r2 <= K.still2;
-      r2f = (float)r2;
+      word |= code << (2 * u);
     }
-    if (w.special && on) {
-      const int bo = gb_bond_order(i - S.first, w.j0 + jj - S.first, S.mid, band + S.band_off,
-                                   sp_off + S.sp_base, sp_part, sp_ord);
-      on = bo > 2;  // only non-bonded and 1-4 partners (gbff.cpp:460-461)
-    }
-    r2f = on ? r2f : 1.0f;
-    const float Rs = Ri + sR[jj];
-    const float rdivR = r2f * __builtin_amdgcn_rcpf(Rs * Rs);  // hardware reciprocal, 1 ulp
-    float ccf = 1.0f;
-    if (rdivR <= K.invP5) {
-      const float c = 0.5f - 0.5f * cosf(rdivR * K.P5 * K.pi);
-      ccf = c * c;
-    }
-    const float base = K.P4 * ccf * __builtin_amdgcn_rcpf(r2f * r2f);
-    gi += on ? base * sV[jj] : 0.0f;
-    acc[wv][jj] += on ? base * Vi : 0.0f;
+    codes[(size_t)w.code * (kTile / kChunk) * kTile + c * kTile + lane] = word;
   }
-  };
-  if (fast)
-    tile(std::true_type{});
-  else
-    tile(std::false_type{});
-  ipart[wv][lane] = gi;
-  __syncthreads();
-  if (wv == 0) {
-    float si = ipart[0][lane], sj = acc[0][lane];
-#pragma unroll
-    for (int k = 1; k < SPLIT; k++) {
-      si += ipart[k][lane];
-      sj += acc[k][lane];
-    }
-    if (iv) fix_add(&gpol[i], fix_from_float(si));
-    if (lane < nj) fix_add(&gpol[w.j0 + lane], fix_from_float(sj));
+}
+
+// Opens an evaluation: each tile's centre (of its atoms' box) and the largest
+// distance of an atom from it, its largest GB radius; clears the Gpol sums.  One
+// wavefront per tile.
+__global__ __launch_bounds__(256) void k_gb_tiles(int ntiles, const int2 *__restrict__ tile_atoms,
+                                                  const double *__restrict__ x, const double *__restrict__ y,
+                                                  const double *__restrict__ z, const float *__restrict__ gbrad,
+                                                  GBTile *__restrict__ tiles, long long *__restrict__ gpol) {
+  const int t = blockIdx.x * 4 + ((int)threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (t >= ntiles) return;  // whole waves; no barrier follows
+  const int2 A = tile_atoms[t];
+  const bool on = lane < A.y;
+  const int i = A.x + lane;
+  double p[3] = {0.0, 0.0, 0.0}, c[3];
+  float R = 0.0f;
+  if (on) {
+    p[0] = x[i];
+    p[1] = y[i];
+    p[2] = z[i];
+    R = gbrad[i];
+    gpol[i] = 0;
+  }
+  double d2 = 0.0;
+  for (int k = 0; k < 3; k++) {
+    c[k] = 0.5 * (wave_min(on ? p[k] : 1e300) + wave_max(on ? p[k] : -1e300));
+    d2 += (p[k] - c[k]) * (p[k] - c[k]);
+  }
+  const double rad = wave_max(on ? sqrt(d2) : 0.0);
+  const double rmax = wave_max((double)R);
+  if (lane == 0) {
+    GBTile T;
+    T.x = c[0];
+    T.y = c[1];
+    T.z = c[2];
+    T.rad = rad;
+    T.rmax = (float)rmax;
+    T.amax = 0.0f;
+    tiles[t] = T;
   }
 }
 
 // a_i = -halfeconv / (terms123_i + sum) + BornRadiusOffset; the self term
-// premul q^2 / a seeds dE/da (gbff.cpp:1750-1757).
-__global__ void k_gb_finalize_radii(int n, double halfeconv, double offset, double premul,
-                                    const double *__restrict__ terms123, const long long *__restrict__ gpol,
-                                    const float *__restrict__ q, double *__restrict__ born,
-                                    float *__restrict__ bornf, long long *__restrict__ deda,
-                                    double *__restrict__ eself) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const double G = terms123[i] + (double)gpol[i] * (1.0 / kFixScale);
-  const double a = -halfeconv / G + offset;
-  born[i] = a;
-  bornf[i] = (float)a;
-  const double qi = q[i];
-  const double epol = premul * qi * qi / a;
-  eself[i] = epol;
-  deda[i] = fix_from_double(-epol / a);
+// premul q^2 / a seeds dE/da (gbff.cpp:1750-1757).  One wavefront per tile: also the
+// tile's largest Born radius (infinite, so that no tile pair counts as far, when one is
+// not positive).
+__global__ __launch_bounds__(256) void k_gb_finalize_radii(int ntiles, const int2 *__restrict__ tile_atoms,
+                                                           double halfeconv, double offset, double premul,
+                                                           const double *__restrict__ terms123,
+                                                           const long long *__restrict__ gpol,
+                                                           const float *__restrict__ q, double *__restrict__ born,
+                                                           float *__restrict__ bornf, long long *__restrict__ deda,
+                                                           double *__restrict__ eself, GBTile *__restrict__ tiles) {
+  const int t = blockIdx.x * 4 + ((int)threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (t >= ntiles) return;  // whole waves; no barrier follows
+  const int2 A = tile_atoms[t];
+  const int i = A.x + lane;
+  double amax = 0.0;
+  if (lane < A.y) {
+    const double G = terms123[i] + (double)gpol[i] * (1.0 / kFixScale);
+    const double a = -halfeconv / G + offset;
+    born[i] = a;
+    bornf[i] = (float)a;
+    const double qi = q[i];
+    const double epol = premul * qi * qi / a;
+    eself[i] = epol;
+    deda[i] = fix_from_double(-epol / a);
+    amax = a > 0.0 ? a : 1e30;
+  }
+  amax = wave_max(amax);
+  if (lane == 0) tiles[t].amax = (float)amax;
 }
 
-// ---- pass 2: GB cross terms, vacuum Coulomb and LJ ----------------------------------
-// MODE kGbFast: FastMode's calcForcesIncludingVacuo, above.
-// MODE kGbEnergy: FF_GeneralizedBorn_Still::calcEnergies instead (gbff.cpp:178-183,
-// 537-596): the exact GB cross term on every pair within Cutoff, whatever its bond
-// order and with no ExpApproxThreshold swap, plus FF_NonBonded::calcEnergies with
-// Dielectric = DielectricSolute and energy switching; no forces, no dE/da.
-// MODE kGbBorn: calcForces with FastMode off (gbff.cpp:186-196): FF_NonBonded::
-// calcForces with Dielectric = DielectricSolute and energy switching, and the cross
-// term of calcBornForces (gbff.cpp:1189-1345) on every pair within Cutoff, with
-// 1/r in place of 1/f_GB (and no dE/da) where uGB <= ExpApproxThreshold.
-enum { kGbFast = 0, kGbEnergy = 1, kGbBorn = 2 };
-template <int MODE, int SPLIT>
-__global__ __launch_bounds__(64 * SPLIT) void k_gb_pair(
-    GBK K, const GBWork *__restrict__ work, const GBSys *__restrict__ sys, const double *__restrict__ x,
-    const double *__restrict__ y, const double *__restrict__ z, const float *__restrict__ q,
-    const float *__restrict__ ljr, const float *__restrict__ lje, const float *__restrict__ born,
-    const int8_t *__restrict__ band, const int *__restrict__ sp_off, const int *__restrict__ sp_part,
-    const int *__restrict__ sp_ord, long long *__restrict__ fx, long long *__restrict__ fy,
-    long long *__restrict__ fz, long long *__restrict__ deda, double *__restrict__ e_part) {
-  constexpr bool EONLY = MODE == kGbEnergy;
-  __shared__ double sx[kTile], sy[kTile], sz[kTile];
-  __shared__ float sxf[kTile], syf[kTile], szf[kTile];
-  __shared__ float sq[kTile], sr[kTile], se[kTile], sa[kTile], sai[kTile];
-  __shared__ float ax[SPLIT][kTile], ay[SPLIT][kTile], az[SPLIT][kTile], ad[SPLIT][kTile];
-  __shared__ float ip[SPLIT][4][kTile];
-  __shared__ double es[SPLIT][3];
-  const GBWork w = work[blockIdx.x];
-  const GBSys S = sys[w.sys];
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const int end = S.first + S.count;
-  const int ni = min(kTile, end - w.i0), nj = min(kTile, end - w.j0);
-  const bool diag = w.i0 == w.j0;
-  const int i = w.i0 + lane;
-  const bool iv = lane < ni;
-  const double xi = iv ? x[i] : 0.0, yi = iv ? y[i] : 0.0, zi = iv ? z[i] : 0.0;
-  const float qi = iv ? q[i] : 0.0f, ri = iv ? ljr[i] : 0.0f, ei = iv ? lje[i] : 0.0f;
-  const float ai = iv ? born[i] : 1.0f;
-  double x0, y0, z0;
-  bool fast;
-  {
-    const int j = w.j0 + lane;
-    const bool v = lane < nj;
-    const double xj = v ? x[j] : 0.0, yj = v ? y[j] : 0.0, zj = v ? z[j] : 0.0;
-    // inside both cutoffs and both switching radii
-    const double bd = tile_bound(xi, yi, zi, iv, xj, yj, zj, v, x0, y0, z0);
-    fast = bd * bd < fmin(K.cut2, K.vdwcut2) && bd < (double)fminf(K.inner, K.vdwinner);
-    if (wv == 0) {
-      sx[lane] = xj;
-      sy[lane] = yj;
-      sz[lane] = zj;
-      sxf[lane] = (float)(xj - x0);
-      syf[lane] = (float)(yj - y0);
-      szf[lane] = (float)(zj - z0);
-      sq[lane] = v ? q[j] : 0.0f;
-      sr[lane] = v ? ljr[j] : 0.0f;
-      se[lane] = v ? lje[j] : 0.0f;
-      const float aj = v ? born[j] : 1.0f;
-      sa[lane] = aj;
-      sai[lane] = 1.0f / aj;
-    }
-    ax[wv][lane] = ay[wv][lane] = az[wv][lane] = ad[wv][lane] = 0.0f;
-  }
-  const float xif = (float)(xi - x0), yif = (float)(yi - y0), zif = (float)(zi - z0);
-  const float ai_q = 0.25f / ai;  // uGB = -r^2 / (4 a_i a_j) = -r^2 (0.25 / a_i) (1 / a_j)
-  __syncthreads();
-  float fix = 0.0f, fiy = 0.0f, fiz = 0.0f, dai = 0.0f;
-  double epol = 0.0, evdw = 0.0, eel = 0.0;
-  auto tile = [&](auto fast_c) {
-  constexpr bool FAST = decltype(fast_c)::value;
-  // energies: FP32 sums over 8 consecutive pairs of a lane, then FP64
-  for (int t0 = wv * (kTile / SPLIT); t0 < (wv + 1) * (kTile / SPLIT); t0 += 8) {
-  float ep8 = 0.0f, ev8 = 0.0f, el8 = 0.0f;
-#pragma unroll 1
-  for (int t = t0; t < t0 + 8; t++) {
-    const int jj = (lane + t) & (kTile - 1);
-    bool on = tile_pair_valid(lane, t, ni, nj, diag, jj);
-    float dxf, dyf, dzf, r2raw;
-    double r2 = 0.0;
-    bool on_gb = false;
-    if (FAST) {
-      dxf = xif - sxf[jj];
-      dyf = yif - syf[jj];
-      dzf = zif - szf[jj];
-      r2raw = dxf * dxf + dyf * dyf + dzf * dzf;
-      if (EONLY) on_gb = on;
-    } else {
-      double dx, dy, dz;
-      {
-#pragma clang fp contract(off)
-        dx = xi - sx[jj];
-        dy = yi - sy[jj];
-        dz = zi - sz[jj];
-        r2 = dx * dx + dy * dy + dz * dz;  // gbff.cpp:1588-1591
-      }
-      if (EONLY) {
-        on_gb = on && sqrt(r2) <= K.cut;  // calcBornEnergy's test on the distance (gbff.cpp:560)
-        on = on && r2 <= K.cut2;
-      } else {
-        on = on && r2 <= K.cut2;
-      }
-      dxf = (float)dx;
-      dyf = (float)dy;
-      dzf = (float)dz;
-      r2raw = (float)r2;
-    }
-    int bo = 7;
-    if (w.special && on)
-      bo = gb_bond_order(i - S.first, w.j0 + jj - S.first, S.mid, band + S.band_off, sp_off + S.sp_base, sp_part,
-                         sp_ord);
-    const float r2f = (on || on_gb) ? r2raw : 1.0f;
-    const float rinv = __builtin_amdgcn_rsqf(r2f);
-    const float r = r2f * rinv;
-    const float aj = sa[jj];
-    const float qq = qi * sq[jj];
-    const float aiaj = ai * aj;
-    const float uGB = -r2f * (ai_q * sai[jj]);
-    const bool nb = bo >= 3;                      // vdW/elec only for non-bonded and 1-4 pairs
-    const float s14e = bo == 3 ? K.elec14 : 1.0f;
-    // switching (r >= InnerCutoff), gbff.cpp:1640-1651; none inside a fast tile
-    float dS = 0.0f, Sw = 1.0f;
-    if (!FAST) {
-      const float st = fmaxf(r - K.inner, 0.0f);
-      const float S0 = 1.0f - (K.invw * st) * (K.invw * st);
-      dS = -K.invw2_4 * st * S0;
-      Sw = S0 * S0;
-    }
-    float ep = 0.0f, dedr = 0.0f, dal = 0.0f, Eel = 0.0f, Fel = 0.0f;
-    if (EONLY) {
-      ep = on_gb ? K.premul * qq * __builtin_amdgcn_rsqf(r2f + aiaj * __expf(uGB)) * Sw : 0.0f;
-      if (nb) Eel = K.ec_in * s14e * qq * rinv * Sw;
-    } else if (MODE == kGbBorn) {
-      if (uGB > K.thresh) {
-        const float tGB = __expf(uGB);
-        const float fGB = __builtin_amdgcn_rsqf(r2f + tGB * aiaj);
-        const float lGB = fGB * fGB;
-        ep = K.premul * qq * fGB;
-        dedr = -ep * (r - 0.25f * r * tGB) * lGB;
-        dal = -ep * tGB * (1.0f - uGB) * lGB;  // (1 + r^2 / 4 a_i a_j)
-      } else {
-        ep = K.premul * qq * rinv;
-        dedr = -ep * rinv;
-      }
-      if (nb) {
-        Eel = K.ec_in * s14e * qq * rinv;
-        Fel = -Eel * rinv;
-      }
-      Fel = Sw * Fel + Eel * dS;
-      Eel *= Sw;
-      dedr = Sw * dedr + dS * ep;
-      dal *= Sw;
-      ep *= Sw;
-    } else if (uGB > K.thresh) {
-      const float tGB = __expf(uGB);
-      const float fGB = __builtin_amdgcn_rsqf(r2f + tGB * aiaj);  // 1 / f_GB, 1 ulp
-      const float lGB = fGB * fGB;
-      ep = K.premul * qq * fGB;
-      dedr = -ep * (r - 0.25f * r * tGB) * lGB;
-      dal = -ep * tGB * (1.0f - uGB) * lGB;
-      if (nb) {
-        Eel = K.ec_in * s14e * qq * rinv;
-        Fel = -Eel * rinv;
-      }
-      Fel = Sw * Fel + Eel * dS;
-      Eel *= Sw;
-      dedr = Sw * dedr + dS * ep;
-      dal *= Sw;
-      ep *= Sw;
-    } else if (nb) {
-      Eel = K.ec_out * s14e * qq * rinv;
-      Fel = -Eel * rinv;
-      Fel = Sw * Fel + Eel * dS;
-      Eel *= Sw;
-    }
-    float Ev = 0.0f, Fv = 0.0f;
-    // Dist_ij < VdwCutoff (gbff.cpp:1686): r^2 decides outside a 1e-12 relative
-    // band around VdwCutoff^2, the rounded square root inside it
-    if (nb && (FAST || r2 < K.vdwcut2 * (1.0 - 1e-12) ||
-               (r2 <= K.vdwcut2 * (1.0 + 1e-12) && sqrt(r2) < K.vdwcut))) {
-      const float eps = (bo == 3 ? K.vdw14 : 1.0f) * ei * se[jj];
-      const float Rij = ri + sr[jj];
-      const float s2 = Rij * Rij * rinv * rinv;
-      const float B = s2 * s2 * s2;
-      const float A = B * B;
-      Ev = eps * (A - 2.0f * B);
-      Fv = -12.0f * eps * rinv * (A - B);
-      if (!FAST) {
-        const float vt = fmaxf(r - K.vdwinner, 0.0f);
-        const float V0 = 1.0f - (K.vinvw * vt) * (K.vinvw * vt);
-        const float vdS = -K.vinvw2_4 * vt * V0;
-        const float VS = V0 * V0;
-        Fv = VS * Fv + Ev * vdS;
-        Ev *= VS;
-      }
-    }
-    if (!EONLY) {
-      // gradient along d = p_i - p_j: GB part 2 dedr / r, vdW + elec (dE/dr) / r
-      const float g = on ? (2.0f * dedr + (nb ? (Fv + Fel) : 0.0f)) * rinv : 0.0f;
-      const float gx = g * dxf, gy = g * dyf, gz = g * dzf;
-      fix -= gx;
-      fiy -= gy;
-      fiz -= gz;
-      ax[wv][jj] += gx;
-      ay[wv][jj] += gy;
-      az[wv][jj] += gz;
-      dai += on ? dal * aj : 0.0f;
-      ad[wv][jj] += on ? dal * ai : 0.0f;
-    }
-    ep8 += (EONLY ? on_gb : on) ? ep : 0.0f;
-    ev8 += on && nb ? Ev : 0.0f;
-    el8 += on && nb ? Eel : 0.0f;
-  }
-  epol += (double)ep8;
-  evdw += (double)ev8;
-  eel += (double)el8;
-  }
-  };
-  if (fast)
-    tile(std::true_type{});
-  else
-    tile(std::false_type{});
-  ip[wv][0][lane] = fix;
-  ip[wv][1][lane] = fiy;
-  ip[wv][2][lane] = fiz;
-  ip[wv][3][lane] = dai;
-  {
-    const double se2 = wave_sum(epol), sv = wave_sum(evdw), sl = wave_sum(eel);
-    if (lane == 0) {
-      es[wv][0] = se2;
-      es[wv][1] = sv;
-      es[wv][2] = sl;
-    }
-  }
-  __syncthreads();
-  if (wv != 0) return;
-  // the wavefronts' partial sums in wavefront order
-  float si[4], sj[4];
-#pragma unroll
-  for (int c = 0; c < 4; c++) si[c] = ip[0][c][lane];
-  sj[0] = ax[0][lane];
-  sj[1] = ay[0][lane];
-  sj[2] = az[0][lane];
-  sj[3] = ad[0][lane];
-#pragma unroll
-  for (int k = 1; k < SPLIT; k++) {
-#pragma unroll
-    for (int c = 0; c < 4; c++) si[c] += ip[k][c][lane];
-    sj[0] += ax[k][lane];
-    sj[1] += ay[k][lane];
-    sj[2] += az[k][lane];
-    sj[3] += ad[k][lane];
-  }
-  if (!EONLY && iv) {
-    fix_add(&fx[i], fix_from_float(si[0]));
-    fix_add(&fy[i], fix_from_float(si[1]));
-    fix_add(&fz[i], fix_from_float(si[2]));
-    fix_add(&deda[i], fix_from_float(si[3]));
-  }
-  if (!EONLY && lane < nj) {
-    const int j = w.j0 + lane;
-    fix_add(&fx[j], fix_from_float(sj[0]));
-    fix_add(&fy[j], fix_from_float(sj[1]));
-    fix_add(&fz[j], fix_from_float(sj[2]));
-    fix_add(&deda[j], fix_from_float(sj[3]));
-  }
-  if (lane == 0) {
-    double e3[3] = {es[0][0], es[0][1], es[0][2]};
-    for (int k = 1; k < SPLIT; k++)
-      for (int c = 0; c < 3; c++) e3[c] += es[k][c];
-    e_part[4 * blockIdx.x + 0] = 2.0 * e3[0];  // PD adds each cross term twice (gbff.cpp:1655-1658)
-    e_part[4 * blockIdx.x + 1] = e3[1];
-    e_part[4 * blockIdx.x + 2] = e3[2];
-    e_part[4 * blockIdx.x + 3] = 0.0;
-  }
+// The value of the next lane (lane 63 takes lane 0's): what the rotation of the j
+// atoms by one step asks of their partial sums.  Feeding an add, it costs nothing.
+__device__ __forceinline__ float rotate1(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x134 /* wave_rol:1 */, 0xf, 0xf, true));
 }
 
-// w_i = gpi * dE/da_i * P4 with gpi = a_i^2 / 166.0 (gbff.cpp:1772)
-// The chain-rule weight of atom i: -a_i^2 / -166 dE/da_i P4 (dE/da from its
-// fixed-point sum), evaluated by the chain kernel for its tile's atoms.
+// sin and cos of h in [0, pi/2]: Taylor polynomials to h^13 and h^14 (remainder below 1e-9)
+__device__ __forceinline__ float sin_quarter(float h) {
+  const float s = h * h;
+  float p = fmaf(s, 1.0f / 6227020800.0f, -1.0f / 39916800.0f);
+  p = fmaf(s, p, 1.0f / 362880.0f);
+  p = fmaf(s, p, -1.0f / 5040.0f);
+  p = fmaf(s, p, 1.0f / 120.0f);
+  p = fmaf(s, p, -1.0f / 6.0f);
+  return fmaf(h * s, p, h);
+}
+__device__ __forceinline__ float cos_quarter(float h) {
+  const float s = h * h;
+  float p = fmaf(s, -1.0f / 87178291200.0f, 1.0f / 479001600.0f);
+  p = fmaf(s, p, -1.0f / 3628800.0f);
+  p = fmaf(s, p, 1.0f / 40320.0f);
+  p = fmaf(s, p, -1.0f / 720.0f);
+  p = fmaf(s, p, 1.0f / 24.0f);
+  p = fmaf(s, p, -0.5f);
+  return fmaf(s, p, 1.0f);
+}
+
+// gpi dE/da_i P4 with gpi = a_i^2 / 166.0 (gbff.cpp:1772), dE/da from its fixed-point sum
 __device__ __forceinline__ float chain_weight(const double *__restrict__ born, const long long *__restrict__ deda,
                                               int i, float P4) {
   const double a = born[i];
@@ -482,146 +211,563 @@ __device__ __forceinline__ float chain_weight(const double *__restrict__ born, c
   return (float)(gpi * ((double)deda[i] * (1.0 / kFixScale)) * (double)P4);
 }
 
-// ---- pass 3: Born-radius chain rule ------------------------------------------------
-template <int SPLIT>
-__global__ __launch_bounds__(64 * SPLIT) void k_gb_chain(GBK K, const GBWork *__restrict__ work, const GBSys *__restrict__ sys,
-                                                 const double *__restrict__ x, const double *__restrict__ y,
-                                                 const double *__restrict__ z, const float *__restrict__ gbrad,
-                                                 const float *__restrict__ Vj, const double *__restrict__ born,
-                                                 const long long *__restrict__ deda,
-                                                 const int8_t *__restrict__ band, const int *__restrict__ sp_off,
-                                                 const int *__restrict__ sp_part, const int *__restrict__ sp_ord,
-                                                 long long *__restrict__ fx, long long *__restrict__ fy,
-                                                 long long *__restrict__ fz) {
-  __shared__ double sx[kTile], sy[kTile], sz[kTile];
-  __shared__ float sxf[kTile], syf[kTile], szf[kTile];
-  __shared__ float sR[kTile], sV[kTile], sW[kTile];
-  __shared__ float ax[SPLIT][kTile], ay[SPLIT][kTile], az[SPLIT][kTile];
-  __shared__ float ip[SPLIT][3][kTile];
-  const GBWork w = work[blockIdx.x];
-  const GBSys S = sys[w.sys];
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const int end = S.first + S.count;
-  const int ni = min(kTile, end - w.i0), nj = min(kTile, end - w.j0);
-  const bool diag = w.i0 == w.j0;
-  const int i = w.i0 + lane;
-  const bool iv = lane < ni;
-  const double xi = iv ? x[i] : 0.0, yi = iv ? y[i] : 0.0, zi = iv ? z[i] : 0.0;
-  const float Ri = iv ? gbrad[i] : 0.0f, Vi = iv ? Vj[i] : 0.0f, Wi = iv ? chain_weight(born, deda, i, K.P4) : 0.0f;
-  double x0, y0, z0;
-  bool fast;
-  {
-    const int j = w.j0 + lane;
-    const bool v = lane < nj;
-    const double xj = v ? x[j] : 0.0, yj = v ? y[j] : 0.0, zj = v ? z[j] : 0.0;
-    const double bd = tile_bound(xi, yi, zi, iv, xj, yj, zj, v, x0, y0, z0);
-    fast = bd * bd < K.still2;
-    if (wv == 0) {
-      sx[lane] = xj;
-      sy[lane] = yj;
-      sz[lane] = zj;
-      sxf[lane] = (float)(xj - x0);
-      syf[lane] = (float)(yj - y0);
-      szf[lane] = (float)(zj - z0);
-      sR[lane] = v ? gbrad[j] : 0.0f;
-      sV[lane] = v ? Vj[j] : 0.0f;
-      sW[lane] = v ? chain_weight(born, deda, j, K.P4) : 0.0f;
-    }
-    ax[wv][lane] = ay[wv][lane] = az[wv][lane] = 0.0f;
-  }
-  const float xif = (float)(xi - x0), yif = (float)(yi - y0), zif = (float)(zi - z0);
-  __syncthreads();
-  float fix = 0.0f, fiy = 0.0f, fiz = 0.0f;
-  auto tile = [&](auto fast_c) {
-  constexpr bool FAST = decltype(fast_c)::value;
-  for (int t = wv * (kTile / SPLIT); t < (wv + 1) * (kTile / SPLIT); t++) {
-    const int jj = (lane + t) & (kTile - 1);
-    bool on = tile_pair_valid(lane, t, ni, nj, diag, jj);
-    float dxf, dyf, dzf, r2raw;
-    if (FAST) {
-      dxf = sxf[jj] - xif;
-      dyf = syf[jj] - yif;
-      dzf = szf[jj] - zif;
-      r2raw = dxf * dxf + dyf * dyf + dzf * dzf;
-    } else {
-      double dx, dy, dz, r2;
-      {
-#pragma clang fp contract(off)
-        dx = sx[jj] - xi;
-        dy = sy[jj] - yi;
-        dz = sz[jj] - zi;
-        r2 = dx * dx + dy * dy + dz * dz;  // gbff.cpp:1789-1792
-      }
-      on = on && r2 <= K.still2;
-      dxf = (float)dx;
-      dyf = (float)dy;
-      dzf = (float)dz;
-      r2raw = (float)r2;
-    }
-    if (w.special && on) {
-      const int bo = gb_bond_order(i - S.first, w.j0 + jj - S.first, S.mid, band + S.band_off,
-                                   sp_off + S.sp_base, sp_part, sp_ord);
-      on = bo > 2;
-    }
-    const float r2f = on ? r2raw : 1.0f;
-    const float Rs = Ri + sR[jj];
-    const float rdivR = r2f * __builtin_amdgcn_rcpf(Rs * Rs);
-    float ccf = 1.0f, dccf = 0.0f;
-    if (rdivR <= K.invP5) {
-      const float th = rdivR * K.P5 * K.pi;
-      float sn, cs;
-      sincosf(th, &sn, &cs);
-      const float sq = 0.5f - 0.5f * cs;
-      ccf = sq * sq;
-      dccf = 2.0f * sq * sn * th;
-    }
-    // both directions of the pair: gpi deda_i P4 Vj + gpj deda_j P4 Vi
-    const float r6 = r2f * r2f * r2f;
-    const float dedr = on ? (Wi * sV[jj] + sW[jj] * Vi) * (4.0f * ccf - dccf) * __builtin_amdgcn_rcpf(r6) : 0.0f;
-    const float gx = dedr * dxf, gy = dedr * dyf, gz = dedr * dzf;
-    fix -= gx;  // dedi_i += dedr (p_j - p_i); force = -dedi
-    fiy -= gy;
-    fiz -= gz;
-    ax[wv][jj] += gx;
-    ay[wv][jj] += gy;
-    az[wv][jj] += gz;
-  }
-  };
-  if (fast)
-    tile(std::true_type{});
-  else
-    tile(std::false_type{});
-  ip[wv][0][lane] = fix;
-  ip[wv][1][lane] = fiy;
-  ip[wv][2][lane] = fiz;
-  __syncthreads();
-  if (wv != 0) return;
-  float si[3] = {ip[0][0][lane], ip[0][1][lane], ip[0][2][lane]};
-  float sj[3] = {ax[0][lane], ay[0][lane], az[0][lane]};
-#pragma unroll
-  for (int k = 1; k < SPLIT; k++) {
-#pragma unroll
-    for (int c = 0; c < 3; c++) si[c] += ip[k][c][lane];
-    sj[0] += ax[k][lane];
-    sj[1] += ay[k][lane];
-    sj[2] += az[k][lane];
-  }
-  if (iv) {
-    fix_add(&fx[i], fix_from_float(si[0]));
-    fix_add(&fy[i], fix_from_float(si[1]));
-    fix_add(&fz[i], fix_from_float(si[2]));
-  }
-  if (lane < nj) {
-    const int j = w.j0 + lane;
-    fix_add(&fx[j], fix_from_float(sj[0]));
-    fix_add(&fy[j], fix_from_float(sj[1]));
-    fix_add(&fz[j], fix_from_float(sj[2]));
-  }
+// max(a, |b|), NaN if b is
+__device__ __forceinline__ float fmax_nan(float a, float b) { return fabsf(b) <= a ? a : fabsf(b); }
+
+// 1 / r^2 to FP32 rounding: r2f the rounded r^2, r2lo what the rounding took.  The LJ
+// terms raise it to the 6th and 7th power; taken from the hardware's reciprocal square
+// root (1 ulp, biased) its error was the largest part of the forces' error.
+__device__ __forceinline__ float rcp_near(float r2f, float r2lo) {
+  const float y = __builtin_amdgcn_rcpf(r2f);
+  return fmaf(y, fmaf(-r2lo, y, fmaf(-r2f, y, 1.0f)), y);
 }
 
-__global__ void k_zero_ll1(long long *__restrict__ a, int n) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) a[i] = 0;
+__device__ __forceinline__ void lds_add(long long *p, long long v) {
+  atomicAdd(reinterpret_cast<unsigned long long *>(p), static_cast<unsigned long long>(v));
+}
+
+// The passes.  kGbFast: FastMode's calcForcesIncludingVacuo, above.
+// kGbEnergy: FF_GeneralizedBorn_Still::calcEnergies instead (gbff.cpp:178-183,
+// 537-596): the exact GB cross term on every pair within Cutoff, whatever its bond
+// order and with no ExpApproxThreshold swap, plus FF_NonBonded::calcEnergies with
+// Dielectric = DielectricSolute and energy switching; no forces, no dE/da.
+// kGbBorn: calcForces with FastMode off (gbff.cpp:186-196): FF_NonBonded::
+// calcForces with Dielectric = DielectricSolute and energy switching, and the cross
+// term of calcBornForces (gbff.cpp:1189-1345) on every pair within Cutoff, with
+// 1/r in place of 1/f_GB (and no dE/da) where uGB <= ExpApproxThreshold.
+enum { kGbFast = 0, kGbEnergy = 1, kGbBorn = 2, kGbRadii = 3, kGbChain = 4 };
+
+// Sums of a pass per atom: forces x, y, z and dE/da (pair), Gpol (radii), forces (chain).
+constexpr int gb_sums(int pass) { return pass == kGbRadii ? 1 : (pass == kGbChain ? 3 : (pass == kGbEnergy ? 0 : 4)); }
+
+// One workgroup of SPLIT wavefronts per task: one or two i tiles against a run of j
+// tiles.  The wavefronts share the staged j tile and take its chunks of 16 steps in
+// turn.  Per-pair FP32 arithmetic; FP32 sums over a chunk, fixed point beyond it; the
+// energies FP32 over 8 steps, then FP64.
+template <int PASS, int SPLIT>
+__global__ __launch_bounds__(64 * SPLIT) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_gb_pass(GBPassArgs A) {
+  constexpr int NS = gb_sums(PASS);
+  constexpr bool PAIR = PASS == kGbFast || PASS == kGbEnergy || PASS == kGbBorn;
+  constexpr int T = 64 * SPLIT;
+  const GBK K = A.K;
+  // the j tile: far loops read the records at lane + t < 128 (each atom twice, no
+  // wrap), near loops the FP64 positions and two records at (lane + t) & 63
+  __shared__ __align__(16) union Stage {
+    struct {
+      float4 a[2 * kTile];  // x, y, z (about the tiles' midpoint) and q | V | V
+      float2 b[2 * kTile];  // LJ radius, sqrt(eps) | - | W, -
+    } far;
+    struct {
+      double x[kTile], y[kTile], z[kTile];
+      float2 p01[kTile], p23[kTile], ia[kTile];  // q, LJ radius, sqrt(eps), a | R, V | R, V, W; 1 / a
+    } near;
+  } st;
+  __shared__ long long jacc[NS > 0 ? NS : 1][kTile], iacc[2][NS > 0 ? NS : 1][kTile];
+  __shared__ double es[SPLIT][3];
+  const GBTask w = A.tasks[blockIdx.x];
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+
+  // An atom's position and parameters; a pad (i < 0) has zero parameters and sits far
+  // from everything.  Read again for each tile pair: kept, they would cost the loops
+  // the registers that let four wavefronts share a SIMD.
+  struct Atom {
+    double x, y, z;
+    float p0, p1, p2, p3;  // q, LJ radius, sqrt(eps), a | R, V | R, V, W
+  };
+  auto atom = [&](int i, double pad) __attribute__((always_inline)) {
+    Atom P{pad, pad, pad, 0.0f, 0.0f, 0.0f, 1.0f};
+    if (i >= 0) {
+      P.x = A.x[i];
+      P.y = A.y[i];
+      P.z = A.z[i];
+      if (PAIR) {
+        P.p0 = A.q[i];
+        P.p1 = A.ljr[i];
+        P.p2 = A.lje[i];
+        P.p3 = A.bornf[i];
+      } else {
+        P.p0 = A.gbrad[i];
+        P.p1 = A.Vj[i];
+        if (PASS == kGbChain) P.p2 = chain_weight(A.born, A.deda_in, i, K.P4);
+      }
+    }
+    return P;
+  };
+  auto lane_atom = [&](int tile) __attribute__((always_inline)) {
+    const int2 at = A.tile_atoms[tile];
+    return lane < at.y ? at.x + lane : -1;
+  };
+  for (int k = tid; k < 2 * NS * kTile; k += T) (&iacc[0][0][0])[k] = 0;
+  double epol = 0.0, evdw = 0.0, eel = 0.0, efar = 0.0;  // eel: without econv / eps_solute
+  // dE/da carries premul, Gpol P4: applied in FP64 as a chunk goes to fixed point
+  const double scale_d = K.premul_d, scale_g = (double)K.P4;
+  auto sum_of = [&](int c) { return c == 0 ? A.s0 : (c == 1 ? A.s1 : (c == 2 ? A.s2 : A.s3)); };
+  // A chunk's sums of one kind to fixed point.  scale * v + 1.5 2^52 holds round(scale v)
+  // in its low bits while |scale v| < 2^51: two FP64 instructions a value against seven,
+  // and the constant leaves with one subtraction; larger sums (atoms on top of each
+  // other) take the long way.
+  auto scale_of = [&](int c) {
+    return (PASS == kGbRadii ? scale_g : (PAIR && c == 3 ? scale_d : 1.0)) * kFixScale;
+  };
+  auto to_fix = [&](int c, float v, bool big) __attribute__((always_inline)) -> long long {
+    if (big) return fix_from_double((double)v * (scale_of(c) / kFixScale));
+    constexpr double kMagic = 6755399441055744.0;
+    return __double_as_longlong(fma((double)v, scale_of(c), kMagic)) - __double_as_longlong(kMagic);
+  };
+  // wave-uniform: some sum of the chunk is too large (or not a number) for the short way
+  auto any_big = [&](float m) __attribute__((always_inline)) { return __ballot(!(m < K.fix_lim)) != 0ull; };
+
+  for (int tj = w.tj; tj < w.tj + w.nj; tj++) {
+    // ---- what the geometry of the tile pairs allows ---------------------------------
+    const GBTile B = A.tiles[tj];
+    bool far[2] = {false, false}, inside[2] = {false, false}, live[2] = {false, false};
+#pragma unroll
+    for (int m = 0; m < 2; m++) {
+      if (m >= w.ni) continue;
+      const GBTile &C = A.tiles[w.ti + m];
+      // FP32 from here on: the margins (1e-3 A and 1e-4 of the distances) are far wider
+      // than its rounding
+      const float dx = (float)(C.x - B.x), dy = (float)(C.y - B.y), dz = (float)(C.z - B.z);
+      const float d = __builtin_amdgcn_sqrtf(dx * dx + dy * dy + dz * dz);
+      const float rb = (float)B.rad, reach = (float)C.rad + rb + 1e-3f;
+      // every pair's distance is within [lo, hi]
+      const float lo = d * (1.0f - 1e-4f) - reach, hi = d * (1.0f + 1e-4f) + reach;
+      inside[m] = hi < K.inside;
+      live[m] = !(lo > K.outside);
+      if (PASS == kGbEnergy || PASS == kGbBorn || w.code >= 0 || !inside[m]) continue;
+      // Far: each i atom lies beyond the short-range reach of every j atom, by its
+      // distance from the j tile's sphere.  Pair pass: uGB = -r^2 / 4 a_i a_j <=
+      // threshold; radii and chain: r^2 / (Ri + Rj)^2 > 1 / P5, where CCF is 1.
+      const int i = lane_atom(w.ti + m);
+      bool beyond = true;
+      if (i >= 0) {
+        const float ex = (float)(A.x[i] - B.x), ey = (float)(A.y[i] - B.y), ez = (float)(A.z[i] - B.z);
+        const float e = __builtin_amdgcn_sqrtf(ex * ex + ey * ey + ez * ez);
+        float need;
+        if (PAIR) {
+          const float a = A.bornf[i];
+          need = a > 0.0f ? __builtin_amdgcn_sqrtf(K.far_k * a * B.amax) : 1e30f;
+        } else {
+          need = K.far_k * (A.gbrad[i] + B.rmax);
+        }
+        beyond = e * (1.0f - 1e-4f) > need + rb + 1e-3f;
+      }
+      far[m] = (!PAIR || K.thresh < 0.0f) && __ballot(!beyond) == 0ull;
+    }
+    const bool both = far[0] && far[1];
+    __syncthreads();  // the previous tile's sums are flushed, its stage is read
+    for (int k = tid; k < NS * kTile; k += T) (&jacc[0][0])[k] = 0;
+    // the chunks of a tile pair; a diagonal one ends at step 32
+    const int nch = tj == w.ti ? 3 : kTile / kChunk;
+
+    // ---- the far loop over a j tile: one i tile or both ------------------------------
+    auto far_loop = [&](auto ni_c, int m0, double ox, double oy, double oz) __attribute__((always_inline)) {
+      constexpr int NI = decltype(ni_c)::value;  // m0 (uniform): the i tile when it is one
+      float px[NI], py[NI], pz[NI], p0[NI], p1[NI], p2[NI];
+#pragma unroll
+      for (int n = 0; n < NI; n++) {
+        const Atom P = atom(lane_atom(w.ti + (NI == 2 ? n : m0)), 5.0e3);
+        px[n] = (float)(P.x - ox);
+        py[n] = (float)(P.y - oy);
+        pz[n] = (float)(P.z - oz);
+        p0[n] = PAIR ? P.p0 * K.ec_out : P.p0;
+        p1[n] = P.p1;
+        p2[n] = P.p2;
+      }
+      for (int c = wv; c < nch; c += SPLIT) {
+      float fx[NI], fy[NI], fz[NI];
+      float ax = 0.0f, ay = 0.0f, az = 0.0f;
+#pragma unroll
+      for (int n = 0; n < NI; n++) fx[n] = fy[n] = fz[n] = 0.0f;
+      const int base = lane + c * kChunk;
+      for (int h = 0; h < kChunk; h += 8) {
+        float ev8 = 0.0f, el8 = 0.0f;
+#pragma unroll 2
+        for (int u = 0; u < 8; u++) {
+          const float4 a = st.far.a[base + h + u];
+          float2 b = make_float2(0.0f, 0.0f);
+          if (PASS != kGbRadii) b = st.far.b[base + h + u];
+          float gx = 0.0f, gy = 0.0f, gz = 0.0f;
+#pragma unroll
+          for (int n = 0; n < NI; n++) {
+            const float dx = px[n] - a.x, dy = py[n] - a.y, dz = pz[n] - a.z;
+            const float r2 = dx * dx + dy * dy + dz * dz;
+            float g;
+            if (PASS == kGbRadii) {
+              const float v = __builtin_amdgcn_rcpf(r2 * r2);
+              fx[n] = fmaf(v, a.w, fx[n]);
+              gx = n == 0 ? v * p1[n] : fmaf(v, p1[n], gx);
+              continue;
+            } else if (PASS == kGbChain) {
+              // -(gpi dE/da_i P4 Vj + gpj dE/da_j P4 Vi) 4 / r^6
+              g = -4.0f * fmaf(p2[n], a.w, b.x * p1[n]) * __builtin_amdgcn_rcpf(r2 * r2 * r2);
+            } else {
+              const float rinv = __builtin_amdgcn_rsqf(r2);
+              const float ri2 = rinv * rinv;
+              const float e = p0[n] * a.w * rinv;
+              const float s = (p1[n] + b.x) * rinv;
+              const float s2 = s * s;
+              const float Bq = s2 * s2 * s2;
+              const float eB = p2[n] * b.y * Bq;
+              const float v = fmaf(eB, Bq, -eB);  // eps (B^2 - B)
+              el8 += e;
+              ev8 += v - eB;
+              g = -fmaf(12.0f, v, e) * ri2;
+            }
+            fx[n] = fmaf(-g, dx, fx[n]);
+            fy[n] = fmaf(-g, dy, fy[n]);
+            fz[n] = fmaf(-g, dz, fz[n]);
+            gx = n == 0 ? g * dx : fmaf(g, dx, gx);
+            gy = n == 0 ? g * dy : fmaf(g, dy, gy);
+            gz = n == 0 ? g * dz : fmaf(g, dz, gz);
+          }
+          ax = rotate1(ax) + gx;
+          if (PASS != kGbRadii) {
+            ay = rotate1(ay) + gy;
+            az = rotate1(az) + gz;
+          }
+        }
+        if (PAIR) {
+          evdw += (double)ev8;
+          efar += (double)el8;
+        }
+      }
+      const int jj = (base + kChunk - 1) & (kTile - 1);
+      const float s_j[3] = {ax, ay, az};
+      float big = 0.0f;
+#pragma unroll
+      for (int k = 0; k < (NS >= 3 ? 3 : 1); k++) {
+        big = fmax_nan(big, s_j[k]);
+#pragma unroll
+        for (int n = 0; n < NI; n++) big = fmax_nan(big, k == 0 ? fx[n] : (k == 1 ? fy[n] : fz[n]));
+      }
+      auto flush = [&](bool slow) __attribute__((always_inline)) {
+#pragma unroll
+        for (int k = 0; k < (NS >= 3 ? 3 : 1); k++) {
+          lds_add(&jacc[k][jj], to_fix(k, s_j[k], slow));
+#pragma unroll
+          for (int n = 0; n < NI; n++)
+            lds_add(&iacc[NI == 2 ? n : m0][k][lane], to_fix(k, k == 0 ? fx[n] : (k == 1 ? fy[n] : fz[n]), slow));
+        }
+      };
+      if (any_big(big))
+        flush(true);
+      else
+        flush(false);
+      }
+    };
+
+    // ---- the near loop: one i tile ----------------------------------------------------
+    auto near_loop = [&](auto coded_c, auto inside_c, int m) __attribute__((always_inline)) {
+      constexpr bool CODED = decltype(coded_c)::value, IN = decltype(inside_c)::value;
+      const Atom P = atom(lane_atom(w.ti + m), 5.0e3);
+      const double qx = P.x, qy = P.y, qz = P.z;
+      const float p0 = P.p0, p1 = P.p1, p2 = P.p2, p3 = P.p3;
+      const float quarter = 0.25f / p3;
+      for (int c = wv; c < nch; c += SPLIT) {
+      unsigned cw = CODED ? A.codes[((size_t)w.code * (kTile / kChunk) + c) * kTile + lane] : 0u;
+      float fx = 0.0f, fy = 0.0f, fz = 0.0f, fd = 0.0f, ax = 0.0f, ay = 0.0f, az = 0.0f, ad = 0.0f;
+      for (int h = 0; h < kChunk; h += 8) {
+        float ep8 = 0.0f, ev8 = 0.0f, el8 = 0.0f;
+        // two steps at a time: the arithmetic of two pairs overlaps, and the short-range
+        // part of the pass, which few steps need, is behind one branch for the wavefront
+#pragma unroll 1
+        for (int u2 = 0; u2 < 8; u2 += 2) {
+          double r2d[2];
+          float dx[2], dy[2], dz[2], r2f[2];
+          float2 a01[2], a23[2], aia[2];
+          bool on[2], on_gb[2], nb[2], s14[2], lj[2];
+#pragma unroll
+          for (int v = 0; v < 2; v++) {
+            const int jj = (lane + c * kChunk + h + u2 + v) & (kTile - 1);
+            const unsigned code = CODED ? cw & 3u : (unsigned)kPairPlain;
+            if (CODED) cw >>= 2;
+            const bool valid = !CODED || code != kPairNone;
+            double r2 = 0.0;
+            {
+#pragma clang fp contract(off)
+              const double ex = qx - st.near.x[jj], ey = qy - st.near.y[jj], ez = qz - st.near.z[jj];
+              if (PAIR || !IN) r2 = ex * ex + ey * ey + ez * ez;  // PD's expression (gbff.cpp:455, 1588-1591)
+              dx[v] = (float)ex;
+              dy[v] = (float)ey;
+              dz[v] = (float)ez;
+            }
+            r2f[v] = !PAIR && IN ? dx[v] * dx[v] + dy[v] * dy[v] + dz[v] * dz[v] : (float)r2;
+            a01[v] = st.near.p01[jj];
+            if (PASS != kGbRadii) a23[v] = st.near.p23[jj];
+            r2d[v] = r2;
+            if (PAIR) {
+              aia[v] = st.near.ia[jj];
+              on[v] = valid && (IN || r2 <= K.cut2);
+              // calcBornEnergy's test on the distance (gbff.cpp:560)
+              on_gb[v] = PASS == kGbEnergy ? valid && (IN || r2 < K.gb_lim) : on[v];
+              // vdW and Coulomb only for non-bonded and 1-4 pairs
+              nb[v] = on[v] && (!CODED || code < kPairBonded);
+              s14[v] = CODED && code == kPair14;
+              lj[v] = nb[v] && (IN || r2 < K.vdw_lim);  // Dist_ij < VdwCutoff (gbff.cpp:1686)
+              if (!(on[v] || on_gb[v])) r2d[v] = r2f[v] = 1.0f;
+            } else {
+              // only non-bonded and 1-4 partners (gbff.cpp:460-461)
+              on[v] = (!CODED || code < kPairBonded) && (IN || r2 <= K.still2);
+              r2f[v] = on[v] ? r2f[v] : 1.0f;
+            }
+          }
+          if (!PAIR) {
+            // CCF = (0.5 - 0.5 cos th)^2 = sin(th/2)^4 with th = pi P5 r^2 / (Ri + Rj)^2,
+            // dccf = 2 (0.5 - 0.5 cos th) sin th th; 1 and 0 beyond r^2 / (Ri + Rj)^2 = 1 / P5
+            float rdivR[2], ccf[2], f4[2];  // f4: 4 CCF - dccf
+#pragma unroll
+            for (int v = 0; v < 2; v++) {
+              const float Rs = p0 + a01[v].x;
+              rdivR[v] = r2f[v] * __builtin_amdgcn_rcpf(Rs * Rs);
+              ccf[v] = 1.0f;
+              f4[v] = 4.0f;
+            }
+            if (__ballot(rdivR[0] <= K.invP5 || rdivR[1] <= K.invP5) != 0ull) {
+#pragma unroll
+              for (int v = 0; v < 2; v++) {
+                const bool close = rdivR[v] <= K.invP5;
+                const float hf = close ? rdivR[v] * K.half_pi_P5 : 0.0f;
+                const float sn = sin_quarter(hf);
+                const float s3 = sn * sn * sn;
+                ccf[v] = close ? s3 * sn : 1.0f;
+                if (PASS == kGbChain) f4[v] = fmaf(4.0f, ccf[v], -8.0f * hf * s3 * cos_quarter(hf));
+              }
+            }
+#pragma unroll
+            for (int v = 0; v < 2; v++) {
+              if (PASS == kGbRadii) {
+                const float e = on[v] ? ccf[v] * __builtin_amdgcn_rcpf(r2f[v] * r2f[v]) : 0.0f;
+                fx = fmaf(e, a01[v].y, fx);
+                ax = rotate1(ax) + e * p1;
+              } else {
+                // both directions of the pair: gpi deda_i P4 Vj + gpj deda_j P4 Vi
+                const float g = on[v] ? -fmaf(p2, a01[v].y, a23[v].x * p1) * f4[v] *
+                                            __builtin_amdgcn_rcpf(r2f[v] * r2f[v] * r2f[v])
+                                      : 0.0f;
+                fx = fmaf(-g, dx[v], fx);
+                fy = fmaf(-g, dy[v], fy);
+                fz = fmaf(-g, dz[v], fz);
+                ax = rotate1(ax) + g * dx[v];
+                ay = rotate1(ay) + g * dy[v];
+                az = rotate1(az) + g * dz[v];
+              }
+            }
+          } else {
+            float rinv[2], r[2], qq[2], uGB[2], dS[2], Sw[2];
+            // ep, dal: without premul; gg: (dE/dr) / r of the cross term without premul
+            float ep[2], dal[2], gg[2], ratio[2];
+            bool close[2], edge[2];
+#pragma unroll
+            for (int v = 0; v < 2; v++) {
+              rinv[v] = __builtin_amdgcn_rsqf(r2f[v]);
+              r[v] = r2f[v] * rinv[v];
+              qq[v] = (PASS == kGbEnergy || on[v]) ? p0 * a01[v].x : 0.0f;
+              uGB[v] = -r2f[v] * (quarter * aia[v].x);
+              close[v] = PASS == kGbEnergy ? on_gb[v] : on[v] && uGB[v] > K.thresh;
+              edge[v] = PASS != kGbEnergy && on[v] && fabsf(uGB[v] - K.thresh) < K.edge;
+              ep[v] = dal[v] = gg[v] = 0.0f;
+              // switching (r >= InnerCutoff), gbff.cpp:1640-1651; none inside
+              dS[v] = 0.0f;
+              Sw[v] = 1.0f;
+              if (!IN) {
+                const float t = fmaxf(r[v] - K.inner, 0.0f);
+                const float S0 = 1.0f - (K.invw * t) * (K.invw * t);
+                dS[v] = -K.invw2_4 * t * S0;
+                Sw[v] = S0 * S0;
+              }
+            }
+            // a pair at the threshold (where the terms jump) is decided in FP64, as PD does
+            if (PASS != kGbEnergy && __builtin_expect(__ballot(edge[0] || edge[1]) != 0ull, 0)) {
+              const int at = A.tile_atoms[tj].x, i = lane_atom(w.ti + m);
+#pragma unroll
+              for (int v = 0; v < 2; v++)
+                if (edge[v]) {
+                  const int jj = (lane + c * kChunk + h + u2 + v) & (kTile - 1);
+                  close[v] = -r2d[v] * 0.25 / (A.born[i] * A.born[at + jj]) > (double)K.thresh;
+                }
+            }
+            if (PASS != kGbFast || __ballot(close[0] || close[1]) != 0ull) {
+#pragma unroll
+              for (int v = 0; v < 2; v++) {
+                const float aiaj = p3 * a23[v].y;
+                if (PASS == kGbEnergy) {
+                  ep[v] = close[v] ? qq[v] * __builtin_amdgcn_rsqf(r2f[v] + aiaj * __expf(uGB[v])) * Sw[v] : 0.0f;
+                } else {
+                  // 1 / f_GB, 1 ulp; kGbBorn: 1 / r beyond the threshold (tg = 0 gives it)
+                  const float tg = close[v] ? __expf(uGB[v]) : 0.0f;
+                  const float f = __builtin_amdgcn_rsqf(fmaf(tg, aiaj, r2f[v]));
+                  const float e0 = (close[v] || PASS == kGbBorn) ? qq[v] * f : 0.0f;
+                  const float el = e0 * (f * f);
+                  gg[v] = -el * fmaf(-0.25f, tg, 1.0f);
+                  dal[v] = -el * tg * (1.0f - uGB[v]);
+                  dal[v] = close[v] ? dal[v] : 0.0f;
+                  ep[v] = e0;
+                  if (!IN) {
+                    gg[v] = fmaf(Sw[v], gg[v], dS[v] * e0 * rinv[v]);
+                    dal[v] *= Sw[v];
+                    ep[v] *= Sw[v];
+                  }
+                }
+              }
+            }
+#pragma unroll
+            for (int v = 0; v < 2; v++) {
+              const float ri2 = rcp_near(r2f[v], (float)(r2d[v] - (double)r2f[v]));
+              // eps_solvent where FastMode drops the GB term
+              ratio[v] = PASS == kGbFast && !close[v] ? K.ec_ratio : 1.0f;
+              // Ee, Fe: without econv / eps_solute; Fe, Fv: (dE/dr) / r
+              const float e1 = nb[v] ? qq[v] * (s14[v] ? K.elec14 : 1.0f) * rinv[v] * ratio[v] : 0.0f;
+              float Ee = e1, Fe = -e1 * ri2;
+              if (!IN) {
+                Fe = fmaf(Sw[v], Fe, dS[v] * e1 * rinv[v]);
+                Ee *= Sw[v];
+              }
+              const float eps = (s14[v] ? K.vdw14 : 1.0f) * p2 * a23[v].x;
+              const float s = p1 + a01[v].y;
+              const float s2 = s * s * ri2;
+              const float Bq = s2 * s2 * s2;
+              const float eB = lj[v] ? eps * Bq : 0.0f;
+              const float w2 = fmaf(eB, Bq, -eB);
+              float Ev = w2 - eB, Fv = -12.0f * w2 * ri2;
+              if (!IN) {
+                const float t = fmaxf(r[v] - K.vdwinner, 0.0f);
+                const float V0 = 1.0f - (K.vinvw * t) * (K.vinvw * t);
+                const float vdS = -K.vinvw2_4 * t * V0;
+                const float VS = V0 * V0;
+                Fv = fmaf(VS, Fv, Ev * vdS * rinv[v]);
+                Ev *= VS;
+              }
+              ep8 += ep[v];
+              ev8 += Ev;
+              el8 += Ee;
+              if (PASS == kGbEnergy) continue;
+              // along d = p_i - p_j: twice the cross term, vdW and Coulomb
+              const float g = fmaf(K.premul2, gg[v], fmaf(K.ec_in, Fe, Fv));
+              fd = fmaf(dal[v], a23[v].y, fd);
+              ad = rotate1(ad) + dal[v] * p3;
+              fx = fmaf(-g, dx[v], fx);
+              fy = fmaf(-g, dy[v], fy);
+              fz = fmaf(-g, dz[v], fz);
+              ax = rotate1(ax) + g * dx[v];
+              ay = rotate1(ay) + g * dy[v];
+              az = rotate1(az) + g * dz[v];
+            }
+          }
+        }
+        if (PAIR) {
+          epol += (double)ep8;
+          evdw += (double)ev8;
+          eel += (double)el8;
+        }
+      }
+      if constexpr (NS > 0) {
+        const int jj = (lane + c * kChunk + kChunk - 1) & (kTile - 1);
+        const float s_i[4] = {fx, fy, fz, fd}, s_j[4] = {ax, ay, az, ad};
+        float big = 0.0f;
+#pragma unroll
+        for (int k = 0; k < NS; k++) big = fmax_nan(fmax_nan(big, s_i[k]), s_j[k]);
+        auto flush = [&](bool slow) __attribute__((always_inline)) {
+#pragma unroll
+          for (int k = 0; k < NS; k++) {
+            lds_add(&jacc[k][jj], to_fix(k, s_j[k], slow));
+            lds_add(&iacc[m][k][lane], to_fix(k, s_i[k], slow));
+          }
+        };
+        if (any_big(big))
+          flush(true);
+        else
+          flush(false);
+      }
+      }
+    };
+
+    auto stage_far = [&](double ox, double oy, double oz) {
+      if (wv == 0) {
+        const Atom P = atom(lane_atom(tj), -5.0e3);
+        const float4 a =
+            make_float4((float)(P.x - ox), (float)(P.y - oy), (float)(P.z - oz), PAIR ? P.p0 : P.p1);
+        const float2 b = PAIR ? make_float2(P.p1, P.p2) : make_float2(P.p2, 0.0f);
+        st.far.a[lane] = a;
+        st.far.a[lane + kTile] = a;
+        if (PASS != kGbRadii) {
+          st.far.b[lane] = b;
+          st.far.b[lane + kTile] = b;
+        }
+      }
+    };
+    if (both) {
+      const GBTile C0 = A.tiles[w.ti], C1 = A.tiles[w.ti + 1];
+      const double ox = 0.25 * (C0.x + C1.x) + 0.5 * B.x, oy = 0.25 * (C0.y + C1.y) + 0.5 * B.y,
+                   oz = 0.25 * (C0.z + C1.z) + 0.5 * B.z;
+      stage_far(ox, oy, oz);
+      __syncthreads();
+      far_loop(std::integral_constant<int, 2>{}, 0, ox, oy, oz);
+    } else {
+      for (int m = 0; m < w.ni; m++) {
+        const bool in = m ? inside[1] : inside[0];
+        if (!(m ? live[1] : live[0])) continue;  // uniform over the workgroup
+        if (m == 1) __syncthreads();             // the first tile's stage is read
+        if (m ? far[1] : far[0]) {
+          const GBTile C = A.tiles[w.ti + m];
+          const double ox = 0.5 * (C.x + B.x), oy = 0.5 * (C.y + B.y), oz = 0.5 * (C.z + B.z);
+          stage_far(ox, oy, oz);
+          __syncthreads();
+          far_loop(std::integral_constant<int, 1>{}, m, ox, oy, oz);
+          continue;
+        }
+        if (wv == 0) {
+          const Atom P = atom(lane_atom(tj), -5.0e3);
+          st.near.x[lane] = P.x;
+          st.near.y[lane] = P.y;
+          st.near.z[lane] = P.z;
+          st.near.p01[lane] = make_float2(P.p0, P.p1);
+          if (PASS != kGbRadii) st.near.p23[lane] = make_float2(P.p2, P.p3);
+          if (PAIR) st.near.ia[lane] = make_float2(1.0f / P.p3, 0.0f);
+        }
+        __syncthreads();
+        if (w.code >= 0)
+          in ? near_loop(std::true_type{}, std::true_type{}, m) : near_loop(std::true_type{}, std::false_type{}, m);
+        else
+          in ? near_loop(std::false_type{}, std::true_type{}, m) : near_loop(std::false_type{}, std::false_type{}, m);
+      }
+    }
+    if constexpr (NS > 0) {  // this j tile's sums
+      __syncthreads();
+      const int j = lane_atom(tj);
+      for (int c = wv; c < NS; c += SPLIT) {
+        const long long v = jacc[c][lane];
+        if (j >= 0 && v != 0) fix_add(&sum_of(c)[j], v);
+      }
+    }
+  }
+  if constexpr (NS > 0) {  // the i tiles' sums (the last barrier above follows every add)
+    for (int k = wv; k < w.ni * NS; k += SPLIT) {
+      const int m = k / NS, c = k % NS;
+      const int i = lane_atom(w.ti + m);
+      const long long v = iacc[m][c][lane];
+      if (i >= 0 && v != 0) fix_add(&sum_of(c)[i], v);
+    }
+  }
+  if (PAIR) {
+    const double sp = wave_sum(epol), sv = wave_sum(evdw), sl = wave_sum(K.ec_in_d * eel + efar);
+    if (lane == 0) {
+      es[wv][0] = sp;
+      es[wv][1] = sv;
+      es[wv][2] = sl;
+    }
+    __syncthreads();
+    if (tid == 0) {
+      double e3[3] = {0.0, 0.0, 0.0};
+      for (int k = 0; k < SPLIT; k++)
+        for (int c = 0; c < 3; c++) e3[c] += es[k][c];
+      // PD adds each cross term twice (gbff.cpp:1655-1658)
+      A.e_part[4 * (size_t)w.slot + 0] = 2.0 * scale_d * e3[0];
+      A.e_part[4 * (size_t)w.slot + 1] = e3[1];
+      A.e_part[4 * (size_t)w.slot + 2] = e3[2];
+      A.e_part[4 * (size_t)w.slot + 3] = 0.0;
+    }
+  }
 }
 
 
@@ -892,11 +1038,23 @@ void GBState::set_params(const pdgpu_gb_params &p) {
   k.cut2 = p.Cutoff * p.Cutoff;
   k.cut = p.Cutoff;
   k.still2 = p.GbsaStillCutoff * p.GbsaStillCutoff;
-  k.vdwcut2 = p.VdwCutoff * p.VdwCutoff;
-  k.vdwcut = p.VdwCutoff;
-  k.premul = (float)(-Consts::halfeconv() * (1 / p.DielectricSolute - 1 / p.DielectricSolvent));
-  k.ec_in = (float)(ec / p.DielectricSolute);
+  // PD compares rounded distances: sqrt(r2) < VdwCutoff and (calcBornEnergy)
+  // sqrt(r2) <= Cutoff.  The rounded square root never decreases, so each test is
+  // r2 below one FP64 value, found here.
+  auto first_at = [](double c, auto beyond) {
+    double v = c * c;
+    while (!beyond(std::sqrt(v))) v = std::nextafter(v, HUGE_VAL);
+    while (v > 0.0 && beyond(std::sqrt(std::nextafter(v, 0.0)))) v = std::nextafter(v, 0.0);
+    return v;
+  };
+  k.vdw_lim = p.VdwCutoff > 0.0 ? first_at(p.VdwCutoff, [&](double r) { return r >= p.VdwCutoff; }) : 0.0;
+  k.gb_lim = p.Cutoff >= 0.0 ? first_at(p.Cutoff, [&](double r) { return r > p.Cutoff; }) : 0.0;
+  k.premul_d = -Consts::halfeconv() * (1 / p.DielectricSolute - 1 / p.DielectricSolvent);
+  k.ec_in_d = ec / p.DielectricSolute;
+  k.premul2 = (float)(2.0 * k.premul_d);
+  k.ec_in = (float)k.ec_in_d;
   k.ec_out = (float)(ec / p.DielectricSolvent);
+  k.ec_ratio = (float)(p.DielectricSolute / p.DielectricSolvent);
   const double w = p.Cutoff - p.InnerCutoff;
   k.inner = (float)p.InnerCutoff;
   k.invw = w > 0 ? (float)(1.0 / w) : 0.0f;
@@ -907,16 +1065,28 @@ void GBState::set_params(const pdgpu_gb_params &p) {
   k.vinvw2_4 = vw > 0 ? (float)(4.0 / (vw * vw)) : 0.0f;
   k.thresh = (float)p.ExpApproxThreshold;
   k.P4 = (float)p.P4;
-  k.P5 = (float)p.P5;
   k.invP5 = (float)(1 / p.P5);
+  k.half_pi_P5 = (float)(0.5 * Consts::PI * p.P5);
   k.vdw14 = (float)p.Vdw14Scaling;
   k.elec14 = (float)p.Elec14Scaling;
-  k.pi = (float)Consts::PI;
-  kp = k;
+  // the passes' geometry tests (k_gb_pass), for the pair pass and for radii / chain: a tile
+  // pair inside every cutoff and switching radius, one beyond the cutoff, and the reach
+  // of the short-range part (of sqrt(a_i a_j), of Ri + Rj)
+  kp = kr = k;
+  kp.inside = std::min(std::min((float)std::sqrt(k.cut2), (float)std::sqrt(k.vdw_lim)), std::min(k.inner, k.vdwinner)) - 1e-3f;
+  // a chunk sum up to here stays below 2^51 in fixed point, its factor (premul, P4) included
+  kp.fix_lim = (float)(4.0e5 / std::max(1.0, std::fabs(k.premul_d)));
+  kr.fix_lim = (float)(4.0e5 / std::max(1.0, std::fabs((double)k.P4)));
+  kp.edge = 4e-6f * std::max(1.0f, std::fabs(k.thresh));  // FP32's error of uGB is below 1e-6 of it
+  kp.outside = (float)p.Cutoff + 1e-3f;
+  kp.far_k = -4.0f * k.thresh * (1.0f + 1e-3f);
+  kr.inside = (float)p.GbsaStillCutoff - 1e-3f;
+  kr.outside = (float)p.GbsaStillCutoff + 1e-3f;
+  kr.far_k = std::sqrt(k.invP5) * (1.0f + 1e-3f);
 }
 
 // Adds one system (atoms [first, first+count) of the concatenated arrays) and
-// its tile pairs to the work list.
+// its tiles; the tasks are made from all systems in upload().
 void GBState::add_system(int first, int count, int mid, const std::vector<int8_t> &band_sys,
                          const std::vector<int> &spi, const std::vector<int> &spj, const std::vector<int> &spo) {
   GBSys S{};
@@ -934,33 +1104,77 @@ void GBState::add_system(int first, int count, int mid, const std::vector<int8_t
   std::vector<int> fill(cnt.begin(), cnt.end() - 1);
   h_sp_part.resize(part_base + spi.size());
   h_sp_ord.resize(part_base + spi.size());
-  std::vector<std::vector<int>> partner_tiles((count + kTile - 1) / kTile);
+  const int nt = (count + kTile - 1) / kTile;
+  std::vector<std::pair<int, int>> linked;  // tile pairs that hold a sparse partner
   for (size_t k = 0; k < spi.size(); k++) {
     const int lo = std::min(spi[k], spj[k]), hi = std::max(spi[k], spj[k]);
     h_sp_part[part_base + fill[lo]] = hi;
     h_sp_ord[part_base + fill[lo]] = spo[k];
     fill[lo]++;
+    linked.emplace_back(lo / kTile, hi / kTile);
   }
+  std::sort(linked.begin(), linked.end());
+  h_linked.push_back(std::move(linked));
   for (int i = 0; i <= count; i++) h_sp_off.push_back(part_base + cnt[i]);
-  const int sysi = (int)h_sys.size();
   h_sys.push_back(S);
-  // tile pairs (upper triangle); special when bond orders can differ from 7
-  const int nt = (count + kTile - 1) / kTile;
-  std::vector<char> sp_tile((size_t)nt * nt, 0);
-  for (size_t k = 0; k < spi.size(); k++) {
-    const int a = std::min(spi[k], spj[k]) / kTile, b = std::max(spi[k], spj[k]) / kTile;
-    sp_tile[(size_t)a * nt + b] = 1;
-  }
-  h_work_beg.push_back((int)h_work.size());
-  for (int ti = 0; ti < nt; ti++)
-    for (int tj = ti; tj < nt; tj++) {
-      const int i0 = ti * kTile, j0 = tj * kTile;
-      const int gap = j0 - (i0 + kTile - 1);  // smallest j - i over the tile pair
-      GBWork wk{sysi, first + i0, first + j0, (gap < mid || sp_tile[(size_t)ti * nt + tj]) ? 1 : 0};
-      h_work.push_back(wk);
-    }
-  h_work_end.push_back((int)h_work.size());
+  h_tile_beg.push_back((int)h_tile_atoms.size());
+  for (int t = 0; t < nt; t++) h_tile_atoms.push_back(make_int2(first + t * kTile, std::min(kTile, count - t * kTile)));
   n_atoms_total = std::max(n_atoms_total, first + count);
+}
+
+// The tasks of every system.  A tile pair whose bond orders can differ from 7 (and
+// every diagonal one) is a task with codes; the others are taken two i tiles (2a,
+// 2a + 1) at a time against runs of j tiles.  A longer run shares the i tiles' sums and
+// the task's opening over more j tiles but leaves fewer tasks.  Pair pass at runs of
+// 1 / 2 / 3 / 4 (each at its best split): 54,560 tile pairs 287 / 277 / 274 / 281 us,
+// 13,640 90 / 92 / 92 / 92, 8,704 83 / 78 / 92 / 80, 3,160 30 / 32 / 38 / 46.  Heavier
+// tasks come first, so the light ones fill the end.
+void GBState::make_tasks() {
+  h_tasks.clear();
+  h_coded.clear();
+  h_slot_beg.clear();
+  h_slot_end.clear();
+  long units = 0;
+  for (size_t s = 0; s < h_sys.size(); s++) {
+    const long nt = (h_sys[s].count + kTile - 1) / kTile;
+    units += nt * (nt + 1) / 2;
+  }
+  const int run = units >= 32768 ? 3 : (units >= 8192 ? 2 : 1);
+  int slot = 0, codes = 0;
+  for (size_t s = 0; s < h_sys.size(); s++) {
+    const int nt = (h_sys[s].count + kTile - 1) / kTile, base = h_tile_beg[s], mid = h_sys[s].mid;
+    auto coded = [&](int ti, int tj) {
+      return (tj - ti) * kTile - (kTile - 1) < mid ||  // the smallest j - i over the tile pair
+             std::binary_search(h_linked[s].begin(), h_linked[s].end(), std::make_pair(ti, tj));
+    };
+    h_slot_beg.push_back(slot);
+    auto push = [&](int ti, int ni, int tj, int nj, bool with_codes) {
+      h_tasks.push_back(GBTask{(int)s, base + ti, ni, base + tj, nj, with_codes ? codes++ : -1, slot++, 0});
+    };
+    for (int a = 0; a < nt; a += 2) {
+      for (int m = 0; m < 2; m++)
+        for (int tj = a + m; a + m < nt && tj < nt; tj++)
+          if (coded(a + m, tj)) push(a + m, 1, tj, 1, true);
+      // the i tiles that take j tile tj without codes: 0 none, 1 the first, 2 the second, 3 both
+      auto takes = [&](int tj) {
+        return (tj > a && !coded(a, tj) ? 1 : 0) | (a + 1 < nt && tj > a + 1 && !coded(a + 1, tj) ? 2 : 0);
+      };
+      for (int tj = a + 1; tj < nt;) {
+        const int who = takes(tj);
+        int nj = 1;
+        while (nj < run && tj + nj < nt && takes(tj + nj) == who) nj++;
+        if (who) push(who == 2 ? a + 1 : a, who == 3 ? 2 : 1, tj, nj, false);
+        tj += nj;
+      }
+    }
+    h_slot_end.push_back(slot);
+  }
+  n_slots = slot;
+  auto weight = [](const GBTask &w) { return w.code >= 0 ? 3 : 2 * w.ni * w.nj; };
+  std::stable_sort(h_tasks.begin(), h_tasks.end(),
+                   [&](const GBTask &a, const GBTask &b) { return weight(a) > weight(b); });
+  for (size_t k = 0; k < h_tasks.size(); k++)
+    if (h_tasks[k].code >= 0) h_coded.push_back((int)k);
 }
 
 namespace {
@@ -980,8 +1194,11 @@ void GBState::upload(hipStream_t s) {
     if (it != g_split_choice.end())
       for (int k = 0; k < 3; k++) split[k] = it->second[k];
   }
-  work.upload(h_work.data(), h_work.size(), s);
+  make_tasks();
+  tasks.upload(h_tasks, s);
   sysd.upload(h_sys.data(), h_sys.size(), s);
+  tile_atoms.upload(h_tile_atoms, s);
+  tiles.resize(h_tile_atoms.size());
   if (h_band.empty()) h_band.push_back(7);
   band.upload(h_band, s);
   sp_off.upload(h_sp_off, s);
@@ -991,8 +1208,8 @@ void GBState::upload(hipStream_t s) {
   }
   sp_part.upload(h_sp_part, s);
   sp_ord.upload(h_sp_ord, s);
-  work_beg.upload(h_work_beg, s);
-  work_end.upload(h_work_end, s);
+  slot_beg.upload(h_slot_beg, s);
+  slot_end.upload(h_slot_end, s);
   std::vector<int> f, c;
   for (auto &S : h_sys) {
     f.push_back(S.first);
@@ -1006,21 +1223,58 @@ void GBState::upload(hipStream_t s) {
   born.resize(n);
   bornf.resize(n);
   eself.resize(n);
-  e_part.resize(h_work.size() * 4);
+  e_part.resize((size_t)n_slots * 4);
+  coded.upload(h_coded, s);
+  codes.resize(h_coded.size() * (kTile / kChunk) * kTile);
+  hipLaunchKernelGGL(k_gb_codes, dim3((unsigned)h_coded.size()), dim3(64), 0, s, tasks.p, coded.p, tile_atoms.p,
+                     sysd.p, band.p, sp_off.p, sp_part.p, sp_ord.p, codes.p);
+  PDGPU_HIP(hipGetLastError());
 }
 
-namespace {
-// Calls f with std::integral_constant<int, split> for a split of 1, 2 or 4.
-template <typename F>
-void by_split(int split, F &&f) {
-  if (split == 4)
-    f(std::integral_constant<int, 4>{});
-  else if (split == 2)
-    f(std::integral_constant<int, 2>{});
+// A pass's launch: every task at `split` wavefronts, or (0) at the number that fills
+// the chip: a task's chunks follow each other in one wavefront, so few tasks leave
+// SIMDs idle, while many pay for each wavefront's share of the opening.  Radii / pair
+// / chain at splits 1, 2, 4: 1,700 tasks 22 / 44 / 32, 16 / 33 / 25, 14 / 30 / 22 us; 4,000
+// tasks 39 / 88 / 59, 31 / 78 / 46, 34 / 82 / 48; 21,000 tasks 101 / 274 / 171, 113 / 302 /
+// 187, 153 / 346 / 213.
+template <int PASS>
+void GBState::launch_pass(hipStream_t s, const GBPassArgs &A, int sp) {
+  const unsigned nt = (unsigned)h_tasks.size();
+  if (sp == 0) sp = nt < 3072 ? 4 : (nt < 12288 ? 2 : 1);
+  if (sp == 4)
+    hipLaunchKernelGGL((k_gb_pass<PASS, 4>), dim3(nt), dim3(256), 0, s, A);
+  else if (sp == 2)
+    hipLaunchKernelGGL((k_gb_pass<PASS, 2>), dim3(nt), dim3(128), 0, s, A);
   else
-    f(std::integral_constant<int, 1>{});
+    hipLaunchKernelGGL((k_gb_pass<PASS, 1>), dim3(nt), dim3(64), 0, s, A);
 }
-}  // namespace
+
+GBPassArgs GBState::pass_args(const double *x, const double *y, const double *z, long long *fx, long long *fy,
+                              long long *fz) const {
+  GBPassArgs A{};
+  A.K = kp;
+  A.tasks = tasks.p;
+  A.tile_atoms = tile_atoms.p;
+  A.tiles = tiles.p;
+  A.codes = codes.p;
+  A.x = x;
+  A.y = y;
+  A.z = z;
+  A.q = q.p;
+  A.ljr = ljr.p;
+  A.lje = lje.p;
+  A.bornf = bornf.p;
+  A.gbrad = gbrad.p;
+  A.Vj = Vj.p;
+  A.born = born.p;
+  A.deda_in = deda.p;
+  A.s0 = fx;
+  A.s1 = fy;
+  A.s2 = fz;
+  A.s3 = deda.p;
+  A.e_part = e_part.p;
+  return A;
+}
 
 PlainGB GBState::plain_args() const {
   PlainGB P{};
@@ -1062,11 +1316,7 @@ void GBState::set_split(const int32_t *s3) {
 void GBState::run(hipStream_t s, const double *x, const double *y, const double *z, long long *fx, long long *fy,
                   long long *fz, double *out, int out_stride, int out_off, Engine *timer_owner, bool energy_only) {
   const int n = n_atoms_total;
-  const int nw = (int)h_work.size();
   const int nsys = (int)h_sys.size();
-  const GBK &K = kp;
-  const GBWork *W = work.p;
-  const GBSys *SY = sysd.p;
   if (plain) {
     if (energy_only || !prm.FastMode || nsys != 1)
       throw EngineError(PDGPU_ERR_ARG, "the plain GB comparator runs one system's FastMode forces");
@@ -1095,44 +1345,37 @@ void GBState::run(hipStream_t s, const double *x, const double *y, const double 
                        out_stride, out_off + 4);
     return;
   }
-  hipLaunchKernelGGL(k_zero_ll1, dim3((n + 255) / 256), dim3(256), 0, s, gpol.p, n);
+  const GBPassArgs A = pass_args(x, y, z, fx, fy, fz);
+  const int ntiles = (int)h_tile_atoms.size();
+  const dim3 tg((ntiles + 3) / 4);
+  hipLaunchKernelGGL(k_gb_tiles, tg, dim3(256), 0, s, ntiles, tile_atoms.p, x, y, z, gbrad.p, tiles.p, gpol.p);
   {
     ScopedTimerOpt t(timer_owner, "gb_radii");
-    by_split(split[0], [&](auto c) {
-      constexpr int SP = decltype(c)::value;
-      hipLaunchKernelGGL(k_gb_radii<SP>, dim3(nw), dim3(64 * SP), 0, s, K, W, SY, x, y, z, gbrad.p, Vj.p, band.p,
-                         sp_off.p, sp_part.p, sp_ord.p, gpol.p);
-    });
+    GBPassArgs R = A;
+    R.K = kr;
+    R.s0 = gpol.p;
+    launch_pass<kGbRadii>(s, R, split[0]);
   }
-  hipLaunchKernelGGL(k_gb_finalize_radii, dim3((n + 255) / 256), dim3(256), 0, s, n, Consts::halfeconv(),
-                     prm.BornRadiusOffset, (double)kp.premul, terms123.p, gpol.p, q.p, born.p, bornf.p, deda.p,
-                     eself.p);
+  hipLaunchKernelGGL(k_gb_finalize_radii, tg, dim3(256), 0, s, ntiles, tile_atoms.p, Consts::halfeconv(),
+                     prm.BornRadiusOffset, kp.premul_d, terms123.p, gpol.p, q.p, born.p, bornf.p, deda.p, eself.p,
+                     tiles.p);
   {
     ScopedTimerOpt t(timer_owner, "gb_pair");
-    by_split(split[1], [&](auto c) {
-      constexpr int SP = decltype(c)::value;
-      if (energy_only) {
-        hipLaunchKernelGGL((k_gb_pair<kGbEnergy, SP>), dim3(nw), dim3(64 * SP), 0, s, K, W, SY, x, y, z, q.p, ljr.p,
-                           lje.p, bornf.p, band.p, sp_off.p, sp_part.p, sp_ord.p, fx, fy, fz, deda.p, e_part.p);
-      } else if (prm.FastMode) {
-        hipLaunchKernelGGL((k_gb_pair<kGbFast, SP>), dim3(nw), dim3(64 * SP), 0, s, K, W, SY, x, y, z, q.p, ljr.p,
-                           lje.p, bornf.p, band.p, sp_off.p, sp_part.p, sp_ord.p, fx, fy, fz, deda.p, e_part.p);
-      } else {
-        hipLaunchKernelGGL((k_gb_pair<kGbBorn, SP>), dim3(nw), dim3(64 * SP), 0, s, K, W, SY, x, y, z, q.p, ljr.p,
-                           lje.p, bornf.p, band.p, sp_off.p, sp_part.p, sp_ord.p, fx, fy, fz, deda.p, e_part.p);
-      }
-    });
+    if (energy_only)
+      launch_pass<kGbEnergy>(s, A, split[1]);
+    else if (prm.FastMode)
+      launch_pass<kGbFast>(s, A, split[1]);
+    else
+      launch_pass<kGbBorn>(s, A, split[1]);
   }
   if (!energy_only) {
     ScopedTimerOpt t(timer_owner, "gb_chain");
-    by_split(split[2], [&](auto c) {
-      constexpr int SP = decltype(c)::value;
-      hipLaunchKernelGGL(k_gb_chain<SP>, dim3(nw), dim3(64 * SP), 0, s, K, W, SY, x, y, z, gbrad.p, Vj.p, born.p, deda.p,
-                         band.p, sp_off.p, sp_part.p, sp_ord.p, fx, fy, fz);
-    });
+    GBPassArgs C = A;
+    C.K = kr;
+    launch_pass<kGbChain>(s, C, split[2]);
   }
   PDGPU_HIP(hipGetLastError());
-  hipLaunchKernelGGL(k_gb_sums, dim3(nsys, 2), dim3(256), 0, s, e_part.p, work_beg.p, work_end.p, eself.p,
+  hipLaunchKernelGGL(k_gb_sums, dim3(nsys, 2), dim3(256), 0, s, e_part.p, slot_beg.p, slot_end.p, eself.p,
                      sys_first.p, sys_count.p, out, out_stride, out_off);
 }
 
@@ -1142,37 +1385,28 @@ void GBState::run(hipStream_t s, const double *x, const double *y, const double 
 void GBState::autotune(hipStream_t s, const double *x, const double *y, const double *z, long long *fx,
                        long long *fy, long long *fz, double *out, int out_stride, int out_off, double *us) {
   constexpr int kTuneLaunches = 5;
-  const int nw = (int)h_work.size();
   run(s, x, y, z, fx, fy, fz, out, out_stride, out_off, nullptr, false);
   hipEvent_t a, b;
   PDGPU_HIP(hipEventCreate(&a));
   PDGPU_HIP(hipEventCreate(&b));
-  const GBK &K = kp;
-  const GBWork *W = work.p;
-  const GBSys *SY = sysd.p;
+  const GBPassArgs A = pass_args(x, y, z, fx, fy, fz);
+  GBPassArgs R = A, Q = A;
+  R.K = Q.K = kr;
+  R.s0 = gpol.p;
   for (int k = 0; k < 3; k++) {
     double best = 1e300;
     int best_split = 1;
     for (int m = 0; m < 3; m++) {
       const int sp = 1 << m;
       auto launch = [&]() {
-        by_split(sp, [&](auto c) {
-          constexpr int SP = decltype(c)::value;
-          if (k == 0)
-            hipLaunchKernelGGL(k_gb_radii<SP>, dim3(nw), dim3(64 * SP), 0, s, K, W, SY, x, y, z, gbrad.p, Vj.p,
-                               band.p, sp_off.p, sp_part.p, sp_ord.p, gpol.p);
-          else if (k == 1 && prm.FastMode)
-            hipLaunchKernelGGL((k_gb_pair<kGbFast, SP>), dim3(nw), dim3(64 * SP), 0, s, K, W, SY, x, y, z, q.p,
-                               ljr.p, lje.p, bornf.p, band.p, sp_off.p, sp_part.p, sp_ord.p, fx, fy, fz, deda.p,
-                               e_part.p);
-          else if (k == 1)
-            hipLaunchKernelGGL((k_gb_pair<kGbBorn, SP>), dim3(nw), dim3(64 * SP), 0, s, K, W, SY, x, y, z, q.p,
-                               ljr.p, lje.p, bornf.p, band.p, sp_off.p, sp_part.p, sp_ord.p, fx, fy, fz, deda.p,
-                               e_part.p);
-          else
-            hipLaunchKernelGGL(k_gb_chain<SP>, dim3(nw), dim3(64 * SP), 0, s, K, W, SY, x, y, z, gbrad.p, Vj.p,
-                               born.p, deda.p, band.p, sp_off.p, sp_part.p, sp_ord.p, fx, fy, fz);
-        });
+        if (k == 0)
+          launch_pass<kGbRadii>(s, R, sp);
+        else if (k == 1 && prm.FastMode)
+          launch_pass<kGbFast>(s, A, sp);
+        else if (k == 1)
+          launch_pass<kGbBorn>(s, A, sp);
+        else
+          launch_pass<kGbChain>(s, Q, sp);
       };
       launch();  // warm
       PDGPU_HIP(hipEventRecord(a, s));

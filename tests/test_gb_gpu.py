@@ -209,6 +209,37 @@ def test_gb_split_variants_and_autotuner():
     assert set(bc.tolist()) <= {1, 2, 4}
 
 
+@pytest.mark.parametrize("n_atoms", [63, 64, 65, 128, 129, 257, 640])
+@pytest.mark.parametrize("kw", [ALL_PAIRS, SWITCHED], ids=["all", "switch"])
+def test_gb_tile_edges_and_far_tiles(n_atoms, kw):
+    """Systems cut at the edges of the 64-atom tiles, stretched so that distant tile
+    pairs take the far loops (one i tile and two, and the single tile of an odd count),
+    against the oracle at the bars above; every split gives the same bits."""
+    s = S.peptide_chain(44, seed=31, phi_mu=-120.0, psi_mu=130.0)
+    # the first n_atoms atoms, with the covalent partners among them
+    def cut(off, idx, *more):
+        keep = [k for i in range(n_atoms) for k in range(s.cov[off][i], s.cov[off][i + 1]) if s.cov[idx][k] < n_atoms]
+        cnt = [sum(s.cov[idx][k] < n_atoms for k in range(s.cov[off][i], s.cov[off][i + 1])) for i in range(n_atoms)]
+        return {off: np.concatenate([[0], np.cumsum(cnt)]).astype(np.int32), idx: s.cov[idx][keep],
+                **{m: s.cov[m][keep] for m in more}}
+    assert s.n >= 640
+    s.cov = {**cut("off12", "idx12", "d12"), **cut("off13", "idx13", "d13"), **cut("off14", "idx14")}
+    for f in ("pos", "radius", "epsilon", "charge", "mass", "gbrad", "resid"):
+        setattr(s, f, getattr(s, f)[:n_atoms].copy())
+    s.mol_last = np.array([n_atoms - 1], dtype=np.int32)
+    print(f"case tile edges n={n_atoms} cutoff {kw['Cutoff']}", flush=True)
+    born_ref, f_ref, e_ref = oracle_gb(s, kw)
+    e, f, en = gpu_gb(s, kw)
+    assert np.abs(e.born_radii() - born_ref).max() <= 1e-6 * np.abs(born_ref).max()
+    assert rel_rms(f, f_ref) <= 1e-5
+    scale = coulomb_abs_sum(s, kw)
+    for k in ("epot", "epot_pol", "epot_vdw", "epot_elec"):
+        assert abs(en[k] - e_ref[k]) <= 1e-5 * abs(e_ref[k]) + 1e-6 * scale, k
+    for sp in ((1, 1, 1), (2, 2, 2), (4, 4, 4)):
+        e.set_gb_split(sp)
+        assert np.array_equal(e.compute(G.PDGPU_GB)[0], f), sp
+
+
 @pytest.mark.parametrize("kw", [ALL_PAIRS, SWITCHED], ids=["all", "switch"])
 def test_gb_plain_comparator_matches_oracle(kw):
     """The plain FP64 comparator (one thread per atom, FP64 sums) against the
