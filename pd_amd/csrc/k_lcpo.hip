@@ -10,8 +10,8 @@
 //                 overlap partners (d < R_i + R_j, hydrogens excluded) in
 //                 ascending index order, at most 80 (Nlistmax, lcpo.h:24) --
 //                 the order and truncation PD's fill loop produces
-//                 (lcpo.cpp:713-767); then, one lane per partner, the overlap
-//                 A_ij = 2 pi R_i (R_i - d/2 - (R_i^2 - R_j^2) / 2d);
+//                 (lcpo.cpp:713-767); for the energy path also, one lane per
+//                 partner, the overlap A_ij = 2 pi R_i (R_i - d/2 - (R_i^2 - R_j^2) / 2d);
 //   k_lcpo_sasa   one wavefront per atom: SASA_i and the derivative that PD
 //                 collects on atom i (its own self terms plus the derivatives
 //                 of its neighbours' SASA with respect to x_i), clamped to zero
@@ -50,8 +50,11 @@ __device__ __forceinline__ bool lcpo_full(const int *step_ptr, int step_host, in
 // their used atoms) against R_i + max R; then, tile by tile in ascending order,
 // each near tile's 64 atoms one per lane, and a ballot places the partners in
 // index order, so each list comes out ascending and the first kLcpoMax are
-// kept, as PD's fill loop does.  The overlaps follow, one lane per partner.
+// kept, as PD's fill loop does.  A list that is cut at kLcpoMax, or has a partner at
+// exactly R_i + R_j (no partner, but still inside the test of PD's inner loop), is
+// flagged (kListCut) for k_lcpo_sasa.  EONLY: the overlaps follow, one lane per partner.
 constexpr int kListWaves = 4;
+constexpr int kListCut = 0x100;  // in nl_cnt, above the count
 // workgroups of k_lcpo_lists at most (each wave walks atoms wave, + 4 * grid, ...):
 // the launch returns at once on the steps that re-apply the stored forces, and
 // the cost of that empty launch grows with its workgroup count (16 us for the
@@ -83,9 +86,10 @@ __global__ __launch_bounds__(64 * kListWaves) void k_lcpo_lists(
     const double reach = (ri + max_R) * (1.0 + 1e-12);
     const unsigned long long below = (1ull << lane) - 1ull;
     int *my = s_list[wave];
-    int cnt = 0;
+    int cnt = 0, cut = 0;
     const int tfirst = first / 64, tlast = (end - 1) / 64;
-    for (int t0 = tfirst; t0 <= tlast && cnt < kLcpoMax; t0 += 64) {
+    // one past the last partner that is kept, to know whether any is dropped
+    for (int t0 = tfirst; t0 <= tlast && cnt <= kLcpoMax; t0 += 64) {
       bool near = false;
       const int t = t0 + lane;
       if (t <= tlast) {
@@ -96,11 +100,11 @@ __global__ __launch_bounds__(64 * kListWaves) void k_lcpo_lists(
         near = gx * gx + gy * gy + gz * gz <= reach * reach;
       }
       unsigned long long nb = __ballot(near);
-      while (nb != 0ull && cnt < kLcpoMax) {
+      while (nb != 0ull && cnt <= kLcpoMax) {
         const int tt = t0 + __ffsll((long long)nb) - 1;
         nb &= nb - 1ull;
         const int j = tt * 64 + lane;
-        bool ok = false;
+        bool ok = false, edge = false;
         if (j >= first && j < end && j != i) {
           const double4 pj = pr[j];
           if (pj.w > 0.0) {
@@ -108,8 +112,10 @@ __global__ __launch_bounds__(64 * kListWaves) void k_lcpo_lists(
             const double d2 = g * g + h * h + k * k;
             const double rj = pj.w;
             ok = EONLY ? sqrt(d2) < (ri + rj) : d2 < (ri + rj) * (ri + rj);
+            edge = !EONLY && d2 == (ri + rj) * (ri + rj);
           }
         }
+        if (__ballot(edge) != 0ull) cut = kListCut;
         const unsigned long long b = __ballot(ok);
         const int pos = cnt + __popcll(b & below);
         if (ok && pos < kLcpoMax) {
@@ -119,8 +125,10 @@ __global__ __launch_bounds__(64 * kListWaves) void k_lcpo_lists(
         cnt += __popcll(b);
       }
     }
+    if (cnt > kLcpoMax) cut = kListCut;
     cnt = min(cnt, kLcpoMax);
-    if (lane == 0) nl_cnt[i] = cnt;
+    if (lane == 0) nl_cnt[i] = EONLY ? cnt : cnt | cut;
+    if (!EONLY) continue;
     // the list is read back by other lanes of the same wave
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
@@ -134,15 +142,9 @@ __global__ __launch_bounds__(64 * kListWaves) void k_lcpo_lists(
       const double d2 = g * g + h * h + k * k;
       const double rj = pj.w;
       const double d = sqrt(d2);
-      double sij;
-      if (EONLY) {  // sphereSurfaceOverlap (maths.cpp:120-123), negative overlaps set to 0
-        sij = TwoPI * ri * (ri - d / 2.0 - (ri * ri - rj * rj) / (2.0 * d));
-        if (sij < 0) sij = 0;
-      } else {
-        const double inv = 1 / d;
-        const double tt = 0.5 * (ri * ri - rj * rj) * inv;
-        sij = TwoPI * ri * (ri - d * 0.5 - tt);
-      }
+      // sphereSurfaceOverlap (maths.cpp:120-123), negative overlaps set to 0
+      double sij = TwoPI * ri * (ri - d / 2.0 - (ri * ri - rj * rj) / (2.0 * d));
+      if (sij < 0) sij = 0;
       nl_s[(size_t)i * kLcpoMax + c] = sij;
     }
     // the next atom's list overwrites this one after every lane has read it
@@ -188,17 +190,114 @@ __global__ void k_lcpo_pack(int n, const double *__restrict__ x, const double *_
 // the neighbours k of j are rearranged as one flat sum over the (j, k) pairs:
 // every k-term enters the derivative linearly, with weights that depend on j
 // alone (P3_j sigma_j, P4_j sigma_j, the overlap s_ji, the pair derivative of
-// s_ji), so the lanes take (j, k) pairs in turn after a first pass over j has
-// put those weights in LDS; the sums are reduced over the wave in a fixed
-// order.  EONLY: calcLCPOSasaEnergies (lcpo.cpp:522-556), the SASA alone, with
-// k excluded when (R_i + R_k) < d_ik.
-constexpr int kLcpoDepth = 4;  // (j, k) tasks per lane in flight in k_lcpo_sasa
-// waves of k_lcpo_sasa (each walks atoms blockIdx.x, + gridDim.x, ...): on the
-// 256-chain batch (285,363 atoms) 4096 / 8192 / 16384 / 65536 / one wave per atom
-// gave 197.6k / 199.7k / 202.9k / 204.6k / 199.6k aggregate steps/s
+// s_ji).
+//
+// The k that count are neighbours of j that overlap i: when the lists of i and of its
+// neighbours are whole (kListCut unset), that is every pair (j, k) of i's own list
+// with d_jk < R_j + R_k.  So the wavefront puts its list's atoms and weights in LDS once
+// and computes the pairs from there: lane (k mod 16, j mod 4) holds up to three k and
+// walks the j, recomputing the overlap s_jk (one reciprocal square root) instead of
+// fetching it; sums over j alone (the k's share of the derivative) and over k alone
+// (SASA_i's own terms) stay in registers.  It is bound by FP64 issue (38 instructions a
+// pair; four wavefronts a SIMD, 128 registers).  Gathering each j's list and overlaps
+// from memory instead waited on loads most of its time: average over the steps of a run
+// (a full update every fifth) on 256 chains 241 -> 116 us, 64 replicas 69 -> 39; a full
+// update of a 300-residue chain 46 -> 24, of a 20-residue chain 26 -> 12.
+//
+// EONLY (calcLCPOSasaEnergies, lcpo.cpp:522-556: the SASA alone, with k excluded
+// when (R_i + R_k) < d_ik) and atoms with a cut list take the pairs from the
+// neighbours' lists: lanes take (j, k) pairs in turn after a first pass over j has put
+// the weights in LDS.  All sums are reduced over the wave in a fixed order.
+constexpr int kLcpoDepth = 4;  // (j, k) tasks per lane in flight when gathering
+// waves of k_lcpo_sasa (each walks atoms blockIdx.x, + gridDim.x, ...)
 constexpr int kLcpoGrid = 65536;
+
+// 1 / sqrt(x) in FP64: the hardware's estimate y (relative error 2^-24) with one step of
+// third order, y (1 + e/2 + 3 e^2/8) with e = 1 - x y^2 (what is left: e^3, below 2^-70)
+__device__ __forceinline__ double rsqrt_fp64(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  const double e = fma(-x * y, y, 1.0);
+  return fma(y, e * fma(0.375, e, 0.5), y);
+}
+
+// A neighbour of i in LDS, as seven 16-byte arrays (consecutive j: no bank conflicts)
+struct LcpoLds {
+  double2 xy[kLcpoMax], zr[kLcpoMax];      // position, R
+  double2 w34[kLcpoMax], sw[kLcpoMax];     // P3 sigma, P4 sigma | s_ij, P4 sigma s_ji
+  double2 dxy[kLcpoMax], dza[kLcpoMax];    // d s_ji / d x_i (its j part): x, y | z, x of the i part
+  double2 ayz[kLcpoMax];                   // the i part (d s_ij / d x_i): y, z
+};
+
+// The pairs (j, k) of the list with k = 16 m + (lane & 15), m0 <= m < m0 + MB.
+template <int MB>
+__device__ __forceinline__ void lcpo_pairs(const LcpoLds &L, int n, int m0, int lane, double der[3], double a4[3],
+                                           double &Si3, double &Si4) {
+  const double PI = Consts::PI;
+  double xk[MB], yk[MB], zk[MB], rk[MB], hk[MB];
+  double c3[MB], ca[MB], cb[MB], vx[MB], vy[MB], vz[MB];
+  int kk[MB];
+#pragma unroll
+  for (int m = 0; m < MB; m++) {
+    const int k = 16 * (m0 + m) + (lane & 15);
+    kk[m] = min(k, n - 1);
+    const double2 a = L.xy[kk[m]], b = L.zr[kk[m]];
+    xk[m] = k < n ? a.x : 1e30;  // a pad overlaps nothing
+    yk[m] = a.y;
+    zk[m] = b.x;
+    rk[m] = b.y;
+    hk[m] = 0.5 * b.y * b.y;
+    c3[m] = ca[m] = cb[m] = vx[m] = vy[m] = vz[m] = 0.0;
+  }
+  for (int j0 = 0; j0 < n; j0 += 4) {
+    const int j = min(j0 + (lane >> 4), n - 1);
+    const double2 a = L.xy[j], b = L.zr[j], w = L.w34[j], s2 = L.sw[j], d01 = L.dxy[j], d2a = L.dza[j], a12 = L.ayz[j];
+    const double xj = j0 + (lane >> 4) < n ? a.x : -1e30;
+    const double rj = b.y, hj = 0.5 * rj * rj, cj = 2.0 * PI * rj;
+    double T = 0.0;
+#pragma unroll
+    for (int m = 0; m < MB; m++) {
+      double d2, lim;
+      {
+#pragma clang fp contract(off)
+        const double g = xj - xk[m], h = a.y - yk[m], q = b.x - zk[m];
+        d2 = g * g + h * h + q * q;  // the list's test, bit for bit
+        lim = (rj + rk[m]) * (rj + rk[m]);
+      }
+      const bool on = d2 < lim && kk[m] != j;
+      const double inv = rsqrt_fp64(d2);
+      const double d = d2 * inv;
+      const double s0 = cj * fma(-(hj - hk[m]), inv, fma(-0.5, d, rj));
+      const double s = on ? s0 : 0.0, o = on ? 1.0 : 0.0;
+      T += s;
+      c3[m] = fma(o, w.x, c3[m]);
+      ca[m] = fma(o, s2.y, ca[m]);
+      cb[m] = fma(w.y, s, cb[m]);
+      const double ow = o * w.y;
+      vx[m] = fma(ow, d01.x, vx[m]);
+      vy[m] = fma(ow, d01.y, vy[m]);
+      vz[m] = fma(ow, d2a.x, vz[m]);
+    }
+    Si3 += T;
+    Si4 = fma(s2.x, T, Si4);
+    a4[0] = fma(T, d2a.y, a4[0]);
+    a4[1] = fma(T, a12.x, a4[1]);
+    a4[2] = fma(T, a12.y, a4[2]);
+  }
+#pragma unroll
+  for (int m = 0; m < MB; m++) {
+    const int k = kk[m];
+    if (16 * (m0 + m) + (lane & 15) >= n) continue;
+    // s_ik, its derivatives with respect to x_i (i part, k part)
+    const double s = L.sw[k].x, p1 = c3[m] + ca[m], p2 = c3[m] + cb[m];
+    const double2 d01 = L.dxy[k], d2a = L.dza[k], a12 = L.ayz[k];
+    der[0] += fma(p1, d2a.y, fma(p2, d01.x, s * vx[m]));
+    der[1] += fma(p1, a12.x, fma(p2, d01.y, s * vy[m]));
+    der[2] += fma(p1, a12.y, fma(p2, d2a.x, s * vz[m]));
+  }
+}
+
 template <bool EONLY>
-__global__ __launch_bounds__(64) void k_lcpo_sasa(int n, const double4 *__restrict__ pr, const int8_t *__restrict__ use,
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_lcpo_sasa(int n, const double4 *__restrict__ pr, const int8_t *__restrict__ use,
                                                   const double4 *__restrict__ P,
                                                   const double *__restrict__ sig, const int *__restrict__ step_ptr,
                                                   int step_host, int update, const int *__restrict__ nl_cnt,
@@ -206,8 +305,17 @@ __global__ __launch_bounds__(64) void k_lcpo_sasa(int n, const double4 *__restri
                                                   double *__restrict__ sasa, double *__restrict__ dvx,
                                                   double *__restrict__ dvy, double *__restrict__ dvz) {
 #pragma clang fp contract(off)
-  __shared__ int jidx[kLcpoMax], joff[kLcpoMax + 1];
-  __shared__ double jw[kLcpoMax][10];  // s_ji, P3 sigma, P4 sigma, Si2_t, d2(3), a2t(3)
+  // gathering: jw holds s_ji, P3 sigma, P4 sigma, Si2_t, d2(3), a2t(3) of each j
+  __shared__ __align__(16) union {
+    LcpoLds list;
+    struct {
+      int jidx[kLcpoMax], joff[kLcpoMax + 1];
+      double jw[kLcpoMax][10];
+    } g;
+  } sh;
+  auto &jidx = sh.g.jidx;
+  auto &joff = sh.g.joff;
+  auto &jw = sh.g.jw;
   const int lane = threadIdx.x;
   if (!lcpo_full(step_ptr, step_host, update)) return;  // uniform: the step is the same for all
   // at most kLcpoGrid waves walk the atoms; on the steps that re-apply stored
@@ -225,17 +333,29 @@ __global__ __launch_bounds__(64) void k_lcpo_sasa(int n, const double4 *__restri
   const double4 pi4 = pr[i];
   const double pix = pi4.x, piy = pi4.y, piz = pi4.z;
   const double ri = pi4.w;
-  const int ni = nl_cnt[i];
-  // pass over j: per-j weights and the k counts
+  const int ni = nl_cnt[i] & (kListCut - 1);
   double der[3] = {0, 0, 0}, a2[3] = {0, 0, 0}, a4[3] = {0, 0, 0};
   double Si2 = 0, Si3 = 0, Si4 = 0;
+  // whole lists (uniform over the wave)?
+  bool gather = EONLY;
+  if (!EONLY) {
+    int cut = nl_cnt[i] & kListCut;
+    for (int jn = lane; jn < ni; jn += 64) cut |= nl_cnt[nl_idx[(size_t)i * kLcpoMax + jn]] & kListCut;
+    gather = __ballot(cut != 0) != 0ull;
+  }
+  // pass over j: per-j weights, and the k counts when gathering
   for (int jn = lane; jn < ni; jn += 64) {
     const int ja = nl_idx[(size_t)i * kLcpoMax + jn];
-    const double Si2_t = nl_s[(size_t)i * kLcpoMax + jn];
-    jidx[jn] = ja;
-    joff[jn + 1] = nl_cnt[ja];
-    jw[jn][3] = Si2_t;
-    Si2 += Si2_t;
+    double Si2_t = 0.0;
+    if (EONLY) {
+      Si2_t = nl_s[(size_t)i * kLcpoMax + jn];
+      Si2 += Si2_t;
+      jw[jn][3] = Si2_t;
+    }
+    if (gather) {
+      jidx[jn] = ja;
+      joff[jn + 1] = nl_cnt[ja] & (kListCut - 1);
+    }
     if (!EONLY) {
       const double4 pj4 = pr[ja];
       const double pjx = pj4.x, pjy = pj4.y, pjz = pj4.z;
@@ -244,25 +364,53 @@ __global__ __launch_bounds__(64) void k_lcpo_sasa(int n, const double4 *__restri
       const double rj = pj4.w;
       const double inv = 1 / dij;
       double t = 0.5 * (ri * ri - rj * rj) * inv;
+      Si2_t = TwoPI * ri * (ri - dij * 0.5 - t);
+      Si2 += Si2_t;
       const double sji = TwoPI * rj * (rj - dij * 0.5 + t);
       t *= 2.0 * inv;
       const double ddd[3] = {-(pix - pjx) / dij, -(piy - pjy) / dij, -(piz - pjz) / dij};
       const double dAj = PI * rj * (-t - 1), dAi = PI * ri * (t - 1);
       const double4 Pj = P[ja];
       const double sj = sig[ja];
-      jw[jn][0] = sji;
-      jw[jn][1] = Pj.z * sj;
-      jw[jn][2] = Pj.w * sj;
+      double d2[3], a2t[3];
       for (int c = 0; c < 3; c++) {
-        const double d2c = dAj * ddd[c];
-        jw[jn][4 + c] = d2c;
-        jw[jn][7 + c] = dAi * ddd[c];
-        der[c] += d2c * (Pj.y * sj);  // the P2 term of SASA_j
-        a2[c] += dAi * ddd[c];
+        d2[c] = dAj * ddd[c];
+        a2t[c] = dAi * ddd[c];
+        der[c] += d2[c] * (Pj.y * sj);  // the P2 term of SASA_j
+        a2[c] += a2t[c];
+      }
+      if (gather) {
+        jw[jn][0] = sji;
+        jw[jn][1] = Pj.z * sj;
+        jw[jn][2] = Pj.w * sj;
+        jw[jn][3] = Si2_t;
+        for (int c = 0; c < 3; c++) {
+          jw[jn][4 + c] = d2[c];
+          jw[jn][7 + c] = a2t[c];
+        }
+      } else {
+        sh.list.xy[jn] = make_double2(pjx, pjy);
+        sh.list.zr[jn] = make_double2(pjz, rj);
+        sh.list.w34[jn] = make_double2(Pj.z * sj, Pj.w * sj);
+        sh.list.sw[jn] = make_double2(Si2_t, Pj.w * sj * sji);
+        sh.list.dxy[jn] = make_double2(d2[0], d2[1]);
+        sh.list.dza[jn] = make_double2(d2[2], a2t[0]);
+        sh.list.ayz[jn] = make_double2(a2t[1], a2t[2]);
       }
     }
   }
   __syncthreads();
+  if (!gather) {
+    for (int m0 = 0; 16 * m0 < ni; m0 += 3) {
+      const int left = (ni + 15) / 16 - m0;
+      if (left >= 3)
+        lcpo_pairs<3>(sh.list, ni, m0, lane, der, a4, Si3, Si4);
+      else if (left == 2)
+        lcpo_pairs<2>(sh.list, ni, m0, lane, der, a4, Si3, Si4);
+      else
+        lcpo_pairs<1>(sh.list, ni, m0, lane, der, a4, Si3, Si4);
+    }
+  } else {
   if (lane == 0) {  // exclusive prefix of the k counts, in j order
     joff[0] = 0;
     for (int jn = 0; jn < ni; jn++) joff[jn + 1] += joff[jn];
@@ -287,7 +435,7 @@ __global__ __launch_bounds__(64) void k_lcpo_sasa(int n, const double4 *__restri
         const int kn = t - joff[jn];
         jnv[u] = jn;
         kav[u] = nl_idx[(size_t)ja * kLcpoMax + kn];
-        sjkv[u] = nl_s[(size_t)ja * kLcpoMax + kn];
+        if (EONLY) sjkv[u] = nl_s[(size_t)ja * kLcpoMax + kn];
       }
     }
     double4 pkv[kLcpoDepth];
@@ -303,7 +451,13 @@ __global__ __launch_bounds__(64) void k_lcpo_sasa(int n, const double4 *__restri
     const double rk = pk4.w;
     const double hx = pkx - pix, hy = pky - piy, hz = pkz - piz;
     double dik = hx * hx + hy * hy + hz * hz;
-    const double sjk = sjkv[u];
+    double sjk = sjkv[u];
+    if (!EONLY) {  // the overlap of j with k, as the neighbour's list would hold it
+      const double4 pj4 = pr[jidx[jn_u]];
+      const double gx = pj4.x - pkx, gy = pj4.y - pky, gz = pj4.z - pkz;
+      const double d = sqrt(gx * gx + gy * gy + gz * gz);
+      sjk = TwoPI * pj4.w * (pj4.w - d * 0.5 - 0.5 * (pj4.w * pj4.w - rk * rk) * (1 / d));
+    }
     if (EONLY) {
       if ((ri + rk) < sqrt(dik)) continue;
     } else {
@@ -327,20 +481,16 @@ __global__ __launch_bounds__(64) void k_lcpo_sasa(int n, const double4 *__restri
     }
     }
   }
-  Si2 = wave_sum(Si2);
-  Si3 = wave_sum(Si3);
-  Si4 = wave_sum(Si4);
-  if (!EONLY)
-    for (int c = 0; c < 3; c++) {
-      der[c] = wave_sum(der[c]);
-      a2[c] = wave_sum(a2[c]);
-      a4[c] = wave_sum(a4[c]);
-    }
-  if (lane != 0) continue;
+  }
+  // SASA and derivative are linear in the sums: combined per lane, then added over the wave
   const double4 Pi = P[i];
   const double Si = FourPI * ri * ri;
-  double SAi = Pi.x * Si + Pi.y * Si2 + Pi.z * Si3 + Pi.w * Si4;
-  for (int c = 0; c < 3; c++) der[c] += a2[c] * (Pi.y * sig[i]) + a4[c] * (Pi.w * sig[i]);
+  double SAi = Pi.x * Si + wave_sum(Pi.y * Si2 + Pi.z * Si3 + Pi.w * Si4);
+  if (!EONLY) {
+    const double k2 = Pi.y * sig[i], k4 = Pi.w * sig[i];
+    for (int c = 0; c < 3; c++) der[c] = wave_sum(der[c] + a2[c] * k2 + a4[c] * k4);
+  }
+  if (lane != 0) continue;
   if (SAi < 0) {  // LCPO can go negative for buried atoms (lcpo.cpp:940-944)
     SAi = 0;
     der[0] = der[1] = der[2] = 0.0;
@@ -364,9 +514,11 @@ __global__ void k_lcpo_apply(int n, double to_kcal, const double *__restrict__ s
   eatom[i] = sasa[i] * sig[i] * to_kcal;
   const double gx = dvx[i], gy = dvy[i], gz = dvz[i];
   if (gx != 0.0 || gy != 0.0 || gz != 0.0) {
-    fix_add(&fx[i], fix_from_double(gx * to_kcal));
-    fix_add(&fy[i], fix_from_double(gy * to_kcal));
-    fix_add(&fz[i], fix_from_double(gz * to_kcal));
+    // to the nearest unit (fix_from_double rounds down): surface forces are small
+    const double half = 0.5 / kFixScale;
+    fix_add(&fx[i], fix_from_double(fma(gx, to_kcal, half)));
+    fix_add(&fy[i], fix_from_double(fma(gy, to_kcal, half)));
+    fix_add(&fz[i], fix_from_double(fma(gz, to_kcal, half)));
   }
 }
 

@@ -112,3 +112,38 @@ def test_lcpo_batch_equals_single_systems():
         assert np.array_equal(fb[k], f), k
         assert eb[k]["epot_surf"] == pytest.approx(en["epot_surf"], rel=1e-12)
         assert eb[k]["epot"] == pytest.approx(en["epot"], rel=1e-12)
+
+
+@pytest.mark.parametrize("n", [2, 3, 16, 17, 18, 33, 34, 49, 50, 65, 66, 81, 82, 90])
+def test_lcpo_list_lengths(n):
+    """Balls of n mutually overlapping atoms: lists of n - 1 partners around the
+    16-partner blocks of the pair loop and the 80-partner limit (82 atoms: the first cut
+    list).  SASA: sums of up to 80^2 FP64 terms of at most 1e4 A^2, so 1e-8 A^2 absolute."""
+    rng = np.random.default_rng(n)
+    pos = rng.normal(size=(n, 3))
+    pos *= (1.9 * rng.random(n) ** (1 / 3) / np.linalg.norm(pos, axis=1))[:, None]
+    use = np.ones(n, np.int8)
+    rad = rng.choice([1.6, 1.65, 1.7, 1.9], n)
+    P = np.array(list(S.LCPO_TYPES.values()))[rng.integers(0, len(S.LCPO_TYPES), n), 1:]
+    print(f"case list length {n - 1}", flush=True)
+    f_ref, sasa_ref, e_ref = _oracle(pos, use, rad, P)
+    e = _bare_engine(pos)
+    e.setup_lcpo(G.LCPOParams(GlobalASP=ASP, UpdateSasa=5), rad, P, use)
+    f, en = e.compute(G.PDGPU_SASA)
+    np.testing.assert_allclose(e.sasa(), sasa_ref, rtol=1e-12, atol=1e-8)
+    assert rel_rms(f, f_ref) <= 1e-8 or np.abs(f_ref).max() == 0.0 == np.abs(f).max()
+
+
+def test_lcpo_touching_atoms():
+    """Atoms at exactly R_i + R_j are no partners, yet PD's inner loop (which leaves out
+    (R_i + R_k)^2 < d^2 alone) counts them as common neighbours of the atom between."""
+    pos = np.array([[0.0, 0, 0], [3.0, 0, 0], [6.0, 0, 0], [3.0, 2.0, 0]])
+    rad, use = np.full(4, 1.6), np.ones(4, np.int8)  # R = 3 exactly
+    P = np.tile([0.7, -0.2, -1e-3, 2e-4], (4, 1))
+    assert (rad + 1.4 == 3.0).all()
+    f_ref, sasa_ref, _ = _oracle(pos, use, rad, P)
+    e = _bare_engine(pos)
+    e.setup_lcpo(G.LCPOParams(GlobalASP=ASP, UpdateSasa=5), rad, P, use)
+    f, _ = e.compute(G.PDGPU_SASA)
+    np.testing.assert_allclose(e.sasa(), sasa_ref, rtol=1e-12, atol=1e-12)
+    assert rel_rms(f, f_ref) <= 1e-8
