@@ -89,30 +89,6 @@ void upload_sparse(Engine &E) {
   E.sp_ord.upload(ord, E.stream);
 }
 
-void read_aos(const double *src, size_t stride, int n, std::vector<double> &a, std::vector<double> &b,
-              std::vector<double> &c) {
-  a.resize(n);
-  b.resize(n);
-  c.resize(n);
-  for (int i = 0; i < n; i++) {
-    const double *p = reinterpret_cast<const double *>(reinterpret_cast<const char *>(src) + (size_t)i * stride);
-    a[i] = p[0];
-    b[i] = p[1];
-    c[i] = p[2];
-  }
-}
-
-void write_aos(double *dst, size_t stride, int n, const std::vector<double> &a, const std::vector<double> &b,
-               const std::vector<double> &c) {
-  for (int i = 0; i < n; i++) {
-    double *p = reinterpret_cast<double *>(reinterpret_cast<char *>(dst) + (size_t)i * stride);
-    p[0] = a[i];
-    p[1] = b[i];
-    p[2] = c[i];
-  }
-}
-
-
 }  // namespace
 }  // namespace pdgpu
 
@@ -355,18 +331,17 @@ int pdgpu_set_bonded(pdgpu_engine *h, int32_t nb, const int32_t *bi, const int32
 int pdgpu_set_positions(pdgpu_engine *h, const double *xyz, size_t stride_bytes) {
   return pdgpu::guarded(h, [&](Engine &E) {
     E.require(xyz && stride_bytes >= 3 * sizeof(double), "bad position array");
-    std::vector<double> a, b, c;
-    pdgpu::read_aos(xyz, stride_bytes, E.n, a, b, c);
-    E.x.upload(a, E.stream);
-    E.y.upload(b, E.stream);
-    E.z.upload(c, E.stream);
+    E.x.resize(E.n);
+    E.y.resize(E.n);
+    E.z.resize(E.n);
+    pdgpu::xyz_to_device(E.stage, E.stream, xyz, stride_bytes, E.n, E.x.p, E.y.p, E.z.p);
     if (E.vx.n < (size_t)E.n) {
       std::vector<double> zero(E.n, 0.0);
       E.vx.upload(zero, E.stream);
       E.vy.upload(zero, E.stream);
       E.vz.upload(zero, E.stream);
+      E.sync();
     }
-    E.sync();
     E.have_positions = true;
   });
 }
@@ -374,36 +349,24 @@ int pdgpu_set_positions(pdgpu_engine *h, const double *xyz, size_t stride_bytes)
 int pdgpu_get_positions(pdgpu_engine *h, double *xyz, size_t stride_bytes) {
   return pdgpu::guarded(h, [&](Engine &E) {
     E.require(E.have_positions && xyz && stride_bytes >= 3 * sizeof(double), "bad call");
-    std::vector<double> a(E.n), b(E.n), c(E.n);
-    E.x.download(a.data(), E.n, E.stream);
-    E.y.download(b.data(), E.n, E.stream);
-    E.z.download(c.data(), E.n, E.stream);
-    E.sync();
-    pdgpu::write_aos(xyz, stride_bytes, E.n, a, b, c);
+    pdgpu::xyz_to_host(E.stage, E.stream, E.x.p, E.y.p, E.z.p, E.n, xyz, stride_bytes);
   });
 }
 
 int pdgpu_set_velocities(pdgpu_engine *h, const double *xyz, size_t stride_bytes) {
   return pdgpu::guarded(h, [&](Engine &E) {
     E.require(xyz && stride_bytes >= 3 * sizeof(double), "bad velocity array");
-    std::vector<double> a, b, c;
-    pdgpu::read_aos(xyz, stride_bytes, E.n, a, b, c);
-    E.vx.upload(a, E.stream);
-    E.vy.upload(b, E.stream);
-    E.vz.upload(c, E.stream);
-    E.sync();
+    E.vx.resize(E.n);
+    E.vy.resize(E.n);
+    E.vz.resize(E.n);
+    pdgpu::xyz_to_device(E.stage, E.stream, xyz, stride_bytes, E.n, E.vx.p, E.vy.p, E.vz.p);
   });
 }
 
 int pdgpu_get_velocities(pdgpu_engine *h, double *xyz, size_t stride_bytes) {
   return pdgpu::guarded(h, [&](Engine &E) {
     E.require(xyz && stride_bytes >= 3 * sizeof(double) && E.vx.n >= (size_t)E.n, "bad call");
-    std::vector<double> a(E.n), b(E.n), c(E.n);
-    E.vx.download(a.data(), E.n, E.stream);
-    E.vy.download(b.data(), E.n, E.stream);
-    E.vz.download(c.data(), E.n, E.stream);
-    E.sync();
-    pdgpu::write_aos(xyz, stride_bytes, E.n, a, b, c);
+    pdgpu::xyz_to_host(E.stage, E.stream, E.vx.p, E.vy.p, E.vz.p, E.n, xyz, stride_bytes);
   });
 }
 

@@ -117,6 +117,59 @@ struct DBuf {
   }
 };
 
+// Host memory the GPU reads and writes directly (pinned), grown as needed: results
+// and states cross the bus in one kernel's loads or stores, where a copy to or from
+// pageable memory goes through the runtime's own staging.
+struct HostStage {
+  double *p = nullptr;
+  size_t n = 0;
+  HostStage() = default;
+  HostStage(const HostStage &) = delete;
+  HostStage &operator=(const HostStage &) = delete;
+  ~HostStage() {
+    if (p) (void)hipHostFree(p);
+  }
+  double *need(size_t count) {
+    if (count > n) {
+      if (p) (void)hipHostFree(p);
+      p = nullptr;
+      n = 0;
+      if (hipHostMalloc(reinterpret_cast<void **>(&p), count * sizeof(double)) != hipSuccess) {
+        (void)hipGetLastError();
+        p = nullptr;
+        throw EngineError(PDGPU_ERR_NOMEM,
+                          "pinned host allocation of " + std::to_string(count * sizeof(double)) + " bytes failed");
+      }
+      n = count;
+    }
+    return p;
+  }
+};
+// xyz vectors between the caller's array (any stride) and device SoA arrays; both
+// return when the data have arrived (state_io.hip)
+void xyz_to_device(HostStage &st, hipStream_t s, const double *xyz, size_t stride_bytes, int n, double *x, double *y,
+                   double *z);
+constexpr int kStagePiece = 1 << 18;  // atoms in pinned memory at once (6 MiB)
+void xyz_to_host(HostStage &st, hipStream_t s, const double *x, const double *y, const double *z, int n, double *xyz,
+                 size_t stride_bytes);
+
+// A trace of `count` doubles on its way to the caller: pinned up to 8 MiB, else pageable.
+struct TraceFetch {
+  std::vector<double> big;
+  const double *get(HostStage &st, const DBuf<double> &d, size_t count, hipStream_t s) {
+    double *h;
+    if (count <= (size_t)1 << 20) {
+      h = st.need(count);
+    } else {
+      big.resize(count);
+      h = big.data();
+    }
+    d.download(h, count, s);
+    PDGPU_HIP(hipStreamSynchronize(s));
+    return h;
+  }
+};
+
 // Position of one cluster slot: one 32-byte record, so a lane fetches it with
 // two 16-byte loads.
 struct alignas(32) SlotPos {
@@ -491,7 +544,7 @@ struct Engine {
   // (running it anyway would be harmless: the same values again)
   void begin_evaluation(bool nonbonded, double *eo = nullptr, bool opened = false);
   void forces_to_host(double *f, size_t stride_bytes);
-  DBuf<double> f_jm;  // forces in J/m (AoS), converted on the device for forces_to_host
+  HostStage stage;    // states, forces and traces on their way to or from the host
   // forces + energies into e_out (step < 0: LCPO in full); flush = false leaves the
   // energy sums pending for the caller's flush_sums
   void evaluate(uint32_t components, int step = -1, bool flush = true);
@@ -499,7 +552,7 @@ struct Engine {
   void energies_from_slots(uint32_t components, const double *h, pdgpu_energies *out) const;
   // noalloc.hip: the allocation-free evaluation of pdgpu_compute_noalloc
   double *scratch = nullptr;               // this device's file-scope scratch array (device address)
-  double *h_eout = nullptr;                // pinned copy of the energy slots
+  double *h_eout = nullptr;                // pinned: the energy slots, a partial update's results
   void evaluate_noalloc(uint32_t components, double *d_f, size_t stride_bytes, pdgpu_energies *out);
   // times trial_steps MD steps at each prune margin from the same state and keeps
   // the fastest (the state is restored; the next evaluation rebuilds the list)
@@ -516,8 +569,8 @@ struct Engine {
   // FF_NonBonded::calcEnergies with UsePartialRecalc (k_partial.hip): the
   // positions and energy terms (J) of the last evaluation, and the list's
   // full-update count then
-  DBuf<double> pr_x, pr_y, pr_z, pr_part, pr_sum, pr_rad, pr_eps, pr_chg;
-  DBuf<int> pr_moved, pr_count;
+  DBuf<double> pr_x, pr_y, pr_z, pr_part, pr_rad, pr_eps, pr_chg;
+  DBuf<int> pr_moved;
   bool pr_valid = false;
   uint32_t pr_update_count = 0;
   double pr_vdw = 0.0, pr_elec = 0.0;

@@ -224,6 +224,7 @@ struct Batch {
   int device = 0;
   hipStream_t stream = nullptr;
   std::string last_error;
+  HostStage stage;  // states and traces on their way to or from the host
   int nsys = 0, natoms = 0;
   std::vector<int> first, count;
   DBuf<double> x, y, z, vx, vy, vz, mass;
@@ -346,9 +347,8 @@ struct Batch {
     }
     hipLaunchKernelGGL(k_set_counters, dim3(1), dim3(64), 0, stream, counters.p, p.step_offset, 0);
     for (int s = 0; s < n; s++) PDGPU_HIP(hipGraphLaunch(graph_exec, stream));
-    std::vector<double> h((size_t)n * nsys * 2);
-    trace.download(h.data(), h.size(), stream);
-    sync();
+    TraceFetch tf;
+    const double *h = tf.get(stage, trace, (size_t)n * nsys * 2, stream);
     bool nan = false;
     for (int s = 0; s < n; s++)
       for (int k = 0; k < nsys; k++) {
@@ -613,29 +613,10 @@ static int batch_state(pdgpu_batch *h, int32_t sys, double *xyz, size_t stride, 
       throw EngineError(PDGPU_ERR_ARG, "bad system index or array");
     const int off = b.first[sys], n = b.count[sys];
     pdgpu::DBuf<double> *d[3] = {which ? &b.vx : &b.x, which ? &b.vy : &b.y, which ? &b.vz : &b.z};
-    std::vector<double> a(n), c(n), e(n);
-    std::vector<double> *v[3] = {&a, &c, &e};
-    if (set) {
-      for (int i = 0; i < n; i++) {
-        const double *p = reinterpret_cast<const double *>(reinterpret_cast<const char *>(xyz) + (size_t)i * stride);
-        a[i] = p[0];
-        c[i] = p[1];
-        e[i] = p[2];
-      }
-      for (int k = 0; k < 3; k++)
-        PDGPU_HIP(hipMemcpyAsync(d[k]->p + off, v[k]->data(), n * sizeof(double), hipMemcpyHostToDevice, b.stream));
-      b.sync();
-    } else {
-      for (int k = 0; k < 3; k++)
-        PDGPU_HIP(hipMemcpyAsync(v[k]->data(), d[k]->p + off, n * sizeof(double), hipMemcpyDeviceToHost, b.stream));
-      b.sync();
-      for (int i = 0; i < n; i++) {
-        double *p = reinterpret_cast<double *>(reinterpret_cast<char *>(xyz) + (size_t)i * stride);
-        p[0] = a[i];
-        p[1] = c[i];
-        p[2] = e[i];
-      }
-    }
+    if (set)
+      pdgpu::xyz_to_device(b.stage, b.stream, xyz, stride, n, d[0]->p + off, d[1]->p + off, d[2]->p + off);
+    else
+      pdgpu::xyz_to_host(b.stage, b.stream, d[0]->p + off, d[1]->p + off, d[2]->p + off, n, xyz, stride);
   });
 }
 

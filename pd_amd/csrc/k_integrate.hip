@@ -9,6 +9,7 @@
 // same forces a step reproduces the oracle's FP64 arithmetic.
 #include "engine.hpp"
 
+#include <algorithm>
 #include <cmath>
 
 namespace pdgpu {
@@ -612,15 +613,15 @@ void Engine::evaluate(uint32_t components, int step, bool flush) {
 }
 
 namespace {
-// The total force of every atom in PD's units (J/m), AoS: the fixed-point sums of
+// The total force of atoms first .. first + n - 1 in PD's units (J/m), AoS: the fixed-point sums of
 // the bonded / GB / LCPO accumulators and of the atom's nonbonded slot, converted
 // on the device so that one array of doubles crosses to the host.
-__global__ void k_forces_jm(int n, double conv, const long long *__restrict__ fbx, const long long *__restrict__ fby,
+__global__ void k_forces_jm(int first, int n, double conv, const long long *__restrict__ fbx, const long long *__restrict__ fby,
                             const long long *__restrict__ fbz, const long long *__restrict__ nbx,
                             const long long *__restrict__ nby, const long long *__restrict__ nbz,
                             const int *__restrict__ orig_slot, double *__restrict__ out) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
+  const int k = blockIdx.x * blockDim.x + threadIdx.x, i = first + k;
+  if (k >= n) return;
   long long fx = fbx[i], fy = fby[i], fz = fbz[i];
   if (nbx) {
     const int s = orig_slot[i];
@@ -628,36 +629,38 @@ __global__ void k_forces_jm(int n, double conv, const long long *__restrict__ fb
     fy += nby[s];
     fz += nbz[s];
   }
-  out[3 * i] = __dmul_rn((double)fx, conv);
-  out[3 * i + 1] = __dmul_rn((double)fy, conv);
-  out[3 * i + 2] = __dmul_rn((double)fz, conv);
+  out[3 * k] = __dmul_rn((double)fx, conv);
+  out[3 * k + 1] = __dmul_rn((double)fy, conv);
+  out[3 * k + 2] = __dmul_rn((double)fz, conv);
 }
 }  // namespace
 
 void Engine::forces_to_host(double *f, size_t stride_bytes) {
   const bool nbon = (last_components & PDGPU_NONBONDED) != 0;
   const double conv = Consts::kcalA_to_Jm() / kFixScale;
-  f_jm.resize((size_t)3 * n);
-  hipLaunchKernelGGL(k_forces_jm, dim3((n + 255) / 256), dim3(256), 0, stream, n, conv, fbx.p, fby.p, fbz.p,
-                     nbon ? nbx.p : nullptr, nby.p, nbz.p, orig_slot.p, f_jm.p);
-  PDGPU_HIP(hipGetLastError());
-  std::vector<double> h((size_t)3 * n);
-  f_jm.download(h.data(), h.size(), stream);
-  sync();
-  // PD's contract: the component adds into wspace.cur.atom[i].f
-  for (int i = 0; i < n; i++) {
-    double *p = reinterpret_cast<double *>(reinterpret_cast<char *>(f) + (size_t)i * stride_bytes);
-    p[0] += h[3 * i];
-    p[1] += h[3 * i + 1];
-    p[2] += h[3 * i + 2];
+  // the kernel stores to pinned host memory, in pieces for large systems
+  double *h = stage.need((size_t)3 * std::min(n, kStagePiece));
+  for (int first = 0; first < n; first += kStagePiece) {
+    const int m = std::min(kStagePiece, n - first);
+    hipLaunchKernelGGL(k_forces_jm, dim3((m + 255) / 256), dim3(256), 0, stream, first, m, conv, fbx.p, fby.p, fbz.p,
+                       nbon ? nbx.p : nullptr, nby.p, nbz.p, orig_slot.p, h);
+    PDGPU_HIP(hipGetLastError());
+    sync();
+    // PD's contract: the component adds into wspace.cur.atom[i].f
+    char *at = reinterpret_cast<char *>(f) + (size_t)first * stride_bytes;
+    for (int i = 0; i < m; i++) {
+      double *p = reinterpret_cast<double *>(at + (size_t)i * stride_bytes);
+      p[0] += h[3 * i];
+      p[1] += h[3 * i + 1];
+      p[2] += h[3 * i + 2];
+    }
   }
 }
 
 void Engine::energies_to_host(uint32_t components, pdgpu_energies *out) {
-  double h[24];
-  e_out.download(h, 24, stream);
+  e_out.download(h_eout, 24, stream);
   sync();
-  energies_from_slots(components, h, out);
+  energies_from_slots(components, h_eout, out);
 }
 
 // The energy slots (kcal/mol, layout of evaluate) as PD's Hamiltonian terms in J.
@@ -940,9 +943,8 @@ void Engine::md(const pdgpu_md_params &p, int n_steps, double *epot_trace, doubl
     PDGPU_HIP(hipGetLastError());
     fused_pending = false;
   }
-  std::vector<double> h((size_t)n_steps * 2);
-  trace.download(h.data(), h.size(), stream);
-  sync();
+  TraceFetch tf;
+  const double *h = tf.get(stage, trace, (size_t)n_steps * 2, stream);
   bool nan = false;
   for (int s = 0; s < n_steps; s++) {
     if (epot_trace) epot_trace[s] = h[2 * s];

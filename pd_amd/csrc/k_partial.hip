@@ -187,11 +187,25 @@ __global__ __launch_bounds__(256) void k_pr_update(PartialArgs A, const int *__r
   }
 }
 
-// The block sums in a fixed order (thread t: blocks t, t+256, ...; then the
-// threads in order), and the snapshot takes the current positions.
+// The first workgroup: the block sums in a fixed order (thread t: blocks t, t+256,
+// ...; then the threads in order), stored to out (pinned host memory).  The others:
+// the snapshot takes the current positions for the next update
+// (getWSpace().old = getWSpace().cur).
 __global__ __launch_bounds__(256) void k_pr_finish(int nparts, const double *__restrict__ part,
-                                                   double *__restrict__ out) {
+                                                   double *__restrict__ out, int n, const double *__restrict__ x,
+                                                   const double *__restrict__ y, const double *__restrict__ z,
+                                                   double *__restrict__ ox, double *__restrict__ oy,
+                                                   double *__restrict__ oz) {
   __shared__ double s[2][256];
+  if (blockIdx.x > 0) {
+    const int i = (blockIdx.x - 1) * 256 + threadIdx.x;
+    if (i < n) {
+      ox[i] = x[i];
+      oy[i] = y[i];
+      oz[i] = z[i];
+    }
+    return;
+  }
   double v = 0.0, e = 0.0;
   for (int k = threadIdx.x; k < nparts; k += 256) {
     v += part[2 * k];
@@ -230,15 +244,18 @@ void Engine::energy_update(uint32_t components, pdgpu_energies *out) {
   pr_y.resize(n);
   pr_z.resize(n);
   pr_moved.resize(n);
-  pr_count.resize(1);
+  // the count of moved atoms and the update's sums come back in pinned memory
+  int *h_count = reinterpret_cast<int *>(h_eout);
+  double *h_sum = h_eout + 1;
   // a list rebuild since the snapshot forces a full evaluation (nonbonded.cpp:1157-1162)
   const bool full = !pr_valid || !list_valid || pr_update_count != full_update_count;
   int m = 0;
   if (!full) {
     hipLaunchKernelGGL(k_pr_compact, dim3(1), dim3(kCompactThreads), 0, stream, n, x.p, y.p, z.p, pr_x.p, pr_y.p,
-                       pr_z.p, pr_moved.p, pr_count.p);
-    pr_count.download(&m, 1, stream);
+                       pr_z.p, pr_moved.p, h_count);
+    PDGPU_HIP(hipGetLastError());
     sync();
+    m = *h_count;
   }
   if (full || m > kPartialMax) {
     pr_rad.upload(h_radius, stream);
@@ -251,6 +268,9 @@ void Engine::energy_update(uint32_t components, pdgpu_energies *out) {
     pr_elec = e.epot_elec;
     pr_update_count = full_update_count;
     pr_valid = true;
+    hipLaunchKernelGGL(k_pr_snapshot, dim3(grid), dim3(T), 0, stream, n, x.p, y.p, z.p, pr_x.p, pr_y.p, pr_z.p);
+    PDGPU_HIP(hipGetLastError());
+    sync();
   } else if (m > 0) {
     PartialArgs A{};
     A.n = n;
@@ -283,22 +303,16 @@ void Engine::energy_update(uint32_t components, pdgpu_energies *out) {
     A.mid = mid;
     const int nb_blocks = grid;
     pr_part.resize((size_t)m * nb_blocks * 2);
-    pr_sum.resize(2);
     hipLaunchKernelGGL(k_pr_update, dim3(m, nb_blocks), dim3(256), 0, stream, A, pr_moved.p, x.p, y.p, z.p, pr_x.p,
                        pr_y.p, pr_z.p, pr_rad.p, pr_eps.p, pr_chg.p, band.p, sp_off.p, sp_part.p, sp_ord.p,
                        pr_part.p);
-    hipLaunchKernelGGL(k_pr_finish, dim3(1), dim3(256), 0, stream, m * nb_blocks, pr_part.p, pr_sum.p);
+    hipLaunchKernelGGL(k_pr_finish, dim3(1 + grid), dim3(256), 0, stream, m * nb_blocks, pr_part.p, h_sum, n, x.p,
+                       y.p, z.p, pr_x.p, pr_y.p, pr_z.p);
     PDGPU_HIP(hipGetLastError());
-    double d[2];
-    pr_sum.download(d, 2, stream);
     sync();
-    pr_vdw += d[0];
-    pr_elec += d[1];
+    pr_vdw += h_sum[0];
+    pr_elec += h_sum[1];
   }
-  // save the coordinates for the next update (getWSpace().old = getWSpace().cur)
-  hipLaunchKernelGGL(k_pr_snapshot, dim3(grid), dim3(T), 0, stream, n, x.p, y.p, z.p, pr_x.p, pr_y.p, pr_z.p);
-  PDGPU_HIP(hipGetLastError());
-  sync();
   pdgpu_energies e{};
   e.epot_vdw = pr_vdw;
   e.epot_elec = pr_elec;
