@@ -384,22 +384,14 @@ int pdgpu_full_update_count(pdgpu_engine *h, uint32_t *count) {
 int pdgpu_get_pair_count(pdgpu_engine *h, int64_t *total) {
   return pdgpu::guarded(h, [&](Engine &E) {
     E.require(total != nullptr, "null total");
-    std::vector<int> counts;
-    std::vector<uint32_t> packed;
-    E.export_pairs(counts, packed);
-    *total = (int64_t)packed.size();
+    *total = E.count_pairs();
   });
 }
 
 int pdgpu_get_pairs(pdgpu_engine *h, int32_t *counts, uint32_t *packed, int64_t capacity) {
   return pdgpu::guarded(h, [&](Engine &E) {
     E.require(counts && packed, "null output arrays");
-    std::vector<int> c;
-    std::vector<uint32_t> p;
-    E.export_pairs(c, p);
-    E.require((int64_t)p.size() <= capacity, "capacity too small for the pair set");
-    std::memcpy(counts, c.data(), sizeof(int) * c.size());
-    std::memcpy(packed, p.data(), sizeof(uint32_t) * p.size());
+    E.export_pairs(counts, packed, capacity);
   });
 }
 

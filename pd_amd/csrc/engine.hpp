@@ -508,7 +508,12 @@ struct Engine {
 
   // list.hip
   void build_list(bool deferred = false);  // deferred: the overflow check waits for finish_list_check
-  void export_pairs(std::vector<int> &counts, std::vector<uint32_t> &packed);
+  // export.hip: the list in PD's packed form
+  int64_t count_pairs();
+  void export_pairs(int32_t *counts, uint32_t *packed, int64_t capacity);
+  DBuf<int> ex_count;
+  DBuf<unsigned long long> ex_start, ex_total;
+  DBuf<uint32_t> ex_packed;
   // kernel timing instrumentation (HIP events on `stream`)
   bool timing = false;
   struct TimerSlot {

@@ -1095,51 +1095,4 @@ bool Engine::finish_list_check() {
   return false;
 }
 
-// PD's packed per-atom form of the pair set (neighbourlist.h:131-151), built on
-// the host from the device entries; used for parity checks and by callers that
-// read the list itself.
-void Engine::export_pairs(std::vector<int> &counts, std::vector<uint32_t> &packed) {
-  require(list_valid, "no neighbour list built");
-  std::vector<int> h_cnt(n_clusters), h_slot((size_t)n_clusters * kClusterSize);
-  std::vector<uint2> h_ent((size_t)n_clusters * entry_capacity);
-  cl_entry_count.download(h_cnt.data(), n_clusters, stream);
-  slot_orig.download(h_slot.data(), h_slot.size(), stream);
-  entries.download(h_ent.data(), h_ent.size(), stream);
-  sync();
-  std::vector<std::vector<uint32_t>> per(n);
-  for (int ci = 0; ci < n_clusters; ci++) {
-    for (int k = 0; k < h_cnt[ci]; k++) {
-      uint2 e = h_ent[(size_t)ci * entry_capacity + k];
-      int sb = (int)(e.x & 0xFFFFFFu);
-      int img = (int)((e.x >> 24) & 31u);
-      int ob = h_slot[sb];
-      unsigned lm = e.y & 0xFFu, codes = e.y >> 8;
-      for (int ii = 0; ii < kClusterSize; ii++) {
-        if (!((lm >> ii) & 1u)) continue;
-        int oa = h_slot[ci * kClusterSize + ii];
-        int c = (codes >> (2 * ii)) & 3;
-        uint32_t bo = c == 0 ? 7u : (uint32_t)c;
-        int hi = std::max(oa, ob), lo = std::min(oa, ob);
-        int img_pd = (oa > ob) ? img : 26 - img;  // image of p_lo - p_hi
-        uint32_t w_hi = (uint32_t)lo | (bo << 24);
-        uint32_t w_lo = (uint32_t)hi | (bo << 24);
-        if (periodic) {
-          w_hi |= (uint32_t)(img_pd & 31) << 27;
-          w_lo |= (uint32_t)((26 - img_pd) & 31) << 27;
-        }
-        per[hi].push_back(w_hi);
-        if (calc_shadow) per[lo].push_back(w_lo);
-      }
-    }
-  }
-  counts.assign(n, 0);
-  packed.clear();
-  for (int i = 0; i < n; i++) {
-    auto &v = per[i];
-    std::sort(v.begin(), v.end(), [](uint32_t a, uint32_t b) { return (a & 0xFFFFFFu) < (b & 0xFFFFFFu); });
-    counts[i] = (int)v.size();
-    packed.insert(packed.end(), v.begin(), v.end());
-  }
-}
-
 }  // namespace pdgpu

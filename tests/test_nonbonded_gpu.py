@@ -9,7 +9,7 @@ import pytest
 
 from pd_amd import engine as G
 from pd_amd import systems as S
-from tests.helpers import energy_close, oracle_nb, rel_rms
+from tests.helpers import O, energy_close, oracle_list, oracle_nb, rel_rms
 
 pytestmark = pytest.mark.gpu
 
@@ -78,6 +78,24 @@ def test_water_pair_set_exact_at_the_limit():
     for a, b, expect in cases:  # the construction really puts pairs on both sides of the limit
         assert _listed(counts, packed, a, b) == expect, (a, b)
     e = _engine(s, WATER_NB, 2.0)
+    e.build_list()
+    gc, gp = e.get_pairs()
+    assert np.array_equal(gc, counts)
+    assert np.array_equal(gp, packed)
+
+
+@pytest.mark.parametrize("n_waters,shadow", [(1, False), (1, True), (43, True), (2732, False)])
+def test_pair_set_row_lengths(n_waters, shadow):
+    # every pair is within the cutoff, so the rows have every length from none up
+    # to 8,195 words: past one sort's 256 threads, each power of two, the longest
+    # row sorted on the device (8,192), and many pieces of the transfer
+    s = S.water_box(n_waters, seed=n_waters)
+    s.box = None
+    print(f"case rows n={3 * n_waters} shadow={shadow}", flush=True)
+    counts, packed = oracle_list(s, O.clean_space(s), 80.0, 2.0, shadow)
+    assert counts.max() == 3 * n_waters - 1
+    e = G.engine_for(s, G.nb_params(Cutoff=80.0, InnerCutoff=70.0, VdwCutoff=80.0, VdwInnerCutoff=70.0),
+                     padding=2.0, calc_shadow=shadow)
     e.build_list()
     gc, gp = e.get_pairs()
     assert np.array_equal(gc, counts)
