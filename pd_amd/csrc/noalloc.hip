@@ -98,7 +98,7 @@ void Engine::evaluate_noalloc(uint32_t components, double *d_f, size_t stride_by
                 pcount_nolj.n >= (size_t)max_clusters,
             "engine buffers not sized: build the neighbour list first");
   }
-  const size_t n_nb = nbon ? (size_t)max_groups * 4 : 0;
+  const size_t n_nb = nbon ? (size_t)max_groups * nb_parts * 4 : 0;
   const size_t n_b = bon ? (size_t)bonded_blocks(nbonds, nangles, ntors) * 4 : 0;
   const size_t need = kScratchSlots + n_nb + n_b;
   if (need > kScratchDoubles)

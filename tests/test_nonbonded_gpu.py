@@ -143,6 +143,30 @@ def test_water_forces(mode):
     assert abs(en["virial"] - e_ref["virial"]) <= 1e-5 * abs(e_ref["virial"])
 
 
+@pytest.mark.parametrize("n_waters", [1, 729, 2197, 6859])
+def test_water_forces_by_size(n_waters):
+    # one partly filled cluster, then boxes on each side of the lines between four, two
+    # and one workgroup per group (the first two in FP64, two waves to a cluster).  A step's recorded energy is
+    # summed by a workgroup of the next step's kernel, from the same partials.
+    s = S.water_box(n_waters, seed=n_waters)
+    if n_waters == 1:
+        s.box = None
+    print(f"case water n={n_waters} forces", flush=True)
+    pos, counts, packed, f_ref, e_ref = oracle_nb(s, WATER_NB, padding=2.0)
+    e = G.engine_for(s, G.nb_params(**WATER_NB), padding=2.0)
+    e.build_list()
+    f, en = e.compute(G.PDGPU_NONBONDED)
+    f2, en2 = e.compute(G.PDGPU_NONBONDED)
+    assert np.array_equal(f, f2) and en == en2
+    assert np.array_equal(f, f_ref) if n_waters == 1 else rel_rms(f, f_ref) <= 1e-5
+    assert energy_close(en["epot"], e_ref["epot_vdw"] + e_ref["epot_elec"], e_ref["abs_sum"])
+    e.set_velocities(np.zeros((e.n, 3)))
+    md = G.MDParams(integrator=G.PDGPU_VELOCITY_VERLET, components=G.PDGPU_NONBONDED, timestep=1e-15,
+                    update_nlist=0, step_offset=0, total_steps=10, seed=1)
+    trace = e.md(md, 2)[0]
+    assert abs(trace[0] - en["epot"]) <= 1e-12 * e_ref["abs_sum"]
+
+
 @pytest.mark.parametrize("cuts", [(10.0, 8.0, 8.0, 6.0), (8.0, 6.0, 10.0, 8.0)])
 def test_water_forces_distinct_cutoffs(cuts):
     # VdwCutoff independent of Cutoff (nonbonded.cpp:722, 742): the kernel then
