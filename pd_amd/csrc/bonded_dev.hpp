@@ -1,7 +1,8 @@
 // bonded_dev.hpp -- the device code of FF_Bonded's terms (bonds, angles,
-// torsions and impropers, FP64), shared by the bonded kernel (k_bonded.hip)
-// and the nonbonded kernel, whose last workgroups take the bonded terms of the
-// same evaluation (k_nonbonded.hip).  Included by those two files only.
+// torsions and impropers, FP64), shared by the bonded kernel (k_bonded.hip),
+// the nonbonded kernel, whose last workgroups take the bonded terms of the
+// same evaluation (k_nonbonded.hip), and the opening kernel of a GB evaluation, whose
+// first ones do (k_gb.hip).  Included by those three files only.
 #pragma once
 
 #include "engine.hpp"

@@ -310,6 +310,23 @@ struct PlainGB {
   double still2, cut2, vdwcut, inner, vdwinner, invw, vinvw, premul, ec_in, ec_out, thresh;
   double P4, P5, invP5, vdw14, elec14, halfeconv, offset, pi;
 };
+// What shares the opening launch of a GB evaluation (k_gb_open): the bonded terms, whose
+// 256-term blocks have no matrix of pairs to hide behind, and a previous step's sums.
+struct GBOpen {
+  BondedArrays bonded;
+  int bonded_blocks = 0;
+  double *bonded_partial = nullptr, *bonded_eterm = nullptr;
+  const struct SumList *sums = nullptr;
+};
+// The final energy sums of a GB evaluation, for a launch that other sums share
+// (gb_sums_block): per system the tile pairs' and the self energies.
+struct GBSums {
+  const double *part, *eself;
+  const int *beg, *end, *first, *count;
+  double *out;
+  int stride, off;
+  int slots;  // of the tile pairs' four sums written (the fourth is zero)
+};
 struct GBState {
   pdgpu_gb_params prm{};
   GBK kp{}, kr{};  // of the pair pass; of radii and chain
@@ -337,7 +354,11 @@ struct GBState {
                   const std::vector<int> &spj, const std::vector<int> &spo);
   void upload(hipStream_t s);
   void run(hipStream_t s, const double *x, const double *y, const double *z, long long *fx, long long *fy,
-           long long *fz, double *out, int out_stride, int out_off, Engine *timer_owner, bool energy_only = false);
+           long long *fz, double *out, int out_stride, int out_off, Engine *timer_owner, bool energy_only = false,
+           const GBOpen *open = nullptr, bool sums = true);  // sums = false: left to the caller (sum_args)
+  GBSums sum_args(double *out, int out_stride, int out_off, int slots = 4) const {
+    return GBSums{e_part.p, eself.p, slot_beg.p, slot_end.p, sys_first.p, sys_count.p, out, out_stride, out_off, slots};
+  }
   // wavefronts per task of the radii, pair and chain passes (1, 2 or 4; 0: by the
   // number of tasks)
   int split[3] = {0, 0, 0};
@@ -375,10 +396,14 @@ struct LCPOState {
                   const double *sigma_j);
   void append(const LCPOState &o, int first);  // another system's atoms, as they are
   void upload(hipStream_t s);
-  // full: recompute now; otherwise recompute when step % update == 0 (step from
-  // step_ptr on the device when given, else step_host) and re-apply otherwise
+  // full: recompute now; otherwise recompute when step % update == 0 and re-apply
+  // the stored forces otherwise.  block_part: the energies' 4-wide block sums too;
+  // gb: the launch of the forces also takes these energy sums
   void run(hipStream_t s, const double *x, const double *y, const double *z, long long *fx, long long *fy,
-           long long *fz, const int *step_ptr, int step_host, bool full, bool energy_only = false);
+           long long *fz, int step, bool full, bool energy_only = false, double *block_part = nullptr,
+           const GBSums *gb = nullptr);
+  // a step that takes the stored areas and forces again
+  bool reapplies(int step) const { return update > 0 && step % update != 0; }
 };
 
 void gb_fixed_terms(int n, const double *gbrad, const pdgpu_gb_params &p, const int32_t *off12,
@@ -554,11 +579,13 @@ struct Engine {
   // bonded.hip
   // energies: bond, angle, torsion, virial; partial: bonded_blocks * 4 doubles
   void launch_bonded(double *energy_slots, double *partial = nullptr);
+  BondedArrays bonded_arrays() const;
   // integrate.hip
   // clears accumulators and the energy slots eo (default e_out) and gathers slot positions
   // opened: the previous MD step's integrator did the opening kernel's work
   // (running it anyway would be harmless: the same values again)
-  void begin_evaluation(bool nonbonded, double *eo = nullptr, bool opened = false);
+  // gb_next: without the nonbonded term, the pending sums are left to the GB opening
+  void begin_evaluation(bool nonbonded, double *eo = nullptr, bool opened = false, bool gb_next = false);
   void forces_to_host(double *f, size_t stride_bytes);
   HostStage stage;    // states, forces and traces on their way to or from the host
   // forces + energies into e_out (step < 0: LCPO in full); flush = false leaves the
@@ -605,11 +632,15 @@ struct Engine {
   // k_lcpo.hip
   std::unique_ptr<LCPOState> lcpo;
   DBuf<double> e_partial_lcpo;
-  void launch_lcpo(double *energy_slot, int step, bool full, bool energy_only = false);
+  // with_gb: the launch of the surface energies also runs the GB energy sums
+  void launch_lcpo(double *energy_slot, int step, bool full, bool energy_only = false, const GBSums *with_gb = nullptr);
   // k_gb.hip
   bool have_gb = false;
   std::unique_ptr<GBState> gb;
-  void launch_gb(double *energy_slots, bool energy_only = false);
+  // bonded_slots: the bonded terms run in the opening launch (their sums go there)
+  void launch_gb(double *energy_slots, bool energy_only = false, double *bonded_slots = nullptr, bool sums = true);
+  SumList gb_sums{};  // a previous step's sums, for that launch
+  int gb_bonded_sel = 0;
 
 };
 
@@ -836,6 +867,7 @@ constexpr int kDmaxStride = 16;
 // position into the slot arrays, its displacement since the last prune folded
 // into the next evaluation's set of maxima, the other set cleared, and the
 // force accumulators cleared once the integrator has read them.
+// Without the nonbonded term (spos null) only the accumulators are cleared.
 struct OpenNext {
   int on;
   int cur;  // the set of maxima of the next evaluation
@@ -851,6 +883,14 @@ struct OpenNext {
 // loaded by the caller with its other loads), (px, py, pz) its new position.
 __device__ __forceinline__ void open_next_at(const OpenNext &O, int i, int n, int s, const SlotPos &r,
                                              double px, double py, double pz) {
+  if (!O.spos) {
+    if (i < n) {
+      O.fbx[i] = 0;
+      O.fby[i] = 0;
+      O.fbz[i] = 0;
+    }
+    return;
+  }
   double d = 0.0;
   if (i < n) {
     SlotPos p;
@@ -882,7 +922,7 @@ __device__ __forceinline__ void open_next(const OpenNext &O, int i, int n, const
                                           double px, double py, double pz) {
   int s = 0;
   SlotPos r{};
-  if (i < n) {
+  if (i < n && O.spos) {
     s = orig_slot[i];
     r = O.pref[s];
   }
@@ -1013,6 +1053,36 @@ __device__ __forceinline__ void sum_lists(const SumList &L) {
     if (R.use_gb) ep += E[8] + E[9] + E[10] + E[12];
     R.trace[2 * R.step] = ep * R.kcal_to_J;
     R.trace[2 * R.step + 1] = E[20];
+  }
+}
+
+// GB's energy sums: `which` 0 sums system sysi's 4-wide tile-pair partials into slots
+// off .. off + slots - 1, 1 its self energies into slot off + 4 (thread-strided sums, then a
+// tree).  Run by a whole workgroup of 256 threads; s: 4 x 256 doubles of LDS.
+__device__ __forceinline__ void gb_sums_block(const GBSums &G, int sysi, int which, double (*s)[256]) {
+  double *out = G.out + (size_t)sysi * G.stride + G.off;
+  if (which == 0) {
+    double a[4] = {0, 0, 0, 0};
+    for (int k = G.beg[sysi] + threadIdx.x; k < G.end[sysi]; k += 256)
+      for (int d = 0; d < 4; d++) a[d] += G.part[4 * k + d];
+    for (int d = 0; d < 4; d++) s[d][threadIdx.x] = a[d];
+    __syncthreads();
+    for (int w = 128; w > 0; w >>= 1) {
+      if ((int)threadIdx.x < w)
+        for (int d = 0; d < 4; d++) s[d][threadIdx.x] += s[d][threadIdx.x + w];
+      __syncthreads();
+    }
+    if ((int)threadIdx.x < G.slots) out[threadIdx.x] = s[threadIdx.x][0];
+  } else {
+    double a = 0.0;
+    for (int k = threadIdx.x; k < G.count[sysi]; k += 256) a += G.eself[G.first[sysi] + k];
+    s[0][threadIdx.x] = a;
+    __syncthreads();
+    for (int w = 128; w > 0; w >>= 1) {
+      if ((int)threadIdx.x < w) s[0][threadIdx.x] += s[0][threadIdx.x + w];
+      __syncthreads();
+    }
+    if (threadIdx.x == 0) out[4] = s[0][0];
   }
 }
 

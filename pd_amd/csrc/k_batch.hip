@@ -28,8 +28,13 @@ constexpr int kStride = 12;  // per-system energy slots, kcal/mol except [8]
 // [0] GB cross  [1] vdW  [2] elec  [3] LCPO cavity  [4] GB self  [5] bond  [6] angle
 // [7] torsion  [8] kinetic (J)  [9] epot (J)
 
-__global__ void k_zero3n(long long *__restrict__ a, long long *__restrict__ b, long long *__restrict__ c, int n) {
+// A step's first kernel: clears the accumulators and moves the step counters on
+// (counters[0]: protocol step, for the Langevin first/last-step guards and the noise;
+// counters[1]: trace row).
+__global__ void k_zero3n(long long *__restrict__ a, long long *__restrict__ b, long long *__restrict__ c, int n,
+                         int *__restrict__ counters) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < 2 && counters) counters[i] += 1;
   if (i < n) {
     a[i] = 0;
     b[i] = 0;
@@ -66,8 +71,13 @@ struct SegLists {
   const int *beg[4], *end[4];
   int off[4];
 };
-__global__ void k_seg_sums(SegLists L, double *__restrict__ out, int stride) {
+__global__ __launch_bounds__(256) void k_seg_sums(SegLists L, double *__restrict__ out, int stride, GBSums G) {
+  __shared__ double s[4][256];
   const int sysi = blockIdx.x, y = blockIdx.y;
+  if (y >= L.n) {  // the GB energies
+    gb_sums_block(G, sysi, y - L.n, s);
+    return;
+  }
   const double t = seg_sum_block(L.v[y], L.beg[y][sysi], L.end[y][sysi]);
   if (threadIdx.x == 0) out[(size_t)sysi * stride + L.off[y]] = t;
 }
@@ -178,13 +188,6 @@ __global__ void k_batch_record(int nsys, const double *__restrict__ ke, const in
   }
 }
 
-__global__ void k_advance(int *__restrict__ counters) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) {
-    counters[0] += 1;  // protocol step (Langevin first/last-step guards, noise counter)
-    counters[1] += 1;  // trace row
-  }
-}
-
 __global__ void k_set_counters(int *__restrict__ counters, int step, int local) {
   if (threadIdx.x == 0 && blockIdx.x == 0) {
     counters[0] = step;
@@ -244,9 +247,10 @@ struct Batch {
   DBuf<double> e_sys, temps, trace;
   DBuf<int> counters;
   std::vector<double> h_temps;
-  // graph of one step
-  hipGraph_t graph = nullptr;
-  hipGraphExec_t graph_exec = nullptr;
+  // graphs of one step: in full, and (LCPO with UpdateSasa > 1) of a step that applies the
+  // stored surface forces again, without the three kernels that would return at once
+  hipGraph_t graph[2] = {nullptr, nullptr};
+  hipGraphExec_t graph_exec[2] = {nullptr, nullptr};
   BatchLangevin graph_args{};
   uint32_t graph_components = 0;
   int graph_trace_rows = 0;
@@ -255,8 +259,10 @@ struct Batch {
   DBuf<double> swap_f;
 
   ~Batch() {
-    if (graph_exec) (void)hipGraphExecDestroy(graph_exec);
-    if (graph) (void)hipGraphDestroy(graph);
+    for (int k = 0; k < 2; k++) {
+      if (graph_exec[k]) (void)hipGraphExecDestroy(graph_exec[k]);
+      if (graph[k]) (void)hipGraphDestroy(graph[k]);
+    }
     if (stream) {
       (void)hipStreamSynchronize(stream);
       (void)hipStreamDestroy(stream);
@@ -264,16 +270,28 @@ struct Batch {
   }
   void sync() { PDGPU_HIP(hipStreamSynchronize(stream)); }
 
-  void record_step(uint32_t comps, const BatchLangevin &L) {
+  void record_step(uint32_t comps, const BatchLangevin &L, bool reapply) {
     const int T = 256;
-    hipLaunchKernelGGL(k_zero3n, dim3((natoms + T - 1) / T), dim3(T), 0, stream, fx.p, fy.p, fz.p, natoms);
-    if ((comps & PDGPU_GB) && have_gb) gb->run(stream, x.p, y.p, z.p, fx.p, fy.p, fz.p, e_sys.p, kStride, 0, nullptr);
-    // the per-system sums of the bonded terms and LCPO, one launch for all
-    SegLists sl{};
-    if ((comps & PDGPU_BONDED) && nb + na + nt > 0) {
-      BondedArrays B{nb, na, nt, bi.p, bj.p, bl.p, bk.p, ai.p, aa.p, aj.p, at0.p, ak.p,
-                     ti.p, ta.p, tb.p, tj.p, tterms.p, tvn.p, tnn.p, tgamma.p, bwin.p};
+    hipLaunchKernelGGL(k_zero3n, dim3((natoms + T - 1) / T), dim3(T), 0, stream, fx.p, fy.p, fz.p, natoms,
+                       counters.p);
+    const bool gbon = (comps & PDGPU_GB) && have_gb, bon = (comps & PDGPU_BONDED) && nb + na + nt > 0;
+    const BondedArrays B{nb, na, nt, bi.p, bj.p, bl.p, bk.p, ai.p, aa.p, aj.p, at0.p, ak.p,
+                         ti.p, ta.p, tb.p, tj.p, tterms.p, tvn.p, tnn.p, tgamma.p, bwin.p};
+    if (gbon) {
+      GBOpen O{};
+      if (bon) {
+        O.bonded = B;
+        O.bonded_blocks = bonded_blocks(nb, na, nt);
+        O.bonded_partial = epart_dummy.p;
+        O.bonded_eterm = eterm.p;
+      }
+      gb->run(stream, x.p, y.p, z.p, fx.p, fy.p, fz.p, e_sys.p, kStride, 0, nullptr, false, &O, false);
+    } else if (bon) {
       launch_bonded_kernel(stream, B, x.p, y.p, z.p, fx.p, fy.p, fz.p, epart_dummy.p, eterm.p);
+    }
+    // the per-system sums of the bonded terms, LCPO and GB, one launch for all
+    SegLists sl{};
+    if (bon) {
       for (int c = 0; c < 3; c++) {
         sl.v[sl.n] = eterm.p;
         sl.beg[sl.n] = seg_beg[c].p;
@@ -281,20 +299,31 @@ struct Batch {
         sl.off[sl.n++] = 5 + c;
       }
     }
-    if ((comps & PDGPU_SASA) && lcpo) {
-      lcpo->run(stream, x.p, y.p, z.p, fx.p, fy.p, fz.p, counters.p, 0, false);
+    const bool sasa = (comps & PDGPU_SASA) && lcpo;
+    if (sasa) {
+      lcpo->run(stream, x.p, y.p, z.p, fx.p, fy.p, fz.p, reapply ? 1 : 0, !reapply);
       sl.v[sl.n] = lcpo->eatom.p;
       sl.beg[sl.n] = atom_beg.p;
       sl.end[sl.n] = atom_end.p;
       sl.off[sl.n++] = 3;
     }
-    if (sl.n > 0) hipLaunchKernelGGL(k_seg_sums, dim3(nsys, sl.n), dim3(256), 0, stream, sl, e_sys.p, kStride);
+    if (sl.n > 0 || gbon)
+      hipLaunchKernelGGL(k_seg_sums, dim3(nsys, sl.n + (gbon ? 2 : 0)), dim3(256), 0, stream, sl, e_sys.p, kStride,
+                         gbon ? gb->sum_args(e_sys.p, kStride, 0, sasa ? 3 : 4) : GBSums{});  // slot 3: LCPO's
     hipLaunchKernelGGL(k_batch_integrate, dim3((natoms + T - 1) / T), dim3(T), 0, stream, natoms, L, counters.p,
                        atom_sys.p, sys_first.p, temps.p, mass.p, fx.p, fy.p, fz.p, x.p, y.p, z.p, vx.p, vy.p, vz.p,
                        ke.p);
     hipLaunchKernelGGL(k_batch_record, dim3(nsys), dim3(256), 0, stream, nsys, ke.p, atom_beg.p, atom_end.p, e_sys.p,
                        Consts::kcal_to_J(), counters.p, trace.p);
-    hipLaunchKernelGGL(k_advance, dim3(1), dim3(64), 0, stream, counters.p);
+  }
+
+  void drop_graphs() {
+    for (int k = 0; k < 2; k++) {
+      if (graph_exec[k]) PDGPU_HIP(hipGraphExecDestroy(graph_exec[k]));
+      graph_exec[k] = nullptr;
+      if (graph[k]) PDGPU_HIP(hipGraphDestroy(graph[k]));
+      graph[k] = nullptr;
+    }
   }
 
   void zero_energies() {
@@ -327,26 +356,29 @@ struct Batch {
     L.stream = p.noise_stream;
     L.conv = Consts::kcalA_to_Jm() / kFixScale;
     const int rows = n;
-    const bool rebuild = !graph_exec || graph_components != p.components || graph_trace_rows < rows ||
+    const bool rebuild = !graph_exec[0] || graph_components != p.components || graph_trace_rows < rows ||
                          std::memcmp(&graph_args, &L, sizeof(L)) != 0;
     if (rebuild) {
-      if (graph_exec) PDGPU_HIP(hipGraphExecDestroy(graph_exec));
-      if (graph) PDGPU_HIP(hipGraphDestroy(graph));
-      graph_exec = nullptr;
-      graph = nullptr;
+      drop_graphs();
       trace.resize((size_t)rows * nsys * 2);
       zero_energies();
       sync();
-      PDGPU_HIP(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
-      record_step(p.components, L);
-      PDGPU_HIP(hipStreamEndCapture(stream, &graph));
-      PDGPU_HIP(hipGraphInstantiate(&graph_exec, graph, nullptr, nullptr, 0));
+      const bool two = (p.components & PDGPU_SASA) && lcpo && lcpo->reapplies(1);
+      for (int k = 0; k < (two ? 2 : 1); k++) {
+        PDGPU_HIP(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
+        record_step(p.components, L, k == 1);
+        PDGPU_HIP(hipStreamEndCapture(stream, &graph[k]));
+        PDGPU_HIP(hipGraphInstantiate(&graph_exec[k], graph[k], nullptr, nullptr, 0));
+      }
       graph_args = L;
       graph_components = p.components;
       graph_trace_rows = rows;
     }
-    hipLaunchKernelGGL(k_set_counters, dim3(1), dim3(64), 0, stream, counters.p, p.step_offset, 0);
-    for (int s = 0; s < n; s++) PDGPU_HIP(hipGraphLaunch(graph_exec, stream));
+    hipLaunchKernelGGL(k_set_counters, dim3(1), dim3(64), 0, stream, counters.p, p.step_offset - 1, -1);
+    for (int s = 0; s < n; s++) {
+      const bool reapply = graph_exec[1] && lcpo->reapplies(p.step_offset + s);
+      PDGPU_HIP(hipGraphLaunch(graph_exec[reapply ? 1 : 0], stream));
+    }
     TraceFetch tf;
     const double *h = tf.get(stage, trace, (size_t)n * nsys * 2, stream);
     bool nan = false;
@@ -582,10 +614,7 @@ int pdgpu_batch_set_temperatures(pdgpu_batch *h, const double *temps) {
 }
 
 static void drop_graph(Batch &b) {  // the recorded step no longer matches the launch settings
-  if (b.graph_exec) PDGPU_HIP(hipGraphExecDestroy(b.graph_exec));
-  if (b.graph) PDGPU_HIP(hipGraphDestroy(b.graph));
-  b.graph_exec = nullptr;
-  b.graph = nullptr;
+  b.drop_graphs();
 }
 
 int pdgpu_batch_set_gb_split(pdgpu_batch *h, const int32_t *split) {
@@ -638,13 +667,13 @@ int pdgpu_batch_compute(pdgpu_batch *h, uint32_t components, double *f_accum, pd
     const int T = 256;
     b.zero_energies();
     hipLaunchKernelGGL(pdgpu::k_zero3n, dim3((b.natoms + T - 1) / T), dim3(T), 0, b.stream, b.fx.p, b.fy.p, b.fz.p,
-                       b.natoms);
+                       b.natoms, nullptr);
     const bool eonly = (components & PDGPU_ENERGY_ONLY) != 0;
     if (eonly && f_accum) throw EngineError(PDGPU_ERR_ARG, "PDGPU_ENERGY_ONLY computes no forces: f_accum must be NULL");
     if ((components & PDGPU_GB) && b.have_gb)
       b.gb->run(b.stream, b.x.p, b.y.p, b.z.p, b.fx.p, b.fy.p, b.fz.p, b.e_sys.p, pdgpu::kStride, 0, nullptr, eonly);
     if ((components & PDGPU_SASA) && b.lcpo) {
-      b.lcpo->run(b.stream, b.x.p, b.y.p, b.z.p, b.fx.p, b.fy.p, b.fz.p, nullptr, 0, true, eonly);
+      b.lcpo->run(b.stream, b.x.p, b.y.p, b.z.p, b.fx.p, b.fy.p, b.fz.p, 0, true, eonly);
       hipLaunchKernelGGL(pdgpu::k_seg_sum, dim3(b.nsys), dim3(256), 0, b.stream, b.lcpo->eatom.p, b.atom_beg.p,
                          b.atom_end.p, b.e_sys.p, pdgpu::kStride, 3);
     }

@@ -62,15 +62,18 @@ void launch_bonded_kernel(hipStream_t s, const BondedArrays &B, const double *x,
   hipLaunchKernelGGL(k_bonded, dim3(grid), dim3(256), 0, s, B, x, y, z, fx, fy, fz, partial, eterm);
 }
 
+BondedArrays Engine::bonded_arrays() const {
+  return BondedArrays{nbonds, nangles, ntors, b_i.p, b_j.p, b_l.p, b_k.p, a_i.p, a_a.p, a_j.p, a_t0.p, a_k.p,
+                      t_i.p, t_a.p, t_b.p, t_j.p, t_terms.p, t_vn.p, t_nn.p, t_gamma.p, b_win.p};
+}
+
 void Engine::launch_bonded(double *energy_out, double *partial) {
   const int grid = bonded_blocks(nbonds, nangles, ntors);
   if (!partial) {
     e_partial_bonded.resize((size_t)grid * 4);
     partial = e_partial_bonded.p;
   }
-  BondedArrays B{nbonds, nangles, ntors, b_i.p, b_j.p, b_l.p, b_k.p, a_i.p, a_a.p, a_j.p, a_t0.p, a_k.p,
-                 t_i.p, t_a.p, t_b.p, t_j.p, t_terms.p, t_vn.p, t_nn.p, t_gamma.p, b_win.p};
-  launch_bonded_kernel(stream, B, x.p, y.p, z.p, fbx.p, fby.p, fbz.p, partial, nullptr);
+  launch_bonded_kernel(stream, bonded_arrays(), x.p, y.p, z.p, fbx.p, fby.p, fbz.p, partial, nullptr);
   PDGPU_HIP(hipGetLastError());
   defer_sum4(partial, grid, energy_out);
 }

@@ -50,6 +50,7 @@
 #include <mutex>
 #include <tuple>
 
+#include "bonded_dev.hpp"
 #include "engine.hpp"
 
 namespace pdgpu {
@@ -108,11 +109,29 @@ __global__ __launch_bounds__(64) void k_gb_codes(const GBTask *__restrict__ task
 // Opens an evaluation: each tile's centre (of its atoms' box) and the largest
 // distance of an atom from it, its largest GB radius; clears the Gpol sums.  One
 // wavefront per tile.
-__global__ __launch_bounds__(256) void k_gb_tiles(int ntiles, const int2 *__restrict__ tile_atoms,
-                                                  const double *__restrict__ x, const double *__restrict__ y,
-                                                  const double *__restrict__ z, const float *__restrict__ gbrad,
-                                                  GBTile *__restrict__ tiles, long long *__restrict__ gpol) {
-  const int t = blockIdx.x * 4 + ((int)threadIdx.x >> 6), lane = threadIdx.x & 63;
+//
+// The launch opens an evaluation: its first workgroups take the bonded terms (FP64 chains
+// of a few us that no other kernel depends on), its last the previous MD step's energy
+// sums.  With those launches gone, and the GB and surface energy sums in the launch of
+// the surface forces, a step of a 20-residue chain takes 64 us where it took 85.
+__global__ __launch_bounds__(256) void k_gb_open(int ntiles, const int2 *__restrict__ tile_atoms,
+                                                 const double *__restrict__ x, const double *__restrict__ y,
+                                                 const double *__restrict__ z, const float *__restrict__ gbrad,
+                                                 GBTile *__restrict__ tiles, long long *__restrict__ gpol,
+                                                 BondedArrays B, int bonded, long long *__restrict__ fx,
+                                                 long long *__restrict__ fy, long long *__restrict__ fz,
+                                                 double *__restrict__ bonded_partial,
+                                                 double *__restrict__ bonded_eterm, SumList L) {
+  __shared__ long long window[3 * kBondedWindow];
+  if ((int)blockIdx.x < bonded) {
+    bonded_block((int)blockIdx.x, B, x, y, z, fx, fy, fz, bonded_partial, bonded_eterm, window);
+    return;
+  }
+  if ((L.n > 0 || L.record) && blockIdx.x == gridDim.x - 1) {
+    sum_lists<true>(L);
+    return;
+  }
+  const int t = ((int)blockIdx.x - bonded) * 4 + ((int)threadIdx.x >> 6), lane = threadIdx.x & 63;
   if (t >= ntiles) return;  // whole waves; no barrier follows
   const int2 A = tile_atoms[t];
   const bool on = lane < A.y;
@@ -954,38 +973,10 @@ __global__ void k_seg_sum_atoms(const double *__restrict__ v, const int *__restr
   if (threadIdx.x == 0) out[(size_t)sysi * out_stride + out_off] = s[0];
 }
 
-// A GB evaluation's per-system energies in one launch: block (s, 0) sums system
-// s's 4-wide tile partials into slots out_off .. out_off + 3, block (s, 1) its
-// self energies into slot out_off + 4 (thread-strided sums, then a tree).
-__global__ void k_gb_sums(const double *__restrict__ part, const int *__restrict__ beg,
-                          const int *__restrict__ endp, const double *__restrict__ eself,
-                          const int *__restrict__ first, const int *__restrict__ count, double *__restrict__ out,
-                          int out_stride, int out_off) {
+// A GB evaluation's energies in a launch of their own: block (s, k) takes system s's.
+__global__ __launch_bounds__(256) void k_gb_sums(GBSums G) {
   __shared__ double s[4][256];
-  const int sysi = blockIdx.x;
-  if (blockIdx.y == 0) {
-    double a[4] = {0, 0, 0, 0};
-    for (int k = beg[sysi] + threadIdx.x; k < endp[sysi]; k += 256)
-      for (int d = 0; d < 4; d++) a[d] += part[4 * k + d];
-    for (int d = 0; d < 4; d++) s[d][threadIdx.x] = a[d];
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-      if ((int)threadIdx.x < w)
-        for (int d = 0; d < 4; d++) s[d][threadIdx.x] += s[d][threadIdx.x + w];
-      __syncthreads();
-    }
-    if (threadIdx.x < 4) out[(size_t)sysi * out_stride + out_off + threadIdx.x] = s[threadIdx.x][0];
-  } else {
-    double a = 0.0;
-    for (int k = threadIdx.x; k < count[sysi]; k += 256) a += eself[first[sysi] + k];
-    s[0][threadIdx.x] = a;
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-      if ((int)threadIdx.x < w) s[0][threadIdx.x] += s[0][threadIdx.x + w];
-      __syncthreads();
-    }
-    if (threadIdx.x == 0) out[(size_t)sysi * out_stride + out_off + 4] = s[0][0];
-  }
+  gb_sums_block(G, blockIdx.x, blockIdx.y, s);
 }
 
 }  // namespace
@@ -1312,9 +1303,11 @@ void GBState::set_split(const int32_t *s3) {
 
 // Runs the three passes.  Forces are added to fx/fy/fz (fixed point, kcal/mol/A);
 // per-system energies (kcal/mol) go to out[s*stride + off + {0: pol cross, 1: vdw,
-// 2: elec, 3: -}] and out[s*stride + off + 4] (pol self).
+// 2: elec, 3: -}] and out[s*stride + off + 4] (pol self).  open: what shares the opening
+// launch; the plain comparator takes nothing along.
 void GBState::run(hipStream_t s, const double *x, const double *y, const double *z, long long *fx, long long *fy,
-                  long long *fz, double *out, int out_stride, int out_off, Engine *timer_owner, bool energy_only) {
+                  long long *fz, double *out, int out_stride, int out_off, Engine *timer_owner, bool energy_only,
+                  const GBOpen *open, bool sums) {
   const int n = n_atoms_total;
   const int nsys = (int)h_sys.size();
   if (plain) {
@@ -1348,7 +1341,11 @@ void GBState::run(hipStream_t s, const double *x, const double *y, const double 
   const GBPassArgs A = pass_args(x, y, z, fx, fy, fz);
   const int ntiles = (int)h_tile_atoms.size();
   const dim3 tg((ntiles + 3) / 4);
-  hipLaunchKernelGGL(k_gb_tiles, tg, dim3(256), 0, s, ntiles, tile_atoms.p, x, y, z, gbrad.p, tiles.p, gpol.p);
+  const GBOpen none{}, &O = open ? *open : none;
+  const SumList L = O.sums ? *O.sums : SumList{};
+  hipLaunchKernelGGL(k_gb_open, dim3(O.bonded_blocks + tg.x + (L.n > 0 || L.record ? 1 : 0)), dim3(256), 0, s, ntiles,
+                     tile_atoms.p, x, y, z, gbrad.p, tiles.p, gpol.p, O.bonded, O.bonded_blocks, fx, fy, fz,
+                     O.bonded_partial, O.bonded_eterm, L);
   {
     ScopedTimerOpt t(timer_owner, "gb_radii");
     GBPassArgs R = A;
@@ -1375,8 +1372,7 @@ void GBState::run(hipStream_t s, const double *x, const double *y, const double 
     launch_pass<kGbChain>(s, C, split[2]);
   }
   PDGPU_HIP(hipGetLastError());
-  hipLaunchKernelGGL(k_gb_sums, dim3(nsys, 2), dim3(256), 0, s, e_part.p, slot_beg.p, slot_end.p, eself.p,
-                     sys_first.p, sys_count.p, out, out_stride, out_off);
+  if (sums) hipLaunchKernelGGL(k_gb_sums, dim3(nsys, 2), dim3(256), 0, s, sum_args(out, out_stride, out_off));
 }
 
 // The tile kernels' inputs (radii, dE/da, chain weights) come from one full pass
@@ -1433,11 +1429,23 @@ void GBState::autotune(hipStream_t s, const double *x, const double *y, const do
 
 // ---- single-system glue ------------------------------------------------------------
 
-void Engine::launch_gb(double *energy_slots, bool energy_only) {
+void Engine::launch_gb(double *energy_slots, bool energy_only, double *bonded_slots, bool sums) {
   require(have_gb, "GB component not set up");
   // gbff.cpp takes every distance as p_j - p_i with no image: GB is a vacuum model
   require(!periodic, "GB runs in vacuum: PD's GB takes raw displacements, no periodic images");
-  gb->run(stream, x.p, y.p, z.p, fbx.p, fby.p, fbz.p, energy_slots, 8, 0, this, energy_only);
+  GBOpen O{};
+  if (bonded_slots) {
+    O.bonded = bonded_arrays();
+    O.bonded_blocks = bonded_blocks(nbonds, nangles, ntors);
+    // alternating halves: the sums of the step before read the other one
+    e_partial_bonded.resize((size_t)O.bonded_blocks * 8);
+    O.bonded_partial = e_partial_bonded.p + (size_t)gb_bonded_sel * O.bonded_blocks * 4;
+    gb_bonded_sel ^= 1;
+  }
+  O.sums = &gb_sums;
+  gb->run(stream, x.p, y.p, z.p, fbx.p, fby.p, fbz.p, energy_slots, 8, 0, this, energy_only, &O, sums);
+  gb_sums = SumList{};
+  if (bonded_slots) defer_sum4(O.bonded_partial, O.bonded_blocks, bonded_slots);
 }
 
 // h: [0] cross (2x pair sum), [1] vdw, [2] elec, [3] -, [4] self, kcal/mol.  With

@@ -28,14 +28,14 @@ __device__ __forceinline__ void slot_loads(int i, long long a0, long long a1, lo
                                            const long long *__restrict__ nbx, const long long *__restrict__ nby,
                                            const long long *__restrict__ nbz, const int *__restrict__ orig_slot,
                                            const OpenNext &O, double conv, double f[3], int &s, SlotPos &r) {
-  if (nbx != nullptr || O.on) s = orig_slot[i];
+  if (nbx != nullptr || (O.on && O.spos)) s = orig_slot[i];
   long long b0 = 0, b1 = 0, b2 = 0;
   if (nbx != nullptr) {
     b0 = nbx[s];
     b1 = nby[s];
     b2 = nbz[s];
   }
-  if (O.on) r = O.pref[s];
+  if (O.on && O.spos) r = O.pref[s];
   f[0] = (double)(a0 + b0) * conv;
   f[1] = (double)(a1 + b1) * conv;
   f[2] = (double)(a2 + b2) * conv;
@@ -605,15 +605,20 @@ void Engine::evaluate(uint32_t components, int step, bool flush) {
   const bool nbon = (components & PDGPU_NONBONDED) != 0;
   pending_sums.clear();
   if (flush) fused_pending = false;  // only pdgpu_md's steps hand their sums on
-  const bool opened = !flush && opened_ahead && nbon && list_valid;
+  const bool gbon = (components & PDGPU_GB) != 0, tiled = gbon && have_gb && !gb->plain;
+  const bool opened = !flush && opened_ahead && (nbon ? list_valid : tiled);
   opened_ahead = false;
   if (nbon && !list_valid) build_list();
-  begin_evaluation(nbon, nullptr, opened);
+  begin_evaluation(nbon, nullptr, opened, tiled);
   const bool bon = (components & PDGPU_BONDED) && (nbonds + nangles + ntors) > 0;
   if (nbon) launch_nonbonded(e_out.p + 0, !eonly, nullptr, bon ? e_out.p + 4 : nullptr);
-  if (bon && !nbon) launch_bonded(e_out.p + 4);
-  if (components & PDGPU_GB) launch_gb(e_out.p + 8, eonly);
-  if (components & PDGPU_SASA) launch_lcpo(e_out.p + 13, step, step < 0, eonly);
+  const bool gb_bonded = bon && !nbon && tiled;
+  if (bon && !nbon && !gb_bonded) launch_bonded(e_out.p + 4);
+  // the GB sums share the launch of the surface energies
+  const bool share = tiled && (components & PDGPU_SASA) && !eonly;
+  if (gbon) launch_gb(e_out.p + 8, eonly, gb_bonded ? e_out.p + 4 : nullptr, !share);
+  const GBSums G = share ? gb->sum_args(e_out.p, 8, 8) : GBSums{};
+  if (components & PDGPU_SASA) launch_lcpo(e_out.p + 13, step, step < 0, eonly, share ? &G : nullptr);
   last_components = components;
   if (flush) flush_sums();
 }
@@ -702,8 +707,14 @@ void Engine::integrate(const pdgpu_md_params &p, int step, double *ke_slot, bool
   e_partial_ke.resize((size_t)grid * 4);
   OpenNext O{};
   open = open && p.thermostat == PDGPU_NO_THERMOSTAT && p.barostat == PDGPU_NO_BAROSTAT &&
-         (last_components & PDGPU_NONBONDED) && step < p.total_steps - 1;
-  if (open) {
+         (last_components & (PDGPU_NONBONDED | PDGPU_GB)) && step < p.total_steps - 1;
+  if (open && !(last_components & PDGPU_NONBONDED)) {
+    O.on = 1;
+    O.fbx = fbx.p;
+    O.fby = fby.p;
+    O.fbz = fbz.p;
+    opened_ahead = true;
+  } else if (open) {
     O = OpenNext{1, dmax_cur ^ 1, spos.p, spos32.p, pref.p, prune_dmax.p, nbx.p, nby.p, nbz.p, fbx.p, fby.p, fbz.p};
     opened_ahead = true;
   }
@@ -916,8 +927,9 @@ void Engine::md(const pdgpu_md_params &p, int n_steps, double *epot_trace, doubl
     }
     // the integrator opens the next step's evaluation when that step keeps the
     // list and this one records no frame (whose sums run now, not deferred)
-    const bool next_rebuild = p.update_nlist > 0 && ((step + 1) % p.update_nlist) == 0;
-    const bool open = (comp & PDGPU_NONBONDED) && s + 1 < n_steps && !next_rebuild && !is_frame(step);
+    const bool next_rebuild =
+        (comp & PDGPU_NONBONDED) && p.update_nlist > 0 && ((step + 1) % p.update_nlist) == 0;
+    const bool open = (comp & (PDGPU_NONBONDED | PDGPU_GB)) && s + 1 < n_steps && !next_rebuild && !is_frame(step);
     integrate(p, step, e_out.p + 20, open);
     if (p.barostat == PDGPU_BERENDSEN_BAROSTAT) {
       // PeriodicBox::scale: the box follows the positions; the next step's

@@ -37,12 +37,6 @@ namespace pdgpu {
 
 namespace {
 
-__device__ __forceinline__ bool lcpo_full(const int *step_ptr, int step_host, int update) {
-  if (update <= 0) return true;
-  const int step = step_ptr ? *step_ptr : step_host;
-  return (step % update) == 0;
-}
-
 // EONLY: the overlap lists of calcLCPOSasaEnergies (lcpo.cpp:469-520): the test
 // on the distance itself and sphereSurfaceOverlap clamped at zero.
 // One wave per atom i at a time (kListWaves waves per workgroup, each striding over the atoms).  The lanes first test
@@ -64,11 +58,10 @@ template <bool EONLY>
 __global__ __launch_bounds__(64 * kListWaves) void k_lcpo_lists(
     int n, const int *__restrict__ atom_sys, const int *__restrict__ sys_first, const int *__restrict__ sys_count,
     const double4 *__restrict__ pr, const double *__restrict__ tile_box, double max_R,
-    const int *__restrict__ step_ptr, int step_host, int update, int *__restrict__ nl_cnt,
+    int *__restrict__ nl_cnt,
     int *__restrict__ nl_idx, double *__restrict__ nl_s) {
 #pragma clang fp contract(off)
   __shared__ int s_list[kListWaves][kLcpoMax];
-  if (!lcpo_full(step_ptr, step_host, update)) return;  // uniform: the step is the same for all
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   // whole waves; no barrier follows
   for (int i = blockIdx.x * kListWaves + wave; i < n; i += gridDim.x * kListWaves) {
@@ -159,9 +152,7 @@ __global__ __launch_bounds__(64 * kListWaves) void k_lcpo_lists(
 // none is used).  Blocks are whole waves, one tile each.
 __global__ void k_lcpo_pack(int n, const double *__restrict__ x, const double *__restrict__ y,
                             const double *__restrict__ z, const int8_t *__restrict__ use,
-                            const double *__restrict__ R, const int *__restrict__ step_ptr, int step_host,
-                            int update, double4 *__restrict__ pr, double *__restrict__ tile_box) {
-  if (!lcpo_full(step_ptr, step_host, update)) return;  // uniform
+                            const double *__restrict__ R, double4 *__restrict__ pr, double *__restrict__ tile_box) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   bool act = false;
   double p[3] = {0.0, 0.0, 0.0};
@@ -299,8 +290,7 @@ __device__ __forceinline__ void lcpo_pairs(const LcpoLds &L, int n, int m0, int 
 template <bool EONLY>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_lcpo_sasa(int n, const double4 *__restrict__ pr, const int8_t *__restrict__ use,
                                                   const double4 *__restrict__ P,
-                                                  const double *__restrict__ sig, const int *__restrict__ step_ptr,
-                                                  int step_host, int update, const int *__restrict__ nl_cnt,
+                                                  const double *__restrict__ sig, const int *__restrict__ nl_cnt,
                                                   const int *__restrict__ nl_idx, const double *__restrict__ nl_s,
                                                   double *__restrict__ sasa, double *__restrict__ dvx,
                                                   double *__restrict__ dvy, double *__restrict__ dvz) {
@@ -317,7 +307,6 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void
   auto &joff = sh.g.joff;
   auto &jw = sh.g.jw;
   const int lane = threadIdx.x;
-  if (!lcpo_full(step_ptr, step_host, update)) return;  // uniform: the step is the same for all
   // at most kLcpoGrid waves walk the atoms; on the steps that re-apply stored
   // forces every wave returns at the test above
   for (int i = blockIdx.x; i < n; i += gridDim.x) {
@@ -503,23 +492,47 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void
   }
 }
 
+// The block's sum of v in a tree (256 threads, s: 256 doubles), as its 4-wide partial.
+__device__ __forceinline__ void block_sum_256(double v, double *s, double *part) {
+  s[threadIdx.x] = v;
+  __syncthreads();
+  for (int w = 128; w > 0; w >>= 1) {
+    if ((int)threadIdx.x < w) s[threadIdx.x] += s[threadIdx.x + w];
+    __syncthreads();
+  }
+  if (threadIdx.x < 4) part[4 * blockIdx.x + threadIdx.x] = threadIdx.x == 0 ? s[0] : 0.0;
+}
+
 // Adds the stored derivatives (J/A per molecule) as forces in fixed point
 // (kcal/mol/A) and writes each atom's sigma * SASA in kcal/mol.
-__global__ void k_lcpo_apply(int n, double to_kcal, const double *__restrict__ sasa, const double *__restrict__ sig,
+// With `part` also each block's energy sum (4-wide, the first slot used), and after the
+// atoms' blocks two that take a GB evaluation's energy sums: three launches in one.
+__global__ __launch_bounds__(256) void k_lcpo_apply(int n, double to_kcal, const double *__restrict__ sasa, const double *__restrict__ sig,
                              const double *__restrict__ dvx, const double *__restrict__ dvy,
                              const double *__restrict__ dvz, long long *__restrict__ fx, long long *__restrict__ fy,
-                             long long *__restrict__ fz, double *__restrict__ eatom) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  eatom[i] = sasa[i] * sig[i] * to_kcal;
-  const double gx = dvx[i], gy = dvy[i], gz = dvz[i];
-  if (gx != 0.0 || gy != 0.0 || gz != 0.0) {
-    // to the nearest unit (fix_from_double rounds down): surface forces are small
-    const double half = 0.5 / kFixScale;
-    fix_add(&fx[i], fix_from_double(fma(gx, to_kcal, half)));
-    fix_add(&fy[i], fix_from_double(fma(gy, to_kcal, half)));
-    fix_add(&fz[i], fix_from_double(fma(gz, to_kcal, half)));
+                             long long *__restrict__ fz, double *__restrict__ eatom, double *__restrict__ part,
+                             GBSums G) {
+  __shared__ double s[4][256];
+  const int blocks = (n + 255) / 256;
+  if ((int)blockIdx.x >= blocks) {
+    gb_sums_block(G, 0, (int)blockIdx.x - blocks, s);
+    return;
   }
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  double e = 0.0;
+  if (i < n) {
+    e = sasa[i] * sig[i] * to_kcal;
+    eatom[i] = e;
+    const double gx = dvx[i], gy = dvy[i], gz = dvz[i];
+    if (gx != 0.0 || gy != 0.0 || gz != 0.0) {
+      // to the nearest unit (fix_from_double rounds down): surface forces are small
+      const double half = 0.5 / kFixScale;
+      fix_add(&fx[i], fix_from_double(fma(gx, to_kcal, half)));
+      fix_add(&fy[i], fix_from_double(fma(gy, to_kcal, half)));
+      fix_add(&fz[i], fix_from_double(fma(gz, to_kcal, half)));
+    }
+  }
+  if (part) block_sum_256(e, s[0], part);
 }
 
 __global__ void k_lcpo_energy(int n, double to_kcal, const double *__restrict__ sasa, const double *__restrict__ sig,
@@ -587,35 +600,33 @@ void LCPOState::upload(hipStream_t s) {
 }
 
 void LCPOState::run(hipStream_t s, const double *x, const double *y, const double *z, long long *fx, long long *fy,
-                    long long *fz, const int *step_ptr, int step_host, bool full, bool energy_only) {
-  const int upd = (full || energy_only) ? 0 : update;
-  // With the step known on the host, a step that re-applies the stored forces
-  // launches only k_lcpo_apply (the three others would return at once); with the
-  // step read on the device (a captured graph) every launch is recorded.
-  const bool host_reapply = step_ptr == nullptr && upd > 0 && (step_host % upd) != 0;
-  if (host_reapply && !energy_only) {
-    hipLaunchKernelGGL(k_lcpo_apply, dim3((n + 255) / 256), dim3(256), 0, s, n, Consts::J_to_kcalmol(), sasa.p,
-                       sig.p, dvx.p, dvy.p, dvz.p, fx, fy, fz, eatom.p);
+                    long long *fz, int step, bool full, bool energy_only, double *block_part, const GBSums *gb) {
+  auto apply = [&]() {
+    hipLaunchKernelGGL(k_lcpo_apply, dim3((n + 255) / 256 + (gb ? 2 : 0)), dim3(256), 0, s, n,
+                       Consts::J_to_kcalmol(), sasa.p, sig.p, dvx.p, dvy.p, dvz.p, fx, fy, fz, eatom.p, block_part,
+                       gb ? *gb : GBSums{});
     PDGPU_HIP(hipGetLastError());
+  };
+  if (!full && !energy_only && reapplies(step)) {  // the stored forces again
+    apply();
     return;
   }
-  hipLaunchKernelGGL(k_lcpo_pack, dim3((n + 255) / 256), dim3(256), 0, s, n, x, y, z, use.p, R.p, step_ptr,
-                     step_host, upd, pr.p, tile_box.p);
+  hipLaunchKernelGGL(k_lcpo_pack, dim3((n + 255) / 256), dim3(256), 0, s, n, x, y, z, use.p, R.p,
+                     pr.p, tile_box.p);
   const int lb = std::min((n + kListWaves - 1) / kListWaves, kListGrid);
   if (energy_only) {
     hipLaunchKernelGGL(k_lcpo_lists<true>, dim3(lb), dim3(64 * kListWaves), 0, s, n, atom_sys.p, sys_first.p,
-                       sys_count.p, pr.p, tile_box.p, max_R, step_ptr, step_host, upd, nl_cnt.p, nl_idx.p, nl_s.p);
-    hipLaunchKernelGGL(k_lcpo_sasa<true>, dim3(std::min(n, kLcpoGrid)), dim3(64), 0, s, n, pr.p, use.p, P.p, sig.p, step_ptr, step_host,
-                       upd, nl_cnt.p, nl_idx.p, nl_s.p, sasa.p, dvx.p, dvy.p, dvz.p);
+                       sys_count.p, pr.p, tile_box.p, max_R, nl_cnt.p, nl_idx.p, nl_s.p);
+    hipLaunchKernelGGL(k_lcpo_sasa<true>, dim3(std::min(n, kLcpoGrid)), dim3(64), 0, s, n, pr.p, use.p, P.p, sig.p,
+                       nl_cnt.p, nl_idx.p, nl_s.p, sasa.p, dvx.p, dvy.p, dvz.p);
     hipLaunchKernelGGL(k_lcpo_energy, dim3((n + 255) / 256), dim3(256), 0, s, n, Consts::J_to_kcalmol(), sasa.p,
                        sig.p, eatom.p);
   } else {
     hipLaunchKernelGGL(k_lcpo_lists<false>, dim3(lb), dim3(64 * kListWaves), 0, s, n, atom_sys.p, sys_first.p,
-                       sys_count.p, pr.p, tile_box.p, max_R, step_ptr, step_host, upd, nl_cnt.p, nl_idx.p, nl_s.p);
-    hipLaunchKernelGGL(k_lcpo_sasa<false>, dim3(std::min(n, kLcpoGrid)), dim3(64), 0, s, n, pr.p, use.p, P.p, sig.p, step_ptr, step_host,
-                       upd, nl_cnt.p, nl_idx.p, nl_s.p, sasa.p, dvx.p, dvy.p, dvz.p);
-    hipLaunchKernelGGL(k_lcpo_apply, dim3((n + 255) / 256), dim3(256), 0, s, n, Consts::J_to_kcalmol(), sasa.p,
-                       sig.p, dvx.p, dvy.p, dvz.p, fx, fy, fz, eatom.p);
+                       sys_count.p, pr.p, tile_box.p, max_R, nl_cnt.p, nl_idx.p, nl_s.p);
+    hipLaunchKernelGGL(k_lcpo_sasa<false>, dim3(std::min(n, kLcpoGrid)), dim3(64), 0, s, n, pr.p, use.p, P.p, sig.p,
+                       nl_cnt.p, nl_idx.p, nl_s.p, sasa.p, dvx.p, dvy.p, dvz.p);
+    apply();
   }
   PDGPU_HIP(hipGetLastError());
 }
@@ -629,27 +640,22 @@ namespace {
 __global__ void k_block_sum(int n, const double *__restrict__ v, double *__restrict__ part) {
   __shared__ double s[256];
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  s[threadIdx.x] = i < n ? v[i] : 0.0;
-  __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {
-    if ((int)threadIdx.x < w) s[threadIdx.x] += s[threadIdx.x + w];
-    __syncthreads();
-  }
-  if (threadIdx.x < 4) part[4 * blockIdx.x + threadIdx.x] = threadIdx.x == 0 ? s[0] : 0.0;
+  block_sum_256(i < n ? v[i] : 0.0, s, part);
 }
 }  // namespace
 
-void Engine::launch_lcpo(double *energy_slot, int step, bool full, bool energy_only) {
+void Engine::launch_lcpo(double *energy_slot, int step, bool full, bool energy_only, const GBSums *with_gb) {
   require(lcpo != nullptr, "LCPO component not set up");
   // lcpo.cpp takes every distance as p_j - p_i with no image
   require(!periodic, "LCPO runs in vacuum: PD's LCPO takes raw displacements, no periodic images");
-  {
-    ScopedTimer t(*this, "lcpo");
-    lcpo->run(stream, x.p, y.p, z.p, fbx.p, fby.p, fbz.p, nullptr, step, full, energy_only);
-  }
   const int blocks = (n + 255) / 256;
   e_partial_lcpo.resize((size_t)blocks * 4);
-  hipLaunchKernelGGL(k_block_sum, dim3(blocks), dim3(256), 0, stream, n, lcpo->eatom.p, e_partial_lcpo.p);
+  {
+    ScopedTimer t(*this, "lcpo");
+    lcpo->run(stream, x.p, y.p, z.p, fbx.p, fby.p, fbz.p, step, full, energy_only, e_partial_lcpo.p,
+              with_gb);
+  }
+  if (energy_only) hipLaunchKernelGGL(k_block_sum, dim3(blocks), dim3(256), 0, stream, n, lcpo->eatom.p, e_partial_lcpo.p);
   defer_sum4(e_partial_lcpo.p, blocks, energy_slot);
 }
 

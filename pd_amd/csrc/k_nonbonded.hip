@@ -470,7 +470,6 @@ __global__ __launch_bounds__(64 * kGroup * kMaxShare) __attribute__((amdgpu_wave
       const int img = (int)((ent.x >> 24) & 31u);
       const unsigned lm = valid ? (ent.y & 0xFFu) : 0u;
       const unsigned codes = (ent.y >> 8) & 0xFFFFu;
-      const unsigned rank = ent.y >> 24;
       const unsigned clo = codes & 0x5555u, chi = (codes >> 1) & 0x5555u;
       const unsigned excl = clo ^ chi;  // codes 1 and 2: 1-2 / 1-3 pairs, scale 0
       const unsigned is14 = clo & chi;  // code 3: 1-4 pair
@@ -771,9 +770,7 @@ __global__ __launch_bounds__(64 * kGroup * kMaxShare) __attribute__((amdgpu_wave
 template <int ELEC, bool VDW, bool FORCES, bool FINE>
 void launch(Engine &E, double *partial, const SumList &L, double *bonded_partial) {
   const int nbb = bonded_partial ? bonded_blocks(E.nbonds, E.nangles, E.ntors) : 0;
-  const BondedArrays B{E.nbonds, E.nangles, E.ntors, E.b_i.p, E.b_j.p, E.b_l.p, E.b_k.p, E.a_i.p, E.a_a.p,
-                       E.a_j.p, E.a_t0.p, E.a_k.p, E.t_i.p, E.t_a.p, E.t_b.p, E.t_j.p, E.t_terms.p, E.t_vn.p,
-                       E.t_nn.p, E.t_gamma.p, E.b_win.p};
+  const BondedArrays B = E.bonded_arrays();
   hipLaunchKernelGGL((k_nonbonded<ELEC, VDW, FORCES, FINE>), dim3(8 * E.nb_per_cap * E.nb_parts + nbb + (L.n > 0 || L.record ? 1 : 0)),
                      dim3(64 * kGroup * E.nb_share), 0, E.stream, E.nbk, 8 * E.nb_per_cap, E.max_groups, E.nb_parts, E.n_groups_d.p, E.grp_order.p, E.grp_first.p, E.grp_count.p, E.wg_ncand.p,
                      E.wg_cand.p,
@@ -909,7 +906,7 @@ void Engine::setup_nonbonded(const pdgpu_nb_params &p) {
   list_valid = false;
 }
 
-void Engine::begin_evaluation(bool nonbonded, double *eo, bool opened) {
+void Engine::begin_evaluation(bool nonbonded, double *eo, bool opened, bool gb_next) {
   const int T = 256;
   fbx.resize(n);
   fby.resize(n);
@@ -923,6 +920,15 @@ void Engine::begin_evaluation(bool nonbonded, double *eo, bool opened) {
   if (fused_pending) {
     L = fused_sums;
     fused_pending = false;
+  }
+  gb_sums = SumList{};
+  if (!nonbonded && gb_next) {  // the sums run in k_gb_open
+    gb_sums = L;
+    L = SumList{};
+  }
+  if (!nonbonded && opened) {  // the previous step's integrator cleared the accumulators
+    require(!zero_e, "an opened evaluation keeps its energy slots");
+    return;
   }
   if (!nonbonded) {
     hipLaunchKernelGGL(k_begin_nb, dim3((std::max(n, 24) + T - 1) / T), dim3(T), 0, stream, 0, n, n_clusters_d.p,

@@ -58,6 +58,38 @@ def test_batch_langevin_equals_single_systems():
         np.testing.assert_allclose(ek_b[:, k], ek, rtol=1e-12)
 
 
+@pytest.mark.parametrize("comps,every", [(G.PDGPU_GB, 1), (COMPS, 1), (COMPS | G.PDGPU_SASA, 1),
+                                         (COMPS | G.PDGPU_SASA, 3)])
+def test_md_steps_share_launches(comps, every):
+    # Within one call a step's opening kernel takes the sums of the step before and
+    # the bonded terms, the integrator clears the next step's accumulators, and a
+    # batch replays one graph for full surface steps and one for the others; one
+    # step per call does none of that.  The physics is the same, bit for bit.
+    sys_ = chains([20, 9], seed0=30)
+    md = dict(integrator=G.PDGPU_LANGEVIN, components=comps, timestep=2e-15, temperature=300.0, fric_coeff=1e12,
+              update_nlist=0, total_steps=100, seed=7)
+
+    def engine(k):
+        e = gb_engine(sys_[k], 60 + k)
+        if comps & G.PDGPU_SASA:
+            use, rad, P = S.lcpo_params(sys_[k])
+            e.setup_lcpo(G.LCPOParams(GlobalASP=0.005, UpdateSasa=every), rad, P, use)
+        return e
+    whole, single = [engine(0), engine(1)], [engine(0), engine(1)]
+    b = G.Batch(whole)
+    b.set_temperatures([300.0, 300.0])
+    ep_b, ek_b = b.md(G.MDParams(step_offset=2, noise_stream=0, **md), 7)
+    for k in range(2):
+        ep, ek = whole[k].md(G.MDParams(step_offset=2, noise_stream=k, **md), 7)
+        steps = [single[k].md(G.MDParams(step_offset=2 + s, noise_stream=k, **md), 1) for s in range(7)]
+        assert np.array_equal(ep, [s[0][0] for s in steps]) and np.array_equal(ek, [s[1][0] for s in steps])
+        for get in ("get_positions", "get_velocities"):
+            x = getattr(whole[k], get)()
+            assert np.array_equal(x, getattr(single[k], get)()) and np.array_equal(x, getattr(b, get)(k))
+        np.testing.assert_allclose(ep_b[:, k], ep, rtol=1e-12)
+        np.testing.assert_allclose(ek_b[:, k], ek, rtol=1e-12)
+
+
 def test_remd_exchanges_follow_metropolis():
     base = S.peptide_chain(6, seed=3)
     temps = 300.0 * (500.0 / 300.0) ** (np.arange(4) / 3.0)
