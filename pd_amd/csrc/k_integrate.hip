@@ -200,7 +200,7 @@ __device__ void langevin_noise(uint32_t k0, uint32_t k1, uint32_t stream, uint32
 
 // ---- thermostats (md.cpp:579-660) and momentum removal (md.cpp:263-272, 412-517) ----
 // With a thermostat, velocity Verlet and Beeman run as two kernels around one
-// reduction: the velocity kick and the kinetic energy (calcKineticEnergy),
+// reduction (which the second one does itself, without the barostat): the velocity kick and the kinetic energy (calcKineticEnergy),
 // then applyThermostat on the velocities and the moving half of the step.
 struct ThermoArgs {
   int kind;          // PDGPU_NO_THERMOSTAT / PDGPU_ANDERSEN / PDGPU_BERENDSEN
@@ -246,6 +246,11 @@ __global__ __launch_bounds__(256) void k_kick(int n, double t, double conv, int 
   block_sum4_dev(ke, ke_partial);
 }
 
+__device__ __forceinline__ double berendsen_chi(const ThermoArgs &A, int natoms, double ekin) {
+  const double Edes = 3.0 * natoms * Consts::kB * A.temp / 2.0;
+  return A.kind == PDGPU_BERENDSEN ? sqrt(1.0 + A.dt * (Edes / ekin - 1.0) / A.tau) : 1.0;
+}
+
 // The kinetic energy of the step (one workgroup) and Berendsen's factor
 // chi = sqrt(1 + dt (Edes/ekin - 1) / tau), Edes = 3 N kB T / 2 (md.cpp:601-617).
 // With the barostat: the pressure of calcKineticEnergy, P = (2 ekin - W) / (3 V)
@@ -266,8 +271,7 @@ __global__ __launch_bounds__(1024) void k_thermo_sum(const double *__restrict__ 
     for (int k = 0; k < 16; k++) ekin += s[k];
     ke_slot[0] = ekin;
     ke_slot[1] = ke_slot[2] = ke_slot[3] = 0.0;
-    const double Edes = 3.0 * natoms * Consts::kB * A.temp / 2.0;
-    chi[0] = A.kind == PDGPU_BERENDSEN ? sqrt(1.0 + A.dt * (Edes / ekin - 1.0) / A.tau) : 1.0;
+    chi[0] = berendsen_chi(A, natoms, ekin);
     chi[1] = 1.0;
     if (A.baro) {
       double vir = 0.0;
@@ -296,9 +300,30 @@ __device__ void andersen_draws(uint32_t k0, uint32_t k1, uint32_t stream, uint32
   z[3] = uniform53(c[0], c[1]);
 }
 
+// k_thermo_sum's kinetic energy by a workgroup of 256, in every thread: each stands
+// for four of the 1024 threads, so the additions and their order are the same.
+__device__ __forceinline__ double thermo_ekin(const double *__restrict__ part, int count) {
+  __shared__ double s[16];
+  for (int q = 0; q < 4; q++) {
+    double a = 0.0;
+    for (int i = 256 * q + (int)threadIdx.x; i < count; i += 1024) a += part[4 * i];
+    a = wave_sum(a);
+    if ((threadIdx.x & 63) == 0) s[4 * q + (threadIdx.x >> 6)] = a;
+  }
+  __syncthreads();
+  double ekin = 0.0;
+  for (int k = 0; k < 16; k++) ekin += s[k];
+  return ekin;
+}
+
+// With `part` (no barostat) every workgroup sums the `count` kinetic-energy partials
+// itself, where a launch of one workgroup between the two kernels took 4 us and two
+// gaps; the O fields make it the next step's opening kernel as well.  An NVT step of
+// 12,288 atoms: 57.6 us with three kernels and k_begin_nb, 54.7 now.
 template <int INTEG>
 __global__ __launch_bounds__(256) void k_thermo_move(
     int n, double t, double conv, int move, ThermoArgs A, const double *__restrict__ chi,
+    const double *__restrict__ part, int count, double *__restrict__ ke_slot, OpenNext O,
     const double *__restrict__ mass, const long long *__restrict__ fbx, const long long *__restrict__ fby,
     const long long *__restrict__ fbz, const long long *__restrict__ nbx, const long long *__restrict__ nby,
     const long long *__restrict__ nbz, const int *__restrict__ orig_slot, double *__restrict__ x,
@@ -306,73 +331,86 @@ __global__ __launch_bounds__(256) void k_thermo_move(
     double *__restrict__ vz, double *__restrict__ fox, double *__restrict__ foy, double *__restrict__ foz) {
 #pragma clang fp contract(off)
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const double m = mass[i];
-  double v[3] = {vx[i], vy[i], vz[i]};
-  if (A.kind == PDGPU_BERENDSEN) {
-    const double c = chi[0];
-    for (int d = 0; d < 3; d++) v[d] *= c;
-  } else if (A.kind == PDGPU_ANDERSEN) {  // applyAndersonThermostat, md.cpp:620-660
-    uint32_t test;
-    double zz[4];
-    andersen_draws(A.k0, A.k1, A.stream, A.step, (uint32_t)i, test, zz);
-    if (!((int)test > A.intrate)) {
-      const double TwoPI = 2.0 * Consts::PI;
-      const double sigma = sqrt(Consts::kB * A.temp / m);
-      double l = sqrt(-2.0 * log(zz[0]));
-      const double nx = l * cos((-TwoPI) * zz[1]) * sigma;
-      l = sqrt(-2.0 * log(zz[2]));
-      const double ny = l * cos((-TwoPI) * zz[3]) * sigma;  // nrand(vy, vz) draws vy again
-      const double nz = l * sin((-TwoPI) * zz[3]) * sigma;
-      if (!(fabs(nx) > (sigma * 4)) && !(fabs(ny) > (sigma * 4)) && !(fabs(nz) > (sigma * 4))) {
-        v[0] = nx;
-        v[1] = ny;
-        v[2] = nz;
+  double px = 0.0, py = 0.0, pz = 0.0;
+  int s = 0;
+  SlotPos r{};
+  double ekin = 0.0;
+  if (part) {  // uniform
+    ekin = thermo_ekin(part, count);
+    if (i < 4) ke_slot[i] = i == 0 ? ekin : 0.0;
+  }
+  if (i < n) {
+    const double m = mass[i];
+    double v[3] = {vx[i], vy[i], vz[i]};
+    if (A.kind == PDGPU_BERENDSEN) {
+      const double c = part ? berendsen_chi(A, n, ekin) : chi[0];
+      for (int d = 0; d < 3; d++) v[d] *= c;
+    } else if (A.kind == PDGPU_ANDERSEN) {  // applyAndersonThermostat, md.cpp:620-660
+      uint32_t test;
+      double zz[4];
+      andersen_draws(A.k0, A.k1, A.stream, A.step, (uint32_t)i, test, zz);
+      if (!((int)test > A.intrate)) {
+        const double TwoPI = 2.0 * Consts::PI;
+        const double sigma = sqrt(Consts::kB * A.temp / m);
+        double l = sqrt(-2.0 * log(zz[0]));
+        const double nx = l * cos((-TwoPI) * zz[1]) * sigma;
+        l = sqrt(-2.0 * log(zz[2]));
+        const double ny = l * cos((-TwoPI) * zz[3]) * sigma;  // nrand(vy, vz) draws vy again
+        const double nz = l * sin((-TwoPI) * zz[3]) * sigma;
+        if (!(fabs(nx) > (sigma * 4)) && !(fabs(ny) > (sigma * 4)) && !(fabs(nz) > (sigma * 4))) {
+          v[0] = nx;
+          v[1] = ny;
+          v[2] = nz;
+        }
       }
     }
-  }
-  double f[3];
-  total_force(i, fbx, fby, fbz, nbx, nby, nbz, orig_slot, conv, f[0], f[1], f[2]);
-  const double ia = 1 / Consts::Angstrom;
-  if (A.baro) {  // WorkSpace::scaleSystem (workspace.cpp:362-369), before the move
-    const double fac = chi[1];
-    x[i] *= fac;
-    y[i] *= fac;
-    z[i] *= fac;
-  }
-  if (INTEG == PDGPU_VELOCITY_VERLET) {  // second loop, md.cpp:836-854
-    const double tinvmass = 0.5 * t / m;
-    double dr[3];
-    for (int d = 0; d < 3; d++) {
-      const double dv = f[d] * tinvmass;
-      v[d] += dv;
-      dr[d] = t * (v[d] + dv);
-      dr[d] *= ia;
-      v[d] += dv;
+    double f[3];
+    slot_loads(i, fbx[i], fby[i], fbz[i], nbx, nby, nbz, orig_slot, O, conv, f, s, r);
+    const double ia = 1 / Consts::Angstrom;
+    if (A.baro) {  // WorkSpace::scaleSystem (workspace.cpp:362-369), before the move
+      const double fac = chi[1];
+      x[i] *= fac;
+      y[i] *= fac;
+      z[i] *= fac;
     }
-    x[i] += dr[0];
-    y[i] += dr[1];
-    z[i] += dr[2];
-  } else if (move) {  // Beeman, md.cpp:894-918
-    const double tinvmass = t / (6.0 * m);
-    const double fo[3] = {fox[i], foy[i], foz[i]};
-    double dr[3], dv[3];
-    for (int d = 0; d < 3; d++) {
-      dr[d] = t * (v[d] + (4.0 * f[d] - fo[d]) * tinvmass);
-      dr[d] *= ia;
-      dv[d] = (5.0 * f[d] - fo[d]) * tinvmass;
+    if (INTEG == PDGPU_VELOCITY_VERLET) {  // second loop, md.cpp:836-854
+      const double tinvmass = 0.5 * t / m;
+      double dr[3];
+      for (int d = 0; d < 3; d++) {
+        const double dv = f[d] * tinvmass;
+        v[d] += dv;
+        dr[d] = t * (v[d] + dv);
+        dr[d] *= ia;
+        v[d] += dv;
+      }
+      x[i] += dr[0];
+      y[i] += dr[1];
+      z[i] += dr[2];
+    } else if (move) {  // Beeman, md.cpp:894-918
+      const double tinvmass = t / (6.0 * m);
+      const double fo[3] = {fox[i], foy[i], foz[i]};
+      double dr[3], dv[3];
+      for (int d = 0; d < 3; d++) {
+        dr[d] = t * (v[d] + (4.0 * f[d] - fo[d]) * tinvmass);
+        dr[d] *= ia;
+        dv[d] = (5.0 * f[d] - fo[d]) * tinvmass;
+      }
+      x[i] += dr[0];
+      y[i] += dr[1];
+      z[i] += dr[2];
+      for (int d = 0; d < 3; d++) v[d] += dv[d];
+      fox[i] = f[0];
+      foy[i] = f[1];
+      foz[i] = f[2];
     }
-    x[i] += dr[0];
-    y[i] += dr[1];
-    z[i] += dr[2];
-    for (int d = 0; d < 3; d++) v[d] += dv[d];
-    fox[i] = f[0];
-    foy[i] = f[1];
-    foz[i] = f[2];
+    vx[i] = v[0];
+    vy[i] = v[1];
+    vz[i] = v[2];
+    px = x[i];
+    py = y[i];
+    pz = z[i];
   }
-  vx[i] = v[0];
-  vy[i] = v[1];
-  vz[i] = v[2];
+  if (O.on) open_next_at(O, i, n, s, r, px, py, pz);
 }
 
 // Sums for the momentum step: mass, m v, m p, m (p x v) (p in A), 10 per block.
@@ -570,8 +608,8 @@ void Engine::flush_sums(const StepRecord *rec) {
   PDGPU_HIP(hipGetLastError());
 }
 
-// The sums of an MD step wait for the next step's opening kernel (k_begin_nb),
-// which saves a launch per step; more lists than one workgroup takes run now.
+// The sums of an MD step wait for a workgroup of the next step's nonbonded or GB opening
+// kernel, which saves a launch per step; more lists than one workgroup takes run now.
 void Engine::defer_step_sums(const StepRecord &rec) {
   if (pending_sums.size() > (size_t)kMaxSums) {
     flush_sums(&rec);
@@ -706,8 +744,7 @@ void Engine::integrate(const pdgpu_md_params &p, int step, double *ke_slot, bool
   const int grid = (n + T - 1) / T;
   e_partial_ke.resize((size_t)grid * 4);
   OpenNext O{};
-  open = open && p.thermostat == PDGPU_NO_THERMOSTAT && p.barostat == PDGPU_NO_BAROSTAT &&
-         (last_components & (PDGPU_NONBONDED | PDGPU_GB)) && step < p.total_steps - 1;
+  open = open && p.barostat == PDGPU_NO_BAROSTAT && (last_components & (PDGPU_NONBONDED | PDGPU_GB)) && step < p.total_steps - 1;
   if (open && !(last_components & PDGPU_NONBONDED)) {
     O.on = 1;
     O.fbx = fbx.p;
@@ -774,14 +811,20 @@ void Engine::integrate(const pdgpu_md_params &p, int step, double *ke_slot, bool
     else
       hipLaunchKernelGGL(k_kick<PDGPU_VELOCITY_VERLET>, dim3(grid), dim3(T), 0, stream, n, p.timestep, conv, first,
                          mass.p, fbx.p, fby.p, fbz.p, ax, ay, az, orig_slot.p, vx.p, vy.p, vz.p, e_partial_ke.p);
-    hipLaunchKernelGGL(k_thermo_sum, dim3(1), dim3(1024), 0, stream, e_partial_ke.p, grid, n, A, ke_slot, thermo.p);
+    // every workgroup reads all partials, so their traffic grows with the square of the
+    // atoms; past 131,072 the sum keeps its own launch, and the barostat needs its factor
+    // on the host
+    const bool own_sum = baro || grid > 512;
+    const double *part = own_sum ? nullptr : e_partial_ke.p;
+    if (own_sum)
+      hipLaunchKernelGGL(k_thermo_sum, dim3(1), dim3(1024), 0, stream, e_partial_ke.p, grid, n, A, ke_slot, thermo.p);
     if (beeman)
       hipLaunchKernelGGL(k_thermo_move<PDGPU_BEEMAN>, dim3(grid), dim3(T), 0, stream, n, p.timestep, conv, move, A,
-                         thermo.p, mass.p, fbx.p, fby.p, fbz.p, ax, ay, az, orig_slot.p, x.p, y.p, z.p, vx.p, vy.p,
-                         vz.p, fox.p, foy.p, foz.p);
+                         thermo.p, part, grid, ke_slot, O, mass.p, fbx.p, fby.p, fbz.p, ax, ay, az, orig_slot.p, x.p,
+                         y.p, z.p, vx.p, vy.p, vz.p, fox.p, foy.p, foz.p);
     else
       hipLaunchKernelGGL(k_thermo_move<PDGPU_VELOCITY_VERLET>, dim3(grid), dim3(T), 0, stream, n, p.timestep, conv,
-                         move, A, thermo.p, mass.p, fbx.p, fby.p, fbz.p, ax, ay, az, orig_slot.p, x.p, y.p, z.p,
+                         move, A, thermo.p, part, grid, ke_slot, O, mass.p, fbx.p, fby.p, fbz.p, ax, ay, az, orig_slot.p, x.p, y.p, z.p,
                          vx.p, vy.p, vz.p, nullptr, nullptr, nullptr);
     PDGPU_HIP(hipGetLastError());
     return;

@@ -309,6 +309,36 @@ def test_md_run_equals_single_step_calls(integ):
     assert np.array_equal(ep1, ep2) and np.array_equal(ek1, ek2)
 
 
+@pytest.mark.parametrize("n_waters,thermo", [(1, G.PDGPU_BERENDSEN), (85, G.PDGPU_ANDERSEN), (86, G.PDGPU_BERENDSEN),
+                                             (343, G.PDGPU_BERENDSEN), (1366, G.PDGPU_BERENDSEN)])
+def test_thermostat_steps_share_launches(n_waters, thermo):
+    """With a thermostat every workgroup of the moving kernel sums the kinetic-energy
+    partials (one to 17 of them here) and opens the next step; one-step calls open
+    theirs apart.  Same bits, and the first step's kinetic energy is the plain sum
+    (FP64 sums of n positive terms in another order: n ulp at most)."""
+    s = S.water_box(n_waters, seed=6)
+    if n_waters < 343:
+        s.box = None
+    comps = G.PDGPU_NONBONDED | G.PDGPU_BONDED
+    v0 = mb_velocities(s, 300.0, 3)
+    runs = []
+    for step_sizes in ([6], [1] * 6):
+        e = G.engine_for(s, G.nb_params(**WATER_NB), padding=2.0, bonded=True)
+        e.set_velocities(v0)
+        print(f"case n={3 * n_waters} thermostat {thermo} calls {len(step_sizes)}", flush=True)
+        ek = []
+        for k in step_sizes:
+            md = G.MDParams(integrator=G.PDGPU_BEEMAN, components=comps, timestep=1e-15, temperature=250.0,
+                            thermostat=thermo, berendsen_tau=100e-15, andersen_rate=0.5, update_nlist=4,
+                            step_offset=len(ek), total_steps=100, seed=4)
+            ek += list(e.md(md, k)[1])
+        runs.append((e.get_positions(), e.get_velocities(), np.array(ek)))
+    for a, b in zip(*runs):
+        assert np.array_equal(a, b)
+    plain = 0.5 * (s.mass[:, None] * v0 ** 2).sum()
+    assert abs(runs[0][2][0] - plain) <= 4 * s.n * np.finfo(float).eps * plain
+
+
 def test_md_autotuner_restores_state():
     """pdgpu_autotune_md times MD steps at each prune margin from the same state,
     keeps the fastest and restores positions, velocities and the update count; the
