@@ -459,7 +459,7 @@ def gb_benchmarks(args, log):
         "roofline_gb_pair": {"bound": "valu", "achieved": round(achieved, 3), "peak": FP32_PEAK_TFLOPS,
                              "unit": "TFLOP/s", "frac": round(achieved / FP32_PEAK_TFLOPS, 5),
                              "algorithmic_flop_per_launch": pairs * GB_FLOP_PAIR,
-                             "executed": executed_flops("k_gb_pair (300-residue chain)", pair_us * 1e-6)},
+                             "executed": executed_flops("k_gb_pass pair (300-residue chain)", pair_us * 1e-6)},
     }
     log(f"single chain ({s.n} atoms): {out['single_chain']['steps_per_s']} steps/s "
         f"({time.perf_counter() - t0:.1f} s)")
