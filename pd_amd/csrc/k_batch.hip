@@ -5,8 +5,8 @@
 // the GB passes walk a flat list of tile pairs of every system (k_gb.hip), the
 // bonded kernel covers the concatenated term lists, and the integrator reads
 // each atom's system temperature.  Per-system energies come from segmented
-// FP64 reductions.  The step is recorded once into a hipGraph and replayed, with
-// the step number kept on the device, so a run of n steps is n graph launches
+// FP64 reductions.  The step is recorded into hipGraphs (see Batch::graph) and replayed,
+// with the step number kept on the device, so a run of n steps is n graph launches
 // and no host round trip.
 //
 // REX_Local (remd.cpp:65-254) runs its replicas one after another on one

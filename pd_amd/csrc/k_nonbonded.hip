@@ -32,7 +32,7 @@
 // with one FP32 wave a cluster, 13 now, and the errors of 50 MD steps against 64 bits
 // 100 to 1,000 times smaller.  A chip-filling launch (98,304 atoms, 95 us) is bound
 // by issue; there the flush without a division per slot, the lane swaps and DPP sums
-// of the epilogue and the energy sums in a workgroup of their own took 8 us off.
+// of the epilogue and the energy sums in a workgroup of their own took it from 101.
 #include "bonded_dev.hpp"
 #include "engine.hpp"
 #include "group_order_dev.hpp"
@@ -50,8 +50,9 @@ enum { EL_NONE = 0, EL_PLAIN = 1, EL_ESWITCH = 3, EL_FSWITCH = 4 };
 // |r^2_fp32 - r^2_exact| is below 1e-5 r^2 (one FP32 rounding of d, three of the
 // sum); pairs within this band of a cutoff are re-tested in FP64.
 constexpr float kNearBand = 0.01f;
-// The FP64 pair arithmetic's r^2 is within 1e-12 of PD's at any cutoff below 64 A.
-constexpr double kFineBand = 1e-9;
+// The FP64 pair arithmetic's r^2 differs from PD's by a few ulp of the coordinates times
+// r: 1e-12 A^2 in a 100 A box, 1e-6 at coordinates of 1e8 A.
+constexpr double kFineBand = 1e-5;
 
 // Image index (i+1)*9 + (j+1)*3 + (k+1) -> the basis vector (i*Lx, j*Ly, k*Lz)
 // of PeriodicBox::setupCellDimensions (space.cpp:94-109).
@@ -381,7 +382,7 @@ __global__ __launch_bounds__(64 * kGroup * kMaxShare) __attribute__((amdgpu_wave
           const double r2s = fma(dx, dx, fma(dy, dy, dz * dz));
           bool inc = r2s <= P.cut2, inv = r2s < P.vdwcut2;
           const bool listed = ((lm >> a) & 1u) && !((excl >> (2 * a)) & 1u);
-          // PD's own test where the cutoff is near (its rounding differs by ~1e-13)
+          // PD's own test where the cutoff is near
           const bool near = fabs(r2s - P.cut2) < kFineBand || fabs(r2s - P.vdwcut2) < kFineBand;
           if (__builtin_expect(__ballot(near && listed) != 0ull, 0)) {
 #pragma clang fp contract(off)
